@@ -402,6 +402,20 @@ def test_triangle_multiplication(device, n, outgoing, bf16):
                  (pair.to(device), mask.to(device)), bf16, "trimul")
 
 
+# One size per contraction tile on a 256-CU device (64 x 64, 192 x 384, 128 x 256, 192 x 192), each just
+# past a multiple of its tile and of the 16 positions of a result block.
+@pytest.mark.parametrize("n,outgoing", [(129, True), (65, False), (307, True), (385, False), (521, False), (529, True),
+                                        (577, True)])
+def test_triangle_multiplication_tiles(device, n, outgoing):
+    announce("trimul tiles", n, outgoing)
+    ref, hip = pair_of("TriangleMultiplication", dict(c_pair=128, _outgoing=outgoing), seed=n)
+    pair = torch.randn(n, n, 128, generator=torch.Generator().manual_seed(n)).bfloat16()
+    mask = torch.ones(n, n)
+    mask[:, -1] = 0
+    check_module(ref, hip, hnn.triangle_multiplication_hip, (pair.float(), mask), (pair.to(device), mask.to(device)),
+                 True, "trimul tiles")
+
+
 @pytest.mark.parametrize("c,n", [(64, 40), (96, 33), (288, 24)])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_triangle_multiplication_other_widths(device, c, n, bf16):

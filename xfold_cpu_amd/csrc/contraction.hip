@@ -8,17 +8,19 @@
 // last k-step needs no bounds. The result goes to the blocked result layout: 16 pair
 // positions' channels contiguous.
 //
-// Tiling: 192 x 384 output tiles, one workgroup of 8 wavefronts per CU (N <= 1024), or
-// 192 x 192 tiles, two workgroups of 4 wavefronts per CU; each wavefront owns 96 x 96 (6 x 6
-// MFMA 16x16x32 tiles). Per k-step of 32 both operand tiles go global -> LDS with
-// global_load_lds_dwordx4 (no registers) into a ring of 4 or 3 slots, so the loads of the
-// next 2 or 1 steps are in flight while step s is multiplied; one barrier per step. Rows
+// Tiling: the output tile is picked by n (pick_tile): 192 x 384 to 64 x 64, one to four workgroups
+// per CU, each wavefront owning 96 x 96, 64 x 64 or 32 x 32 (MFMA 16x16x32 tiles). Per k-step of 32
+// both operand tiles go global -> LDS with global_load_lds_dwordx4 (no registers) into a ring
+// of 3 or 4 slots, so the loads of the next 1 or 2
+// steps are in flight while step s is multiplied; one barrier per step. Rows
 // are 64 B in LDS with the 16-byte slots XOR-swizzled (slot c of row r holds chunk
 // c ^ ((r >> 2) & 3)), so the 16 rows of an MFMA operand read hit distinct bank groups.
 // The MFMA takes R rows as its A operand so that a lane ends up with four consecutive j
 // of one i and writes them as one 8-byte store. Channels are numbered so that each XCD
 // works through a contiguous run of tiles: the workgroups in flight on an XCD cover a few
 // consecutive channels, whose k-slices share 128-byte lines and DRAM pages.
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -26,8 +28,6 @@ namespace xfh {
 
 namespace {
 
-constexpr int WT = 96;                  // wavefront tile edge
-constexpr int NT = WT / 16;             // MFMA tiles per wavefront edge (6)
 constexpr int TK = 32;                  // k-step
 typedef __attribute__((address_space(1))) void global_void;
 typedef __attribute__((address_space(3))) void lds_void;
@@ -45,26 +45,26 @@ template <int P, int MAXY> __device__ __forceinline__ void wait_younger(int youn
   }
 }
 
-// TBI x TBJ output tiles (rows i of L, rows j of R), 2 x WJ wavefronts of WT x WT each,
-// SLOTS ring stages, WGS workgroups per CU.
-template <int TBI_, int TBJ_, int WJ_, int SLOTS_, int WGS_> struct Tiling {
-  static constexpr int TBI = TBI_, TBJ = TBJ_, WJ = WJ_, W = 2 * WJ_, SLOTS = SLOTS_, WGS = WGS_;
+// TBI x TBJ output tiles (rows i of L, rows j of R) of WI x WJ wavefronts, each owning
+// NI x NJ MFMA tiles; SLOTS ring stages, WGS workgroups per CU.
+template <int NI_, int NJ_, int WI_, int WJ_, int SLOTS_, int WGS_> struct Tiling {
+  static constexpr int NI = NI_, NJ = NJ_, WI = WI_, WJ = WJ_, W = WI_ * WJ_, SLOTS = SLOTS_, WGS = WGS_;
+  static constexpr int TBI = 16 * NI * WI, TBJ = 16 * NJ * WJ;
   static constexpr int RBI = TBI / 16, RBJ = TBJ / 16;   // 16-row (1 KB) blocks per operand tile
   static constexpr int PIECES = RBI + RBJ;               // 1 KB direct loads per k-step
   static constexpr int PMAX = (PIECES + W - 1) / W;      // per wavefront (the first PIECES % W one more)
   static constexpr int SLOT_ELEMS = (TBI + TBJ) * TK;
-  static_assert(TBI == 2 * WT && TBJ == WJ * WT, "wavefront grid");
   static_assert(SLOTS * SLOT_ELEMS * 2 * WGS <= 160 * 1024, "LDS budget");
+  static_assert(NJ % 2 == 0, "R fragments are read in pairs");
 };
-// 192 x 192, two independent workgroups per CU.
-using TileSquare = Tiling<192, 192, 2, 3, 2>;
-// 192 x 384, one workgroup of 8 wavefronts per CU: each R row band serves twice the
-// columns, so a k-step moves 36 instead of 48 KB of operands per CU for the same MFMAs.
-using TileWide = Tiling<192, 384, 4, 4, 1>;
+using TileWide = Tiling<6, 6, 2, 4, 4, 1>;     // 192 x 384, one workgroup of 8 wavefronts per CU
+using TileSquare = Tiling<6, 6, 2, 2, 3, 2>;   // 192 x 192, two of 4
+using TileHalf = Tiling<4, 4, 2, 4, 3, 2>;     // 128 x 256, two of 8
+using TileSmall = Tiling<2, 2, 2, 2, 4, 4>;    // 64 x 64, four of 4
 
 template <class T>
 __global__ __launch_bounds__(64 * T::W, T::WGS) void contraction_kernel(ContractionArgs a) {
-  constexpr int TBI = T::TBI, TBJ = T::TBJ, WJ = T::WJ, W = T::W, SLOTS = T::SLOTS;
+  constexpr int TBI = T::TBI, TBJ = T::TBJ, WJ = T::WJ, W = T::W, SLOTS = T::SLOTS, NI = T::NI, NJ = T::NJ;
   constexpr int RBI = T::RBI, PIECES = T::PIECES, PMAX = T::PMAX, SLOT_ELEMS = T::SLOT_ELEMS;
   __shared__ __attribute__((aligned(16))) bf16 lds[SLOTS * SLOT_ELEMS];
   const int n = a.n, ld = a.ld;
@@ -112,11 +112,11 @@ __global__ __launch_bounds__(64 * T::W, T::WGS) void contraction_kernel(Contract
   // grp ^ ((col >> 2) & 3).
   const int frag = col * TK + ((grp ^ ((col >> 2) & 3)) * 8);
 
-  f32x4 acc[NT][NT];   // [jt][it]: rows j (A operand = R), cols i (B operand = L)
+  f32x4 acc[NJ][NI];   // [jt][it]: rows j (A operand = R), cols i (B operand = L)
 #pragma unroll
-  for (int x = 0; x < NT; ++x)
+  for (int x = 0; x < NJ; ++x)
 #pragma unroll
-    for (int y = 0; y < NT; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int y = 0; y < NI; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int steps = ld / TK;
 #pragma unroll
@@ -133,52 +133,48 @@ __global__ __launch_bounds__(64 * T::W, T::WGS) void contraction_kernel(Contract
     if (s + SLOTS - 1 < steps) issue(s + SLOTS - 1, (s + SLOTS - 1) % SLOTS);
     const bf16 *tl = lds + (s % SLOTS) * SLOT_ELEMS, *tr = tl + TBI * TK;
     // All L fragments and the first two R fragments, then each pair of R fragments is read
-    // while the previous pair's 12 MFMAs run (scheduling barriers keep the compiler from
+    // while the previous pair's MFMAs run (scheduling barriers keep the compiler from
     // sinking the reads next to their use).
-    bf16x8 fl[NT], fr[NT];
+    bf16x8 fl[NI], fr[NJ];
 #pragma unroll
-    for (int y = 0; y < NT; ++y)
-      fl[y] = *reinterpret_cast<const bf16x8 *>(tl + (wi * WT + y * 16) * TK + frag);
+    for (int y = 0; y < NI; ++y)
+      fl[y] = *reinterpret_cast<const bf16x8 *>(tl + (wi * NI + y) * 16 * TK + frag);
 #pragma unroll
-    for (int x = 0; x < 2; ++x) fr[x] = *reinterpret_cast<const bf16x8 *>(tr + (wj * WT + x * 16) * TK + frag);
+    for (int x = 0; x < 2; ++x) fr[x] = *reinterpret_cast<const bf16x8 *>(tr + (wj * NJ + x) * 16 * TK + frag);
 #pragma unroll
-    for (int xp = 0; xp < NT / 2; ++xp) {
+    for (int xp = 0; xp < NJ / 2; ++xp) {
       __builtin_amdgcn_sched_barrier(0);
-      if (xp + 1 < NT / 2) {
+      if (xp + 1 < NJ / 2) {
 #pragma unroll
         for (int x = 2 * xp + 2; x < 2 * xp + 4; ++x)
-          fr[x] = *reinterpret_cast<const bf16x8 *>(tr + (wj * WT + x * 16) * TK + frag);
+          fr[x] = *reinterpret_cast<const bf16x8 *>(tr + (wj * NJ + x) * 16 * TK + frag);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int x = 2 * xp; x < 2 * xp + 2; ++x)
 #pragma unroll
-        for (int y = 0; y < NT; ++y) acc[x][y] = mfma16(fr[x], fl[y], acc[x][y]);
+        for (int y = 0; y < NI; ++y) acc[x][y] = mfma16(fr[x], fl[y], acc[x][y]);
     }
   }
 
-  // acc[x][y][e] = out[i = i0 + wi*96 + y*16 + col][j = j0 + wj*96 + x*16 + grp*4 + e],
-  // pair position pos = i n + j at res_offset (16 positions' channels contiguous).
-  auto at = [&](int64_t pos) { return a.out + res_offset(a.channels, int(ch), pos); };
-  const bool vec = (n % 4) == 0;                    // then pos % 4 == 0: 4 positions in one block
+  // acc[x][y][e] = out[i = i0 + (wi NI + y) 16 + col][j = j0 + (wj NJ + x) 16 + 4 grp + e]. A row
+  // of the result layout is a whole number of 16-position blocks, so the 4 positions of a
+  // lane are one 8-byte store whatever n is; the columns of the last block from n on are
+  // written too (finite, never read as results), the tile's columns beyond it are not.
+  bf16 *out = a.out + ch * 16 + grp * 4;
+  const int blocks = int(res_row_blocks(n));
 #pragma unroll
-  for (int y = 0; y < NT; ++y) {
-    const int i = i0 + wi * WT + y * 16 + col;
+  for (int y = 0; y < NI; ++y) {
+    const int i = i0 + (wi * NI + y) * 16 + col;
     if (i >= n) continue;
 #pragma unroll
-    for (int x = 0; x < NT; ++x) {
-      const int j = j0 + wj * WT + x * 16 + grp * 4;
-      const int64_t pos = int64_t(i) * n + j;
-      if (vec && j + 4 <= n) {
-        bf16x4 v;
+    for (int x = 0; x < NJ; ++x) {
+      const int jb = j0 / 16 + wj * NJ + x;
+      if (jb >= blocks) continue;
+      bf16x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = bf16(acc[x][y][e]);
-        *reinterpret_cast<bf16x4 *>(at(pos)) = v;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (j + e < n) *at(pos + e) = bf16(acc[x][y][e]);
-      }
+      for (int e = 0; e < 4; ++e) v[e] = bf16(acc[x][y][e]);
+      *reinterpret_cast<bf16x4 *>(out + (int64_t(i) * blocks + jb) * res_block_stride(a.channels)) = v;
     }
   }
 }
@@ -191,10 +187,30 @@ template <class T> int launch(const ContractionArgs &a, hipStream_t s) {
   return check_launch("contraction");
 }
 
-// Wide tiles up to N = 1024: measured (same box, libraries alternated) the C2 block (N=384)
-// 0.579 -> 0.553 ms and the N=768 contraction 155 -> 152 us; at N=1536 the square tile's
-// two independent workgroups per CU are 7% faster.
-constexpr int kWideTileMaxN = 1024;
+// Tile of an n x n product: the one with the least (rounds of workgroups) x (time of a round's
+// k-step). A last round that is partly empty counts half of what it leaves idle: its
+// workgroups have less company for the L2. The k-step weights are measured (us; all tiles
+// give the same bits): Wide 1.6; Square 1.44-1.6, above n = 1152 as fast as Wide or faster per
+// round; Half 1.4-1.57 up to n = 768 and 1.75-1.9 above (half again the operand bytes per MFMA);
+// Small 0.45 up to n = 384, 0.65-0.75 above. In us per launch, the tile taken against Wide up to n = 1024, Square above: n = 72
+// 4.3 (Small) / 6.7, 128 5.4 (Small) / 9.4, 256 13.0 (Small) / 18.0, 420 42.5 (Half) / 75.0, 509 49.8 (Half)
+// / 81.4, 576 81.8 (Square) / 89.9, 640 120.5 (Half) / 128.2, 900 307 (Square) / 331, 1100 470 (Wide) / 500; Wide
+// stays at 384 and 768 (26.1, 155).
+enum class Tile { Wide, Square, Half, Small };
+template <class T> double tile_cost(int64_t n, int64_t channels, int cus, double step_us) {
+  const int64_t wgs = ceil_div(n, T::TBI) * ceil_div(n, T::TBJ) * channels, slots = int64_t(cus) * T::WGS;
+  return step_us * 0.5 * (double(ceil_div(wgs, slots)) + std::max(1.0, double(wgs) / double(slots)));
+}
+Tile pick_tile(int64_t n, int64_t channels, int cus) {
+  const double cost[4] = {tile_cost<TileWide>(n, channels, cus, 1.6),
+                          tile_cost<TileSquare>(n, channels, cus, n <= 1152 ? 1.62 : 1.5),
+                          tile_cost<TileHalf>(n, channels, cus, n <= 768 ? 1.45 : 1.85),
+                          tile_cost<TileSmall>(n, channels, cus, n <= 384 ? 0.45 : 0.75)};
+  int best = 0;
+  for (int t = 1; t < 4; ++t)
+    if (cost[t] < cost[best]) best = t;
+  return Tile(best);
+}
 
 }  // namespace
 
@@ -203,13 +219,20 @@ int64_t contraction_operand_elems(int64_t n, int64_t channels) {
   return (contraction_ld(n) / TK) * op_step_stride(n, int(channels));
 }
 int64_t contraction_result_elems(int64_t n, int64_t channels) {
-  return ceil_div(n * n, 16) * res_block_stride(int(channels));
+  return n * res_row_blocks(n) * res_block_stride(int(channels));
 }
 
 int contraction(const ContractionArgs &a, hipStream_t s) {
   if (a.n == 0 || a.channels == 0) return XFH_OK;
   if (a.ld != contraction_ld(a.n)) return fail(XFH_EINVAL, "contraction: operand rows must be padded to 32");
-  return a.n <= kWideTileMaxN ? launch<TileWide>(a, s) : launch<TileSquare>(a, s);
+  int cus = 0;
+  XFH_TRY(device_cu_count(&cus));
+  switch (pick_tile(a.n, a.channels, cus)) {
+    case Tile::Wide: return launch<TileWide>(a, s);
+    case Tile::Square: return launch<TileSquare>(a, s);
+    case Tile::Half: return launch<TileHalf>(a, s);
+    default: return launch<TileSmall>(a, s);
+  }
 }
 
 }  // namespace xfh

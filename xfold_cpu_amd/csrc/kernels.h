@@ -219,8 +219,9 @@ int transition_pair_bias(const TransitionArgs &a, const TransitionBias &b, hipSt
 //     16 rows x 32 t (1 KB): block (t/32, i/16) holds the blocks of all channels together,
 //     element at ((t/32) * G + i/16) * op_group_stride + ch * 512 + (i % 16) * 32 + t % 32,
 //     G = ceil(n/16); zero for t >= n;
-//   result: element (ch, pos = i*n + j) at (pos/16) * res_block_stride + ch * 16 + pos % 16:
-//     16 pair positions, all channels of them contiguous (4 KB).
+//   result: element (ch, i, j) at (i * res_row_blocks + j/16) * res_block_stride + ch * 16 + j % 16:
+//     16 pair positions of a row, all channels of them contiguous (4 KB); a row's last block
+//     is filled up with values that are no results when n % 16 != 0.
 // The contraction reads each k-step of 16 rows as one contiguous 1 KB piece; trimul_project's
 // wavefronts write neighbouring grid lines of one k-slice at the same time (64-byte pieces
 // that fill whole rows of a block); trimul_output reads 16 positions' channels as one
@@ -236,9 +237,7 @@ __host__ __device__ inline int64_t op_offset(int64_t n, int c, int ch, int64_t i
   return (s * op_groups(n) + (i >> 4)) * op_group_stride(c) + int64_t(ch) * 512 + (i & 15) * 32;
 }
 __host__ __device__ inline int64_t res_block_stride(int c) { return int64_t(c) * 16 + kResPad; }
-__host__ __device__ inline int64_t res_offset(int c, int ch, int64_t pos) {
-  return (pos >> 4) * res_block_stride(c) + int64_t(ch) * 16 + (pos & 15);
-}
+__host__ __device__ inline int64_t res_row_blocks(int64_t n) { return (n + 15) / 16; }
 struct ContractionArgs {
   const bf16 *left, *right;  // blocked operand layout
   bf16 *out;                 // blocked result layout

@@ -161,10 +161,12 @@ __global__ __launch_bounds__(512, 1) void trimul_output_kernel(TriOutputArgs a) 
   sl_in.load(a.ln_in_w, a.ln_in_b);
   sl_c.load(a.ln_c_w, a.ln_c_b);
 
-  const int64_t npos = int64_t(a.n) * a.n;
-  const int64_t steps = (npos + 15) / 16;
+  // Step st = block st of the result layout: positions j = 16 (st % row_blocks) .. + 15 of
+  // row i = st / row_blocks (those from n on exist in the layout only).
+  const int n = a.n, row_blocks = int(res_row_blocks(n));
+  const int steps = n * row_blocks;                 // < 2^31 (n * n does, and row_blocks <= n)
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const int64_t waves = int64_t(gridDim.x) * (blockDim.x >> 6);
+  const int waves = int(gridDim.x) * int(blockDim.x >> 6);
   const TIN *z = static_cast<const TIN *>(a.pair);
   TOUT *out = static_cast<TOUT *>(a.out);
   constexpr bool kBf16 = sizeof(TIN) == 2 && sizeof(TOUT) == 2;
@@ -178,29 +180,19 @@ __global__ __launch_bounds__(512, 1) void trimul_output_kernel(TriOutputArgs a) 
     bf16x8 c[4];                                   // see fetch
     rowstep::Raw4<TOUT> res[8];                    // O-layout (only when not derived from z)
   };
-  auto fetch = [&](int64_t st, Rows &rw) {
-    const int64_t pos = st * 16 + r, pc = pos < npos ? pos : npos - 1;
+  auto fetch = [&](int st, Rows &rw) {
+    const int i = st / row_blocks, j = (st - i * row_blocks) * 16 + r;
+    const int64_t pc = int64_t(i) * n + (j < n ? j : n - 1);
     rowstep::load_k<TIN>(z + pc * K, rw.z);
     // c[q]: channel 16 q + r (g < 2) or 16 (q + 4) + r (g >= 2), positions 8 (g % 2) .. +7
     // of the step: k = 8 g + j of an A fragment whose k-halves hold tiles q and q + 4.
-    const int64_t p0 = st * 16 + 8 * (g & 1);
+    const bf16 *src = a.contracted + st * res_block_stride(K) + (64 * (g >> 1) + r) * 16 + 8 * (g & 1);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const bf16 *src = a.contracted + res_offset(K, 16 * (q + 4 * (g >> 1)) + r, p0);
-      bf16x8 v = {};
-      if (p0 + 8 <= npos) {
-        v = *reinterpret_cast<const bf16x8 *>(src);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (p0 + j < npos) v[j] = src[j];
-      }
-      rw.c[q] = v;
-    }
+    for (int q = 0; q < 4; ++q) rw.c[q] = *reinterpret_cast<const bf16x8 *>(src + q * 256);
     if (res_load) rowstep::load_o<TOUT>(out + pc * K, rw.res);
   };
 
-  int64_t st = int64_t(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  int st = int(blockIdx.x) * int(blockDim.x >> 6) + int(threadIdx.x >> 6);
   Rows cur;
   if (st < steps) fetch(st, cur);                   // in flight while the weights are stored
   sg.store(w_gate);
@@ -277,8 +269,9 @@ __global__ __launch_bounds__(512, 1) void trimul_output_kernel(TriOutputArgs a) 
 #pragma unroll
         for (int e = 0; e < 4; ++e) res[t][e] = res_load ? cur.res[t][e] : 0.f;
     }
-    const int64_t pos = st * 16 + r;
-    if (pos < npos) {
+    const int i = st / row_blocks, j = (st - i * row_blocks) * 16 + r;
+    if (j < n) {
+      const int64_t pos = int64_t(i) * n + j;
 #pragma unroll
       for (int t = 0; t < 8; ++t) {
         float o[4];
@@ -297,10 +290,13 @@ int trimul_project(const TriProjectArgs &a, int pair_dtype, hipStream_t s) {
   if (a.ld != contraction_ld(a.n)) return fail(XFH_EINVAL, "trimul_project: ld must be contraction_ld(n)");
   int cus = 0;
   XFH_TRY(device_cu_count(&cus));
-  // 32-position units unless that leaves fewer than four per wavefront (the last round of
-  // units would then run on a fraction of the wavefronts).
+  // 32-position units take 1.75 times a 16-position unit's time (the weight fragments are read
+  // once for both row tiles), so they win unless 16-position units need few enough more
+  // rounds: n = 509 59.3 us (32) against 69.2 (16), 900 168 / 301, 256 18.3 / 18.8; 160 19.8 / 16.3,
+  // 384 37.3 / 35.5.
   const int64_t units32 = int64_t(a.n) * (a.ld / 32);
-  const bool wide = units32 >= int64_t(cus) * 8 * 4;
+  const int64_t slots = int64_t(cus) * 8;
+  const bool wide = 1.75 * double(ceil_div(units32, slots)) <= double(ceil_div(2 * units32, slots));
   const int64_t units = wide ? units32 : 2 * units32;
   const dim3 grid(unsigned(balanced_grid(units, 8, cus)));
   KernelTimer timer("trimul_project", s, 0.0, true);
@@ -315,7 +311,7 @@ int trimul_project(const TriProjectArgs &a, int pair_dtype, hipStream_t s) {
 }
 
 int trimul_output(const TriOutputArgs &a, int pair_dtype, int out_dtype, hipStream_t s) {
-  const int64_t steps = ceil_div(int64_t(a.n) * a.n, 16);
+  const int64_t steps = int64_t(a.n) * res_row_blocks(a.n);
   int cus = 0;
   XFH_TRY(device_cu_count(&cus));
   const dim3 grid(unsigned(balanced_grid(steps, 8, cus)));
