@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define XFH_ABI_VERSION 9
+#define XFH_ABI_VERSION 10
 
 enum { XFH_F32 = 0, XFH_BF16 = 1, XFH_BOOL = 2 };
 enum { XFH_OK = 0, XFH_EINVAL = 1, XFH_EUNSUPPORTED = 2, XFH_EWORKSPACE = 3, XFH_EHIP = 4 };
@@ -194,6 +194,80 @@ int xfh_attention_mask_words(const void *mask, int mask_dtype, int64_t mask_stri
 int xfh_attention_operands(const void *q, const void *k, const void *vt, const uint64_t *words, int words_shared,
                            const void *bias, int bias_dtype, const void *gate, void *out, int64_t B, int64_t T,
                            int64_t H, int64_t Dh, void *stream);
+
+/* Weights of xfh_pair_updates (host struct of device pointers, as the single entry points take them). */
+typedef struct XfhPairWeights {
+  struct {
+    const float *norm_w, *norm_b, *center_w, *center_b;
+    const void *projection, *gate, *output, *gating;
+  } triangle[2];
+  struct {
+    const float *norm_w, *norm_b;
+    const void *bias, *q, *k, *v, *gating, *output;
+  } grid[2];
+  struct {
+    const float *norm_w, *norm_b;
+    const void *w1_packed, *w2;
+  } transition;
+} XfhPairWeights;
+
+/* The pair updates of PairformerBlock.forward (xfold/nn/pairformer.py:96-100) in place: two triangle
+ * multiplications (directions outgoing[0..1]), two grid attentions (transpose[0..1]) and, when f > 0,
+ * the transition: xfh_triangle_multiplication, xfh_grid_self_attention and xfh_transition one after
+ * the other on one workspace. eps: the LayerNorms' in the struct's order (2, 2, 1, 1, 1). */
+int64_t xfh_pair_updates_workspace_size(int64_t n, int64_t c, int64_t heads, int64_t f, int dtype);
+int xfh_pair_updates(void *pair, int pair_dtype, const void *mask, int mask_dtype, int64_t n, int64_t c,
+                     int64_t heads, int64_t f, const int *outgoing, const int *transpose,
+                     const XfhPairWeights *weights, const float *eps, int dtype, void *workspace,
+                     int64_t workspace_bytes, void *stream);
+
+/* Weights of xfh_pairformer_single (host struct). */
+typedef struct XfhSingleWeights {
+  const float *pair_norm_w, *pair_norm_b;          /* the pair transition */
+  const void *pair_w1_packed, *pair_w2;
+  const float *logits_norm_w, *logits_norm_b;      /* the pair logits */
+  const void *logits_w;
+  const float *attention_norm_w, *attention_norm_b;
+  const void *w_qkvg;
+  const float *b_qkvg;
+  const void *w_attention_out;
+  const float *transition_norm_w, *transition_norm_b;
+  const void *w1_packed, *w2;
+} XfhSingleWeights;
+
+/* The rest of PairformerBlock.forward with a single track (xfold/nn/pairformer.py:100-113), bf16 compute:
+ * xfh_transition_pair_bias on the bf16 pair [n][n][128], then single [n][c] (fp32 or bf16, c = heads * Dh)
+ * += SelfAttention(single) with those logits (xfh_layer_norm, xfh_attention_project,
+ * xfh_attention_operands, xfh_linear) and += Transition(single) (f hidden features). eps: the four
+ * LayerNorms' in the struct's order; q, k, vt, gate and words as for xfh_attention_operands. */
+int64_t xfh_pairformer_single_workspace_size(int64_t n, int64_t c, int64_t heads, int64_t f);
+int xfh_pairformer_single(void *pair, void *single, int single_dtype, int64_t n, int64_t c, int64_t heads, int64_t f,
+                          const XfhSingleWeights *weights, const float *eps, float qscale, void *q, void *k, void *vt,
+                          void *gate, const uint64_t *words, void *workspace, int64_t workspace_bytes, void *stream);
+
+/* One block of xfh_diffusion_blocks: the stacked [Wq; Wk; Wv; Wg] weight [4c][c] (fp32 bias [4c] or
+ * NULL), its packed logits [H][T][Tpad], the attention's and the transition's AdaLNZero weights
+ * [c][c] and [c][f], the packed transition1 weight (xfh_glu_pack_weight); the conditioning
+ * [cond_rows][c]: scale and shift in bf16, the AdaLNZero conditions in act's dtype. */
+typedef struct XfhDiffusionBlock {
+  const void *w_qkvg;
+  const float *b_qkvg;
+  const void *logits, *w_attention_out, *w_glu, *w_transition_out;
+  const void *attention_scale, *attention_shift, *attention_zero;
+  const void *transition_scale, *transition_shift, *transition_zero;
+  float attention_eps, transition_eps;
+} XfhDiffusionBlock;
+
+/* The blocks of DiffusionTransformer.forward (xfold/nn/diffusion_transformer.py:266-271), bf16 compute:
+ * for each of the n_blocks host structs, act += SelfAttention(act), act += DiffusionTransition(act)
+ * (act [B][T][c] fp32 or bf16, c = H*Dh, f hidden features). The same kernels and results as
+ * xfh_adaptive_layer_norm, xfh_attention_project, xfh_attention_operands, xfh_linear and
+ * xfh_gated_linear_unit called block by block; q, k, vt, gate and words as for them. */
+int64_t xfh_diffusion_blocks_workspace_size(int64_t rows, int64_t c, int64_t f);
+int xfh_diffusion_blocks(void *act, int act_dtype, int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t f,
+                         int64_t cond_rows, const XfhDiffusionBlock *blocks, int64_t n_blocks, int bias_dtype,
+                         float qscale, void *q, void *k, void *vt, void *gate, const uint64_t *words,
+                         int words_shared, void *workspace, int64_t workspace_bytes, void *stream);
 
 /* Linear(LayerNorm(pair)) rearranged 'i j h -> h i j' straight into a packed bias layout:
  * with out_dtype XFH_F32, packed[h][i][j] fp32 = log2(e) * (LN(pair[i][j]) . w[h]) (the

@@ -175,6 +175,45 @@ def test_derived_weight_rebuilds_when_a_source_changes():
     assert len(calls) == 5                            # inference tensors are never cached
 
 
+def test_gathered_weights_follow_every_change_of_a_source():
+    """A module's prepared weights are checked as a group: rebuilt after an in-place update, a
+    new Parameter, a .data swap or transposed .data, a new dtype, and in a copied module."""
+    import copy
+    module = torch.nn.Module()
+    module.lin = torch.nn.Linear(4, 4, bias=False)
+    x = torch.zeros(1)
+
+    def get(m=module, x=x):
+        return nh.gather(m, "t", nh.params(m, ("lin",)), 1, x, lambda dt: nh.linear_weight(m, "lin", dt).clone())
+
+    with torch.no_grad():
+        assert get()[0] == torch.float32
+        first = get()
+        assert get()[1] is first[1]
+        changes = (lambda: module.lin.weight.mul_(2),
+                   lambda: setattr(module.lin, "weight", torch.nn.Parameter(torch.randn(4, 4))),
+                   lambda: setattr(module.lin.weight, "data", torch.randn(4, 4)),
+                   lambda: setattr(module.lin.weight, "data", module.lin.weight.data.t()))
+        for change in changes:
+            change()
+            torch.testing.assert_close(get()[1], module.lin.weight.detach())
+        with pytest.raises(ValueError, match="dtypes must match"):
+            get(x=x.bfloat16())
+        twin = copy.deepcopy(module)
+        twin.lin.weight.mul_(3)
+        torch.testing.assert_close(get(twin)[1], twin.lin.weight.detach())
+        module.lin.weight.data = module.lin.weight.data.bfloat16()
+        assert get(x=x.bfloat16())[1].dtype == torch.bfloat16
+        again = [nh.gather(module, "u", nh.params(module, ("lin",)), 1, x.bfloat16(), lambda dt: dt, again=True)[1]
+                 for _ in range(3)]
+        assert again == [None, torch.bfloat16, torch.bfloat16]      # built from the second pass on
+    with torch.inference_mode():
+        module.lin.weight = torch.nn.Parameter(torch.randn(4, 4), requires_grad=False)
+        got = get()[1]
+        module.lin.weight.mul_(2)
+        assert not torch.equal(get()[1], got)             # no version counter: never kept
+
+
 @pytest.mark.parametrize("fixture,cls", [
     ("pairformer_block", "PairformerBlock"), ("diffusion_transformer", "DiffusionTransformer"),
     ("grid_attention_start", "GridSelfAttention"), ("self_attention_cond", "SelfAttention"),

@@ -455,6 +455,43 @@ int xfh_attention_operands(const void *q, const void *k, const void *vt, const u
                             static_cast<bf16 *>(out), B, T, H, Dh, as_stream(stream));
 }
 
+int64_t xfh_diffusion_blocks_workspace_size(int64_t rows, int64_t c, int64_t f) {
+  if (rows < 0 || c < 0 || f < 0) return -1;
+  return 2 * align_up(rows * c * 2, 256) + align_up(rows * f * 2, 256) + 256;
+}
+
+int xfh_diffusion_blocks(void *act, int act_dtype, int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t f,
+                         int64_t cond_rows, const XfhDiffusionBlock *blocks, int64_t n_blocks, int bias_dtype,
+                         float qscale, void *q, void *k, void *vt, void *gate, const uint64_t *words,
+                         int words_shared, void *workspace, int64_t workspace_bytes, void *stream) {
+  XFH_REQUIRE(B >= 0 && T >= 0 && H > 0 && Dh > 0 && f > 0 && n_blocks >= 0, "diffusion_blocks: bad size");
+  XFH_REQUIRE(float_dtype(act_dtype), "diffusion_blocks: act must be f32/bf16");
+  XFH_REQUIRE(cond_rows > 0 && (B * T) % cond_rows == 0, "diffusion_blocks: the conditions' rows must tile act's");
+  if (B * T == 0 || n_blocks == 0) return XFH_OK;
+  XFH_REQUIRE(act && blocks && gate, "diffusion_blocks: null tensor");
+  const int64_t rows = B * T, c = H * Dh;
+  Carver cv(workspace, workspace_bytes);
+  void *normed = cv.take(rows * c * 2), *attended = cv.take(rows * c * 2), *hidden = cv.take(rows * f * 2);
+  if (!workspace || cv.used > workspace_bytes)
+    return fail(XFH_EWORKSPACE, "diffusion_blocks: workspace too small (need " + std::to_string(cv.used) + " bytes)");
+  for (int64_t i = 0; i < n_blocks; ++i) {
+    const XfhDiffusionBlock &b = blocks[i];
+    XFH_TRY(xfh_adaptive_layer_norm(act, act_dtype, rows, c, b.attention_scale, b.attention_shift, XFH_BF16, cond_rows,
+                                    b.attention_eps, normed, XFH_BF16, stream));
+    XFH_TRY(xfh_attention_project(normed, c, b.w_qkvg, b.b_qkvg, B, T, c, H, Dh, qscale, q, k, vt, gate, stream));
+    XFH_TRY(xfh_attention_operands(q, k, vt, words, words_shared, b.logits, bias_dtype, gate, attended, B, T, H, Dh,
+                                   stream));
+    XFH_TRY(xfh_linear(attended, c, b.w_attention_out, nullptr, rows, c, c, XFH_BF16, act, c, act_dtype,
+                       XFH_EPI_MUL_SIGMOID_AUX_ACCUMULATE, b.attention_zero, c, cond_rows, stream));
+    XFH_TRY(xfh_adaptive_layer_norm(act, act_dtype, rows, c, b.transition_scale, b.transition_shift, XFH_BF16,
+                                    cond_rows, b.transition_eps, normed, XFH_BF16, stream));
+    XFH_TRY(xfh_gated_linear_unit(normed, b.w_glu, rows, c, f, XFH_BF16, hidden, XFH_BF16, stream));
+    XFH_TRY(xfh_linear(hidden, f, b.w_transition_out, nullptr, rows, f, c, XFH_BF16, act, c, act_dtype,
+                       XFH_EPI_MUL_SIGMOID_AUX_ACCUMULATE, b.transition_zero, c, cond_rows, stream));
+  }
+  return XFH_OK;
+}
+
 int xfh_pair_attention_bias(const void *pair, int pair_dtype, int64_t n, int64_t c, const float *ln_w,
                             const float *ln_b, float eps, const void *w, int w_dtype, int64_t heads,
                             void *packed, int out_dtype, void *stream) {
@@ -748,6 +785,78 @@ int xfh_transition_pair_bias(void *pair, int64_t n, int64_t c, int64_t f, const 
   tb.ln_w = bias_ln_w; tb.ln_b = bias_ln_b; tb.eps = bias_eps; tb.w = static_cast<const bf16 *>(bias_w);
   tb.packed = packed; tb.n = int(n); tb.npad = int(align_up(n, 64)); tb.heads = int(heads);
   return transition_pair_bias(ta, tb, as_stream(stream));
+}
+
+int64_t xfh_pair_updates_workspace_size(int64_t n, int64_t c, int64_t heads, int64_t f, int dtype) {
+  if (f < 0) return -1;
+  const int64_t need[3] = {xfh_triangle_multiplication_workspace_size(n, c, dtype),
+                           xfh_grid_self_attention_workspace_size(n, c, heads, dtype),
+                           f > 0 ? xfh_transition_workspace_size(n * n, c, f, dtype) : 0};
+  int64_t most = 0;
+  for (int64_t v : need) {
+    if (v < 0) return -1;
+    most = v > most ? v : most;
+  }
+  return most;
+}
+
+int xfh_pair_updates(void *pair, int pair_dtype, const void *mask, int mask_dtype, int64_t n, int64_t c,
+                     int64_t heads, int64_t f, const int *outgoing, const int *transpose,
+                     const XfhPairWeights *weights, const float *eps, int dtype, void *workspace,
+                     int64_t workspace_bytes, void *stream) {
+  XFH_REQUIRE(outgoing && transpose && weights && eps, "pair_updates: null argument");
+  for (int i = 0; i < 2; ++i) {
+    const auto &w = weights->triangle[i];
+    XFH_TRY(xfh_triangle_multiplication(pair, pair_dtype, mask, mask_dtype, n, c, outgoing[i], w.norm_w, w.norm_b,
+                                        eps[2 * i], w.projection, w.gate, w.center_w, w.center_b, eps[2 * i + 1],
+                                        w.output, w.gating, dtype, pair, pair_dtype, 1, workspace, workspace_bytes,
+                                        stream));
+  }
+  for (int i = 0; i < 2; ++i) {
+    const auto &w = weights->grid[i];
+    XFH_TRY(xfh_grid_self_attention(pair, pair_dtype, mask, mask_dtype, n, c, heads, transpose[i], w.norm_w, w.norm_b,
+                                    eps[4 + i], w.bias, w.q, w.k, w.v, w.gating, w.output, dtype, pair, pair_dtype, 1,
+                                    workspace, workspace_bytes, stream));
+  }
+  if (f <= 0) return XFH_OK;
+  const auto &w = weights->transition;
+  return xfh_transition(pair, pair_dtype, n * n, c, f, w.norm_w, w.norm_b, eps[6], w.w1_packed, w.w2, dtype, pair,
+                        pair_dtype, 1, workspace, workspace_bytes, stream);
+}
+
+int64_t xfh_pairformer_single_workspace_size(int64_t n, int64_t c, int64_t heads, int64_t f) {
+  if (n < 0 || c < 0 || heads < 0 || f < 0) return -1;
+  return align_up(heads * n * align_up(n, 64) * 4, 256) + 2 * align_up(n * c * 2, 256) +
+         xfh_transition_workspace_size(n, c, f, XFH_BF16) + 256;
+}
+
+int xfh_pairformer_single(void *pair, void *single, int single_dtype, int64_t n, int64_t c, int64_t heads, int64_t f,
+                          const XfhSingleWeights *weights, const float *eps, float qscale, void *q, void *k, void *vt,
+                          void *gate, const uint64_t *words, void *workspace, int64_t workspace_bytes, void *stream) {
+  XFH_REQUIRE(n >= 0 && c > 0 && heads > 0 && f > 0 && c % heads == 0, "pairformer_single: bad size");
+  XFH_REQUIRE(float_dtype(single_dtype), "pairformer_single: single must be f32/bf16");
+  if (n == 0) return XFH_OK;
+  XFH_REQUIRE(pair && single && weights && eps && gate, "pairformer_single: null argument");
+  Carver cv(workspace, workspace_bytes);
+  float *packed = static_cast<float *>(cv.take(heads * n * align_up(n, 64) * 4));
+  void *normed = cv.take(n * c * 2), *attended = cv.take(n * c * 2);
+  const int64_t rest = xfh_transition_workspace_size(n, c, f, XFH_BF16);
+  void *transition_ws = cv.take(rest);
+  if (!workspace || cv.used > workspace_bytes)
+    return fail(XFH_EWORKSPACE, "pairformer_single: workspace too small (need " + std::to_string(cv.used) + " bytes)");
+  const XfhSingleWeights &w = *weights;
+  XFH_TRY(xfh_transition_pair_bias(pair, n, 128, 512, w.pair_norm_w, w.pair_norm_b, eps[0], w.pair_w1_packed, w.pair_w2,
+                                   w.logits_norm_w, w.logits_norm_b, eps[1], w.logits_w, heads, packed, stream));
+  XFH_TRY(xfh_layer_norm(single, single_dtype, n, c, w.attention_norm_w, w.attention_norm_b, eps[2], normed, XFH_BF16,
+                         stream));
+  XFH_TRY(xfh_attention_project(normed, c, w.w_qkvg, w.b_qkvg, 1, n, c, heads, c / heads, qscale, q, k, vt, gate,
+                                stream));
+  XFH_TRY(xfh_attention_operands(q, k, vt, words, 1, packed, XFH_BIAS_PACKED, gate, attended, 1, n, heads, c / heads,
+                                 stream));
+  XFH_TRY(xfh_linear(attended, c, w.w_attention_out, nullptr, n, c, c, XFH_BF16, single, c, single_dtype,
+                     XFH_EPI_ACCUMULATE, nullptr, 0, 0, stream));
+  return xfh_transition(single, single_dtype, n, c, f, w.transition_norm_w, w.transition_norm_b, eps[3], w.w1_packed,
+                        w.w2, XFH_BF16, single, single_dtype, 1, transition_ws, rest, stream);
 }
 
 }  // extern "C"

@@ -28,7 +28,7 @@ from typing import Optional
 import torch
 
 LIBRARY_PATH = Path(__file__).resolve().parent.parent / "lib" / "libxfold_hip.so"
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 F32, BF16, BOOL = 0, 1, 2
 BIAS_PACKED = 3                 # bias 'dtype' of a packed fp32 block (times log2(e))
@@ -62,6 +62,13 @@ SIGNATURES = {
     "xfh_attention_project": (_i, [_p, _i64, _p, _p, _i64, _i64, _i64, _i64, _i64, _f, _p, _p, _p, _p, _p]),
     "xfh_attention_mask_words": (_i, [_p, _i, _i64, _i64, _i64, _p, _p]),
     "xfh_attention_operands": (_i, [_p, _p, _p, _p, _i, _p, _i, _p, _p, _i64, _i64, _i64, _i64, _p]),
+    "xfh_pair_updates_workspace_size": (_i64, [_i64, _i64, _i64, _i64, _i]),
+    "xfh_pair_updates": (_i, [_p, _i, _p, _i, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _i, _p, _i64, _p]),
+    "xfh_pairformer_single_workspace_size": (_i64, [_i64, _i64, _i64, _i64]),
+    "xfh_pairformer_single": (_i, [_p, _p, _i, _i64, _i64, _i64, _i64, _p, _p, _f, _p, _p, _p, _p, _p, _p, _i64, _p]),
+    "xfh_diffusion_blocks_workspace_size": (_i64, [_i64, _i64, _i64]),
+    "xfh_diffusion_blocks": (_i, [_p, _i, _i64, _i64, _i64, _i64, _i64, _i64, _p, _i64, _i, _f, _p, _p, _p, _p, _p, _i,
+                                  _p, _i64, _p]),
     "xfh_pair_attention_bias": (_i, [_p, _i, _i64, _i64, _p, _p, _f, _p, _i, _i64, _p, _i, _p]),
     "xfh_triangle_multiplication_workspace_size": (_i64, [_i64, _i64, _i]),
     "xfh_triangle_multiplication": (_i, [_p, _i, _p, _i, _i64, _i64, _i, _p, _p, _f, _p, _p, _p, _p,
@@ -111,6 +118,15 @@ def load_library(path: Optional[str] = None) -> ctypes.CDLL:
     return lib
 
 
+class DiffusionBlock(ctypes.Structure):
+    """``XfhDiffusionBlock`` of include/xfold_hip.h."""
+    _fields_ = [(name, ctypes.c_void_p) for name in
+                ("w_qkvg", "b_qkvg", "logits", "w_attention_out", "w_glu", "w_transition_out",
+                 "attention_scale", "attention_shift", "attention_zero",
+                 "transition_scale", "transition_shift", "transition_zero")] + [
+               ("attention_eps", ctypes.c_float), ("transition_eps", ctypes.c_float)]
+
+
 def call(name: str, *args) -> None:
     lib = load_library()
     status = getattr(lib, name)(*args)
@@ -152,6 +168,9 @@ def runtime_info() -> str:
 
 # ------------------------------------------------------------------------- tensor helpers
 
+_FLOATS = frozenset((torch.float32, torch.bfloat16))
+
+
 def dtype_code(dtype: torch.dtype) -> int:
     if dtype == torch.float32:
         return F32
@@ -175,16 +194,19 @@ def check_gpu_inference(*tensors) -> None:
 
 def compute_dtype(x: torch.Tensor, *weights: torch.Tensor) -> torch.dtype:
     """Compute dtype per reference ``native.py:31-43``, reading the CUDA autocast state."""
-    for tensor in (x, *weights):
-        if tensor.dtype not in (torch.float32, torch.bfloat16):
-            raise ValueError("The 'hip' backend supports FP32/BF16 only.")
+    return _compute_dtype(x.dtype, [w.dtype for w in weights])
+
+
+def _compute_dtype(x: torch.dtype, weights) -> torch.dtype:
+    if x not in _FLOATS or not _FLOATS.issuperset(weights):
+        raise ValueError("The 'hip' backend supports FP32/BF16 only.")
     if torch.is_autocast_enabled("cuda"):
         dtype = torch.get_autocast_dtype("cuda")
     else:
-        dtype = x.dtype
-        if any(w.dtype != dtype for w in weights):
+        dtype = x
+        if any(w != dtype for w in weights):
             raise ValueError("Input/weight dtypes must match outside autocast.")
-    if dtype not in (torch.float32, torch.bfloat16):
+    if dtype not in _FLOATS:
         raise ValueError("The 'hip' backend supports FP32/BF16 autocast only.")
     return dtype
 
@@ -204,6 +226,11 @@ def ptr(tensor: Optional[torch.Tensor]) -> Optional[int]:
     if not tensor.is_cuda:
         raise ValueError("The 'hip' backend requires strided ROCm (cuda) tensors.")
     return tensor.data_ptr()
+
+
+def ptrs(tensors) -> ctypes.Array:
+    """A host struct of device pointers (the pointer-only structs of include/xfold_hip.h)."""
+    return (ctypes.c_void_p * len(tensors))(*map(ptr, tensors))
 
 
 def stream_of(device: torch.device) -> int:
@@ -360,3 +387,79 @@ def fp32_param(module: torch.nn.Module, name: str, param: Optional[torch.Tensor]
     if param.dtype == torch.float32 and param.is_contiguous():
         return param.detach()
     return module_cache(module, name).get(param, torch.float32)
+
+
+_MISSING = object()
+
+
+def param(module: torch.nn.Module, name: str, attr: str = "weight") -> Optional[torch.Tensor]:
+    """``module.<name>.<attr>`` read from the registration tables (``nn.Module.__getattr__``
+    takes several times as long), or as an attribute where it is not a plain parameter."""
+    sub = module._modules.get(name)
+    value = _MISSING if sub is None else sub._parameters.get(attr, _MISSING)
+    return getattr(getattr(module, name), attr) if value is _MISSING else value
+
+
+def params(module: torch.nn.Module, names, norms=()) -> list:
+    """The weights of ``names``, then weight and bias of each LayerNorm of ``norms``."""
+    out = [param(module, name) for name in names]
+    for name in norms:
+        out += (param(module, name), param(module, name, "bias"))
+    return out
+
+
+class WeightGroup:
+    """The prepared weights of one module call, checked as a whole: the same key per source as
+    :class:`HipWeightCache`, compared once. The sources are held, so no address of the key can
+    pass to another tensor; a copied or pickled module starts with an empty group."""
+
+    __slots__ = ("key", "sources", "dtypes", "values")
+
+    def __init__(self):
+        self.key = self.sources = self.dtypes = self.values = None
+
+    def __reduce__(self):
+        return WeightGroup, ()
+
+
+def gather(module: torch.nn.Module, tag: str, sources, weights: int, x: torch.Tensor, build,
+           dtype: Optional[torch.dtype] = None, again: bool = False):
+    """(compute dtype, ``build(dtype)``) of a module's ``sources`` (parameters or None), the first
+    ``weights`` of which take part in :func:`compute_dtype` (unless ``dtype`` is given). ``build``
+    runs again when a source or the dtype has changed; its values are kept for one dtype.
+
+    The first pass over a module keeps nothing and takes no key: its weights are being prepared
+    (each in its own cache) while the GPU waits. ``again``: the values are None on that pass and
+    on the first one after a change, when a whole block's weights are prepared operator by
+    operator behind the operators already queued; the block's one call starts with the next."""
+    groups = module.__dict__.setdefault("_hip_weight_groups", {})
+    group = groups.get(tag)
+    if group is None:
+        groups[tag] = WeightGroup()
+        dtype = dtype or _compute_dtype(x.dtype, [p.dtype for p in sources[:weights]])
+        return dtype, None if again else build(dtype)
+    try:
+        key = [None if p is None else (p.data_ptr(), p._version, p.shape, p.stride(), p.dtype, p.device)
+               for p in sources]
+    except RuntimeError:                             # inference tensors carry no version: nothing is kept
+        dtype = dtype or _compute_dtype(x.dtype, [p.dtype for p in sources[:weights]])
+        return dtype, None if again else build(dtype)
+    changed = group.key is not None and group.key != key
+    if changed or group.key is None:
+        group = WeightGroup()
+        group.key, group.sources = key, sources
+        group.dtypes = {p.dtype for p in sources[:weights]}
+        groups[tag] = group
+    dtype = dtype or _compute_dtype(x.dtype, group.dtypes)
+    values = group.values
+    if values is None or values[0] != dtype:
+        if again and changed:
+            return dtype, None
+        values = group.values = (dtype, build(dtype))
+    return values
+
+
+def norm_params(module: torch.nn.Module, name: str) -> tuple:
+    """fp32 weight and bias of LayerNorm ``module.<name>``."""
+    return (fp32_param(module, name + ".weight", param(module, name)),
+            fp32_param(module, name + ".bias", param(module, name, "bias")))

@@ -312,6 +312,23 @@ def attention_on_operands(operands: AttentionOperands, bias: PackedBias, out: to
     return out
 
 
+def diffusion_blocks(act: torch.Tensor, operands: AttentionOperands, blocks, cond_rows: int, f: int,
+                     bias_dtype: torch.dtype) -> None:
+    """Every block of a diffusion transformer in one library call (``xfh_diffusion_blocks``): act
+    [B, T, c] in place, ``blocks`` an array of :class:`native_hip.DiffusionBlock` whose tensors the
+    caller holds."""
+    B, T, H, Dh = operands.shape
+    if not act.is_contiguous() or act.numel() != B * T * H * Dh or act.numel() // (H * Dh) % cond_rows:
+        raise ValueError("diffusion_blocks: act must be a contiguous [B, T, H*Dh], its rows a multiple of the conditions'")
+    lib = nh.load_library()
+    ws = nh.workspace(lib.xfh_diffusion_blocks_workspace_size(B * T, H * Dh, f), act.device)
+    code = nh.BIAS_PACKED if bias_dtype == torch.float32 else nh.BIAS_PACKED_BF16
+    nh.call("xfh_diffusion_blocks", nh.ptr(act), nh.dtype_code(act.dtype), B, T, H, Dh, f, cond_rows, blocks,
+            len(blocks), code, Dh ** -0.5 * 1.4426950408889634, nh.ptr(operands.q), nh.ptr(operands.k),
+            nh.ptr(operands.vt), nh.ptr(operands.gate), nh.ptr(operands.words), int(operands.words_shared), nh.ptr(ws),
+            ws.numel(), nh.stream_of(act.device))
+
+
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optional[torch.Tensor],
               bias: Optional[torch.Tensor], out: Optional[torch.Tensor] = None,
               scale: Optional[float] = None, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:

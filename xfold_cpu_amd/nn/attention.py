@@ -24,17 +24,15 @@ def grid_self_attention_hip(module: nn.Module, pair: torch.Tensor, mask: Optiona
     first axis with the mask unchanged; the result is in pair layout."""
     nh.check_gpu_inference(pair, mask)
     nh.check_module(module)
-    dtype = nh.compute_dtype(pair, *(getattr(module, n).weight for n in _GRID_WEIGHTS))
+    dtype, (w, nw, nb) = nh.gather(
+        module, "grid_self_attention", nh.params(module, _GRID_WEIGHTS, ("act_norm",)), len(_GRID_WEIGHTS), pair,
+        lambda dt: ([nh.linear_weight(module, n, dt) for n in _GRID_WEIGHTS], *nh.norm_params(module, "act_norm")))
     if pair.dim() != 3 or pair.shape[0] != pair.shape[1] or pair.shape[2] != module.c_pair:
         raise ValueError("GridSelfAttention expects pair [N, N, c_pair].")
     n, c = pair.shape[0], pair.shape[2]
     heads = module.num_head
     pair_c = pair.contiguous()
     mask_t, mask_code = nh.mask_arg(mask, (n, n)) if mask is not None else (None, nh.BOOL)
-    w = {name: nh.linear_weight(module, name, dtype) for name in _GRID_WEIGHTS}
-    norm = module.act_norm
-    nw = nh.fp32_param(module, "norm_w", norm.weight)
-    nb = nh.fp32_param(module, "norm_b", norm.bias)
     if accumulate_into is not None:
         out, accumulate = accumulate_into, 1
         if not out.is_contiguous() or out.shape != pair.shape:
@@ -46,7 +44,7 @@ def grid_self_attention_hip(module: nn.Module, pair: torch.Tensor, mask: Optiona
                       pair.device)
     nh.call("xfh_grid_self_attention", nh.ptr(pair_c), nh.dtype_code(pair.dtype), nh.ptr(mask_t),
             mask_code, n, c, heads, int(bool(module.transpose)), nh.ptr(nw), nh.ptr(nb),
-            float(norm.eps), *(nh.ptr(w[name]) for name in _GRID_WEIGHTS), nh.dtype_code(dtype),
+            float(module.act_norm.eps), *map(nh.ptr, w), nh.dtype_code(dtype),
             nh.ptr(out), nh.dtype_code(out.dtype), accumulate, nh.ptr(ws), ws.numel(),
             nh.stream_of(pair.device))
     return out
@@ -85,7 +83,10 @@ def msa_attention_hip(module: nn.Module, msa: torch.Tensor, msa_mask: Optional[t
     MSA row."""
     nh.check_gpu_inference(msa, msa_mask, pair)
     nh.check_module(module)
-    dtype = nh.compute_dtype(msa, *(getattr(module, n).weight for n in _MSA_WEIGHTS))
+    dtype, (w, aw, ab, pw, pb) = nh.gather(
+        module, "msa_attention", nh.params(module, _MSA_WEIGHTS, ("act_norm", "pair_norm")), len(_MSA_WEIGHTS), msa,
+        lambda dt: ([nh.linear_weight(module, n, dt) for n in _MSA_WEIGHTS], *nh.norm_params(module, "act_norm"),
+                    *nh.norm_params(module, "pair_norm")))
     if msa.dim() != 3 or msa.shape[-1] != module.c_msa:
         raise ValueError("MSAAttention expects msa [S, N, c_msa].")
     rows, n, c_msa = msa.shape
@@ -95,8 +96,6 @@ def msa_attention_hip(module: nn.Module, msa: torch.Tensor, msa_mask: Optional[t
         raise ValueError("The 'hip' backend supports FP32/BF16 only.")
     msa_c, pair_c = msa.contiguous(), pair.contiguous()
     mask_t, mask_code = nh.mask_arg(msa_mask, (rows, n)) if msa_mask is not None else (None, nh.BOOL)
-    w = {name: nh.linear_weight(module, name, dtype) for name in _MSA_WEIGHTS}
-    act_norm, pair_norm = module.act_norm, module.pair_norm
     if accumulate_into is not None:
         out, accumulate = accumulate_into, 1
         if not out.is_contiguous() or out.shape != msa.shape:
@@ -108,11 +107,8 @@ def msa_attention_hip(module: nn.Module, msa: torch.Tensor, msa_mask: Optional[t
                                                            nh.dtype_code(dtype)), msa.device)
     nh.call("xfh_msa_attention", nh.ptr(msa_c), nh.dtype_code(msa.dtype), nh.ptr(mask_t), mask_code,
             nh.ptr(pair_c), nh.dtype_code(pair.dtype), rows, n, c_msa, module.c_pair, module.num_head,
-            nh.ptr(nh.fp32_param(module, "act_norm_w", act_norm.weight)),
-            nh.ptr(nh.fp32_param(module, "act_norm_b", act_norm.bias)), float(act_norm.eps),
-            nh.ptr(nh.fp32_param(module, "pair_norm_w", pair_norm.weight)),
-            nh.ptr(nh.fp32_param(module, "pair_norm_b", pair_norm.bias)), float(pair_norm.eps),
-            *(nh.ptr(w[name]) for name in _MSA_WEIGHTS), nh.dtype_code(dtype), nh.ptr(out),
+            nh.ptr(aw), nh.ptr(ab), float(module.act_norm.eps), nh.ptr(pw), nh.ptr(pb), float(module.pair_norm.eps),
+            *map(nh.ptr, w), nh.dtype_code(dtype), nh.ptr(out),
             nh.dtype_code(out.dtype), accumulate, nh.ptr(ws), ws.numel(), nh.stream_of(msa.device))
     return out
 

@@ -40,14 +40,29 @@ def _adaptive_layer_norm(aln: nn.Module, x: torch.Tensor, single_cond: Optional[
         return ops.layer_norm(x, ln.normalized_shape, ln.weight, ln.bias, ln.eps, out_dtype=out_dtype,
                               owner=ln)
     cln = aln.single_cond_layer_norm
-    cond = ops.layer_norm(single_cond, cln.normalized_shape, cln.weight, cln.bias, cln.eps,
-                          out_dtype=dtype, owner=cln)
-    # scale and shift stay fp32 (one rounding fewer before the sigmoid and the add).
-    scale = ops.linear(cond, nh.linear_weight(aln, "single_cond_scale", dtype),
-                       aln.single_cond_scale.bias, dtype, out_dtype=torch.float32)
-    shift = ops.linear(cond, nh.linear_weight(aln, "single_cond_bias", dtype), None, dtype,
-                       out_dtype=torch.float32)
+    sources = [*nh.params(aln, ("single_cond_scale", "single_cond_bias")), nh.param(aln, "single_cond_scale", "bias")]
+    cond = ops.layer_norm(single_cond, cln.normalized_shape, nh.param(aln, "single_cond_layer_norm"),
+                          nh.param(aln, "single_cond_layer_norm", "bias"), cln.eps, out_dtype=dtype, owner=cln)
+    # scale and shift stay fp32 (one rounding fewer before the sigmoid and the add); one launch
+    # over the stacked weights from the second pass on.
+    _, stacked = nh.gather(aln, "scale_shift", sources, 0, x, lambda dt: _scale_shift_weights(sources, dt), dtype,
+                           again=True)
+    if stacked is not None:
+        scale, shift = ops.linear_batched(cond.reshape(-1, cond.shape[-1]), *stacked, dtype, out_dtype=torch.float32)
+    else:
+        scale, shift = (ops.linear(cond, w.detach().to(dtype).contiguous(), b, dtype, out_dtype=torch.float32)
+                        for w, b in ((sources[0], sources[2]), (sources[1], None)))
     return ops.adaptive_layer_norm(x, scale, shift, aln.layer_norm.eps, out_dtype=out_dtype)
+
+
+def _scale_shift_weights(sources, dtype: torch.dtype):
+    """single_cond_scale and single_cond_bias as one [2, c, c_cond] weight in ``dtype`` and their
+    [2, c] fp32 bias (zeros for single_cond_bias, which has none)."""
+    scale, shift, bias = (None if t is None else t.detach() for t in sources)
+    b = torch.zeros((2, scale.shape[0]), dtype=torch.float32, device=scale.device)
+    if bias is not None:
+        b[0] = bias
+    return torch.stack([scale.to(dtype), shift.to(dtype)]), b
 
 
 def _ada_ln_zero(zero: nn.Module, hidden: torch.Tensor, single_cond: Optional[torch.Tensor],
@@ -55,19 +70,26 @@ def _ada_ln_zero(zero: nn.Module, hidden: torch.Tensor, single_cond: Optional[to
                  cond: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``AdaLNZero.forward`` (``diffusion_transformer.py:85-95``), optionally added in place;
     ``cond`` = adaptive_zero_cond(single_cond) already computed, in the output dtype."""
-    w = nh.linear_weight(zero, "transition2", dtype)
+    conditioned = zero.use_single_cond and cond is None
+    sources = [nh.param(zero, "transition2")]
+    if conditioned:
+        sources.append(nh.param(zero, "adaptive_zero_cond"))
+    _, weights = nh.gather(
+        zero, "conditioned" if conditioned else "zero", sources, 0, hidden,
+        lambda dt: [nh.linear_weight(zero, name, dt) for name in ("transition2", "adaptive_zero_cond")[:len(sources)]],
+        dtype)
     out = accumulate_into
     out_dtype = out.dtype if out is not None else dtype
     acc = out is not None
     if zero.use_single_cond:
         if cond is None:
-            cond = ops.linear(single_cond, nh.linear_weight(zero, "adaptive_zero_cond", dtype),
-                              zero.adaptive_zero_cond.bias, dtype, out_dtype=out_dtype)
+            cond = ops.linear(single_cond, weights[1], nh.param(zero, "adaptive_zero_cond", "bias"), dtype,
+                              out_dtype=out_dtype)
         epi = nh.EPI_MUL_SIGMOID_AUX_ACCUMULATE if acc else nh.EPI_MUL_SIGMOID_AUX
-        return ops.linear(hidden, w, None, dtype, out=out, out_dtype=out_dtype, epilogue=epi,
+        return ops.linear(hidden, weights[0], None, dtype, out=out, out_dtype=out_dtype, epilogue=epi,
                           aux=cond, aux_rows=cond.numel() // cond.shape[-1])
     epi = nh.EPI_ACCUMULATE if acc else nh.EPI_STORE
-    return ops.linear(hidden, w, None, dtype, out=out, out_dtype=out_dtype, epilogue=epi)
+    return ops.linear(hidden, weights[0], None, dtype, out=out, out_dtype=out_dtype, epilogue=epi)
 
 
 def _check_accumulate(out, x):
@@ -82,12 +104,13 @@ def diffusion_transition_hip(module: nn.Module, x: torch.Tensor, single_cond=Non
     (scale, shift, zero_cond) precomputed by :func:`_block_conditioning`."""
     nh.check_gpu_inference(x, single_cond)
     nh.check_module(module)
-    dtype = nh.compute_dtype(x, module.transition1.weight)
+    sources = [nh.param(module, "transition1")]
+    dtype, w_glu = nh.gather(module, "transition1", sources, 1, x,
+                             lambda dt: nh.linear_weight(module, "transition1", dt, "glu"))
     _check_accumulate(accumulate_into, x)
     xn = _adaptive_layer_norm(module.adaptive_layernorm, x, single_cond, dtype,
                               cond=None if _cond is None else _cond[:2])
-    f = module.transition1.weight.shape[0] // 2
-    hidden = ops.gated_linear_unit(xn, nh.linear_weight(module, "transition1", dtype, "glu"), f, dtype)
+    hidden = ops.gated_linear_unit(xn, w_glu, sources[0].shape[0] // 2, dtype)
     return _ada_ln_zero(module.adaptive_zero_init, hidden, single_cond, dtype, accumulate_into,
                         cond=None if _cond is None else _cond[2])
 
@@ -112,6 +135,12 @@ def _projection_bias(module: nn.Module, c: int, parts: int, device: torch.device
     return cached[1]
 
 
+def qkvg_weights(module: nn.Module, dtype: torch.dtype):
+    """[Wq; Wk; Wv; Wgate] in ``dtype`` and its fp32 bias (or None)."""
+    w = nh.fused_linear_weight(module, _QKV + ("gating_query",), dtype)
+    return w, _projection_bias(module, w.shape[0] // 4, 4, w.device)
+
+
 _LOG2E = 1.4426950408889634
 
 
@@ -132,7 +161,8 @@ def self_attention_hip(module: nn.Module, x: torch.Tensor, mask: Optional[torch.
     logits_t = pair_logits.tensor if isinstance(pair_logits, ops.PackedBias) else pair_logits
     nh.check_gpu_inference(x, mask, logits_t, single_cond)
     nh.check_module(module)
-    dtype = nh.compute_dtype(x, *(getattr(module, n).weight for n in _QKV + ("gating_query",)))
+    sources = [*nh.params(module, _QKV + ("gating_query",)), nh.param(module, "q_projection", "bias")]
+    dtype = nh.compute_dtype(x, *sources[:4])
     _check_accumulate(accumulate_into, x)
     if x.dim() not in (2, 3):
         raise ValueError("SelfAttention expects x [N, c] or [S, N, c]")
@@ -149,8 +179,8 @@ def self_attention_hip(module: nn.Module, x: torch.Tensor, mask: Optional[torch.
         if operands is None or not operands.matches(samples, n, heads, d, x.device):
             operands = ops.shared_attention_operands(samples, n, heads, d, x.device)
         operands.set_mask(mask)
-        w_all = nh.fused_linear_weight(module, _QKV + ("gating_query",), dtype)
-        ops.attention_project(xn, w_all, _projection_bias(module, c, 4, x.device), operands, d ** -0.5 * _LOG2E)
+        _, (w_all, b_all) = nh.gather(module, "qkvg", sources, 4, x, lambda dt: qkvg_weights(module, dt), dtype)
+        ops.attention_project(xn, w_all, b_all, operands, d ** -0.5 * _LOG2E)
         o = ops.attention_on_operands(operands, pair_logits, torch.empty((samples, n, c), dtype=dtype, device=x.device))
         return _ada_ln_zero(module.adaptive_zero_init, o.reshape(x.shape), single_cond, dtype, accumulate_into,
                             cond=None if _cond is None else _cond[2])
@@ -212,36 +242,76 @@ def _conditioning_weights(module: nn.Module, alns, zeros, dtype: torch.dtype):
     return nh.derived_weight(module, f"conditioning:{dtype}", srcs, build)
 
 
-def _block_conditioning(module: nn.Module, single_cond: torch.Tensor, dtype: torch.dtype,
-                        zero_dtype: torch.dtype):
+def _block_parts(module: nn.Module):
+    """The transformer's attention and transition blocks, their AdaptiveLayerNorms and AdaLNZeros
+    (every attention's first, then every transition's)."""
+    att, tr = list(module.self_attention._modules.values()), list(module.transition_block._modules.values())
+    alns = [b._modules["adaptive_layernorm"] for b in att + tr]
+    zeros = [b._modules["adaptive_zero_init"] for b in att + tr]
+    return att, tr, alns, zeros
+
+
+def _block_conditioning(single_cond: torch.Tensor, alns, dtype: torch.dtype, zero_dtype: torch.dtype, weights):
     """Every block's conditioning linears (``AdaptiveLayerNorm`` scale/shift,
     ``diffusion_transformer.py:59-62``; ``AdaLNZero`` cond, ``:93``) computed up front: they
     read only single_cond, which is the same for all blocks of one call. Two batched launches
     (one over the normalised single_cond, one over single_cond itself) replace the 6 small
-    GEMMs of every block. Returns [(attention (scale, shift, zero), transition (...))] per
-    block, or None when some block has no single_cond conditioning (the per-block path)."""
-    n_blocks = len(module.self_attention)
-    att = [module.self_attention[i] for i in range(n_blocks)]
-    tr = [module.transition_block[i] for i in range(n_blocks)]
-    alns = [b.adaptive_layernorm for b in att] + [b.adaptive_layernorm for b in tr]
-    zeros = [b.adaptive_zero_init for b in att] + [b.adaptive_zero_init for b in tr]
-    if single_cond is None or not all(a.use_single_cond for a in alns) or \
-            not all(z.use_single_cond for z in zeros):
-        return None
-    eps = {a.single_cond_layer_norm.eps for a in alns}
-    shapes = {tuple(a.single_cond_layer_norm.normalized_shape) for a in alns}
-    if len(eps) != 1 or len(shapes) != 1:
-        return None
-    w_ss, b_ss, w_z, b_z = _conditioning_weights(module, alns, zeros, dtype)
-    s_hat = ops.layer_norm(single_cond, shapes.pop(), None, None, eps.pop(), out_dtype=dtype)
+    GEMMs of every block. Returns the [2A, rows, c] scale/shift pairs of ``alns`` and the
+    [Z, rows, c] conditions (:func:`_conditioning_weights` order)."""
+    w_ss, b_ss, w_z, b_z = weights
+    cln = alns[0].single_cond_layer_norm
+    s_hat = ops.layer_norm(single_cond, cln.normalized_shape, None, None, cln.eps, out_dtype=dtype)
     ss = ops.linear_batched(s_hat.reshape(-1, s_hat.shape[-1]), w_ss, b_ss, dtype)
-    zz = ops.linear_batched(single_cond.reshape(-1, single_cond.shape[-1]), w_z, b_z, dtype,
-                            out_dtype=zero_dtype)
-    lead = single_cond.shape[:-1]
-    view = lambda t: t.reshape(*lead, t.shape[-1])
-    return [((view(ss[2 * i]), view(ss[2 * i + 1]), view(zz[i])),
-             (view(ss[2 * (n_blocks + i)]), view(ss[2 * (n_blocks + i) + 1]), view(zz[n_blocks + i])))
-            for i in range(n_blocks)]
+    zz = ops.linear_batched(single_cond.reshape(-1, single_cond.shape[-1]), w_z, b_z, dtype, out_dtype=zero_dtype)
+    return ss, zz
+
+
+def _conditioned_alike(single_cond, alns, zeros) -> bool:
+    """Whether every block is conditioned on single_cond through LayerNorms of one shape and eps
+    (else the conditioning runs block by block)."""
+    if single_cond is None or not all(a.use_single_cond for a in alns) or not all(z.use_single_cond for z in zeros):
+        return False
+    norms = [a.single_cond_layer_norm for a in alns]
+    return len({(n.eps, tuple(n.normalized_shape)) for n in norms}) == 1
+
+
+def _block_sources(att, tr, alns, zeros):
+    """The parameters of every block: q, k, v, gating and transition1 weights first (the ones
+    that take part in the compute dtype), then the rest."""
+    weights, rest = [], []
+    for a in att:
+        weights += nh.params(a, _QKV + ("gating_query",))
+        rest.append(nh.param(a, "q_projection", "bias"))
+    for t in tr:
+        weights.append(nh.param(t, "transition1"))
+    for z in zeros:
+        rest += (nh.param(z, "transition2"), nh.param(z, "adaptive_zero_cond"), nh.param(z, "adaptive_zero_cond", "bias"))
+    for a in alns:
+        rest += nh.params(a, ("single_cond_scale", "single_cond_bias"), ("single_cond_layer_norm",))
+        rest += (nh.param(a, "single_cond_scale", "bias"), nh.param(a, "single_cond_bias", "bias"))
+    return weights, rest
+
+
+def _stacked_logits_weight(module: nn.Module, projs, dtype: torch.dtype) -> torch.Tensor:
+    """Every super-block's pair-logit projection stacked, in ``dtype``."""
+    return nh.derived_weight(module, f"pair_logits:{dtype}", projs,
+                             lambda *ws: torch.cat([w.detach() for w in ws], dim=0).to(dtype).contiguous())
+
+
+def _block_weights(module, att, tr, alns, zeros, projs, dtype: torch.dtype) -> dict:
+    """What the blocks' call needs of their parameters; ``c`` is None when the blocks differ in
+    shape or the compute dtype is not bf16 (they then run one by one)."""
+    out = [nh.linear_weight(z, "transition2", dtype) for z in zeros]
+    glu = [nh.linear_weight(t, "transition1", dtype, "glu") for t in tr]
+    c, f = out[0].shape[0], nh.param(tr[0], "transition1").shape[0] // 2
+    same = dtype == torch.bfloat16 and \
+        all(tuple(nh.param(a, n).shape) == (c, c) for a in att for n in _QKV + ("gating_query",)) and \
+        all(tuple(nh.param(t, "transition1").shape) == (2 * f, c) for t in tr) and \
+        all(tuple(w.shape) == ((c, c) if i < len(att) else (c, f)) for i, w in enumerate(out))
+    return dict(conditioning=_conditioning_weights(module, alns, zeros, dtype),
+                logits=_stacked_logits_weight(module, projs, dtype),
+                qkvg=[qkvg_weights(a, dtype) for a in att] if same else None,
+                glu=glu, out=out, c=c if same else None, f=f)
 
 
 def _cached(module: nn.Module, name: str, dependencies, factory, modules):
@@ -268,6 +338,29 @@ def _block_operands(module: nn.Module, act: torch.Tensor, mask: Optional[torch.T
     return operands
 
 
+def _block_cond(conds, index: int, n: int):
+    """Block ``index``'s attention and transition (scale, shift, zero condition), of n blocks."""
+    if conds is None:
+        return None, None
+    ss, zz = conds
+    return tuple((ss[2 * i], ss[2 * i + 1], zz[i]) for i in (index, n + index))
+
+
+def _block_struct(i: int, n_blocks: int, weights, conds, packed: torch.Tensor, heads: int, att: nn.Module,
+                  tr: nn.Module) -> "nh.DiffusionBlock":
+    ss, zz = conds
+    n = zz.shape[0] // 2
+    w_qkvg, b_qkvg = weights["qkvg"][i]
+    ss_ptr, ss_step = nh.ptr(ss), ss.stride(0) * ss.element_size()
+    zz_ptr, zz_step = nh.ptr(zz), zz.stride(0) * zz.element_size()
+    return nh.DiffusionBlock(
+        nh.ptr(w_qkvg), nh.ptr(b_qkvg), nh.ptr(packed) + i * heads * packed.stride(0) * packed.element_size(),
+        nh.ptr(weights["out"][i]), nh.ptr(weights["glu"][i]), nh.ptr(weights["out"][n + i]),
+        ss_ptr + 2 * i * ss_step, ss_ptr + (2 * i + 1) * ss_step, zz_ptr + i * zz_step,
+        ss_ptr + 2 * (n + i) * ss_step, ss_ptr + (2 * (n + i) + 1) * ss_step, zz_ptr + (n + i) * zz_step,
+        att._modules["adaptive_layernorm"].layer_norm.eps, tr._modules["adaptive_layernorm"].layer_norm.eps)
+
+
 def diffusion_transformer_hip(module: nn.Module, act: torch.Tensor, mask: torch.Tensor,
                               single_cond: torch.Tensor, pair_cond: torch.Tensor) -> torch.Tensor:
     """``DiffusionTransformer.forward`` (``diffusion_transformer.py:250-272``), updating
@@ -280,13 +373,23 @@ def diffusion_transformer_hip(module: nn.Module, act: torch.Tensor, mask: torch.
     nh.check_gpu_inference(act, mask, single_cond, pair_cond)
     if not act.is_contiguous():
         raise ValueError("DiffusionTransformer (hip) updates act in place; pass a contiguous tensor")
-    dtype = nh.compute_dtype(act, module.pair_logits_projection[0].weight)
     ln = module.pair_input_layer_norm
     heads, size = module.num_head, module.super_block_size
-    # Not an input-cache entry: its key would cover ~400 parameters, whose checks cost more
-    # host time than the two batched GEMMs they would save.
-    conds = _block_conditioning(module, single_cond, dtype, act.dtype)
     n_blocks = module.num_super_blocks * size
+    att, tr, alns, zeros = _block_parts(module)
+    projs = [nh.param(module.pair_logits_projection, name) for name in module.pair_logits_projection._modules]
+    dtype = nh.compute_dtype(act, projs[0])
+    # Not input-cache entries: their key would cover ~400 parameters, whose checks cost more
+    # host time than the two batched GEMMs they would save.
+    conds = weights = None
+    if _conditioned_alike(single_cond, alns, zeros):
+        block_weights, rest = _block_sources(att, tr, alns, zeros)
+        _, weights = nh.gather(
+            module, "blocks", block_weights + projs + rest, len(block_weights), act,
+            lambda dt: _block_weights(module, att, tr, alns, zeros, projs, dt), again=True)
+        conds = _block_conditioning(single_cond, alns, dtype, act.dtype,
+                                    weights["conditioning"] if weights is not None else
+                                    _conditioning_weights(module, alns, zeros, dtype))
     # A packed bias (either path below) feeds the pipelined attention kernel, which takes
     # bf16, head dims <= 64 and at most attention_max_keys() keys.
     packed_bias = dtype == torch.bfloat16 and act.shape[-1] // heads <= 64 and \
@@ -295,9 +398,7 @@ def diffusion_transformer_hip(module: nn.Module, act: torch.Tensor, mask: torch.
             tuple(ln.normalized_shape) == (128,):
         # Every super-block's pair logits in one pass over pair_cond, straight into the
         # attention kernel's bias layout; block b reads heads b*H .. b*H + H - 1.
-        projs = [module.pair_logits_projection[s].weight for s in range(module.num_super_blocks)]
-        w_all = nh.derived_weight(module, f"pair_logits:{dtype}", projs,
-                                  lambda *ws: torch.cat([w.detach() for w in ws], dim=0).to(dtype).contiguous())
+        w_all = weights["logits"] if weights is not None else _stacked_logits_weight(module, projs, dtype)
         # bf16 logits, the dtype of the reference's autocast Linear output (half the bytes of
         # fp32: at N=768 all 24 blocks' logits take 453 MB and fit the input cache's budget).
         packed = _cached(module, "pair_logits_packed", (pair_cond, heads),
@@ -305,8 +406,18 @@ def diffusion_transformer_hip(module: nn.Module, act: torch.Tensor, mask: torch.
                                                          out_dtype=torch.bfloat16),
                          modules=(ln, module.pair_logits_projection))
         operands = _block_operands(module, act, mask)
+        c = act.shape[-1]
+        # The whole stack in one library call when every block has the same shapes.
+        if weights is not None and operands is not None and c % 32 == 0 and act.dim() in (2, 3) and \
+                weights["c"] == c and conds[0].shape[-1] == conds[1].shape[-1] == c and \
+                packed.shape[0] >= n_blocks * heads and tuple(packed.shape[1:]) == (act.shape[-2], operands.tpad) and \
+                all(a.num_head == heads for a in att):
+            blocks = (nh.DiffusionBlock * n_blocks)(*(
+                _block_struct(i, n_blocks, weights, conds, packed, heads, att[i], tr[i]) for i in range(n_blocks)))
+            ops.diffusion_blocks(act, operands, blocks, conds[0].shape[1], weights["f"], packed.dtype)
+            return act
         for index in range(n_blocks):
-            att_cond, tr_cond = (None, None) if conds is None else conds[index]
+            att_cond, tr_cond = _block_cond(conds, index, len(att))
             bias = ops.PackedBias(packed[index * heads:(index + 1) * heads])
             self_attention_hip(module.self_attention[index], act, mask, bias, single_cond,
                                accumulate_into=act, _cond=att_cond, _operands=operands)
@@ -330,7 +441,7 @@ def diffusion_transformer_hip(module: nn.Module, act: torch.Tensor, mask: torch.
             else:
                 bias = logits[..., j * heads:(j + 1) * heads].permute(2, 0, 1)
             index = s * size + j
-            att_cond, tr_cond = (None, None) if conds is None else conds[index]
+            att_cond, tr_cond = _block_cond(conds, index, len(att))
             self_attention_hip(module.self_attention[index], act, mask, bias, single_cond,
                                accumulate_into=act, _cond=att_cond, _operands=operands)
             diffusion_transition_hip(module.transition_block[index], act, single_cond,
@@ -437,8 +548,11 @@ def cross_attention_hip(module: nn.Module, x_q: torch.Tensor, x_k: torch.Tensor,
                          f"{tuple(x_q.shape)}; {tuple(mask_k.shape)}, {tuple(x_k.shape)})")
     nh.check_gpu_inference(x_q, x_k, mask_q, mask_k, pair_logits, single_cond_q, single_cond_k)
     nh.check_module(module)
-    names = ("q_projection", "k_projection", "v_projection", "gating_query")
-    dtype = nh.compute_dtype(x_q, *(getattr(module, n).weight for n in names))
+    dtype, (w_q, w_kv, w_gate) = nh.gather(
+        module, "cross_attention", nh.params(module, _QKV + ("gating_query",)), 4, x_q,
+        lambda dt: (nh.linear_weight(module, "q_projection", dt),
+                    nh.fused_linear_weight(module, ("k_projection", "v_projection"), dt),
+                    nh.linear_weight(module, "gating_query", dt)))
     lead, nq, nk = tuple(x_q.shape[:-2]), x_q.shape[-2], x_k.shape[-2]
     if tuple(x_k.shape[:-2]) != lead:
         raise ValueError("CrossAttention: x_q and x_k must share their leading (subset) dims")
@@ -452,8 +566,8 @@ def cross_attention_hip(module: nn.Module, x_q: torch.Tensor, x_k: torch.Tensor,
         raise ValueError("accumulate_into must be a contiguous [..., Q, value_dim] tensor")
     xq = _adaptive_layer_norm(module.q_adaptive_layernorm, x_q, single_cond_q, dtype)
     xk = _adaptive_layer_norm(module.k_adaptive_layernorm, x_k, single_cond_k, dtype)
-    q = ops.linear(xq, nh.linear_weight(module, "q_projection", dtype), module.q_projection.bias, dtype)
-    kv = ops.linear(xk, nh.fused_linear_weight(module, ("k_projection", "v_projection"), dtype), None, dtype)
+    q = ops.linear(xq, w_q, nh.param(module, "q_projection", "bias"), dtype)
+    kv = ops.linear(xk, w_kv, None, dtype)
     q4 = torch.as_strided(q, (batch, h, nq, dk), (nq * kd, dk, kd, 1))
     k4 = torch.as_strided(kv, (batch, h, nk, dk), (nk * (kd + vd), dk, kd + vd, 1))
     v4 = torch.as_strided(kv, (batch, h, nk, dv), (nk * (kd + vd), dv, kd + vd, 1), kd)
@@ -472,8 +586,7 @@ def cross_attention_hip(module: nn.Module, x_q: torch.Tensor, x_k: torch.Tensor,
     o = torch.empty(lead + (nq, vd), dtype=dtype, device=x_q.device)
     o_view = torch.as_strided(o, (batch, h, nq, dv), (nq * vd, dv, vd, 1))
     ops.attention(q4, k4, v4, None, bias, out=o_view, scale=module.q_scale)
-    ops.linear(xq, nh.linear_weight(module, "gating_query", dtype), None, dtype, out=o,
-               epilogue=nh.EPI_SIGMOID_MUL_AUX, aux=o)
+    ops.linear(xq, w_gate, None, dtype, out=o, epilogue=nh.EPI_SIGMOID_MUL_AUX, aux=o)
     return _ada_ln_zero(module.adaptive_zero_init, o, single_cond_q, dtype, accumulate_into)
 
 

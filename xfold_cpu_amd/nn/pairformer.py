@@ -8,6 +8,7 @@ without a separate update tensor), then the single track (``pairformer.py:102-11
 
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
@@ -17,10 +18,13 @@ from ..fastnn import LayerNorm
 from ..fastnn import config as fastnn_config
 from ..fastnn import native_hip as nh
 from ..fastnn import ops
-from .attention import GridSelfAttention, MSAAttention, grid_self_attention_hip, msa_attention_hip
-from .diffusion_transformer import SelfAttention, self_attention_hip
+from .attention import _GRID_WEIGHTS, GridSelfAttention, MSAAttention, grid_self_attention_hip, msa_attention_hip
+from .diffusion_transformer import _QKV, SelfAttention, qkvg_weights, self_attention_hip
 from .primitives import OuterProductMean, Transition, outer_product_mean_hip, transition_hip
+from .triangle_multiplication import _NORMS as _TRIANGLE_NORMS, _WEIGHTS as _TRIANGLE_WEIGHTS
 from .triangle_multiplication import TriangleMultiplication, triangle_multiplication_hip
+
+_ATTENTION = _QKV + ("gating_query",)
 
 
 def pair_logits_hip(block: nn.Module, pair: torch.Tensor, dtype: torch.dtype):
@@ -49,29 +53,33 @@ def _transition_with_logits_hip(block: nn.Module, pair: torch.Tensor) -> Optiona
     (``pairformer.py:100``, ``:103-106``) in one kernel, whose epilogue computes the logits
     from the values it stores: bf16 pair [N, N, 128], hidden 512, at most 16 heads. None
     (nothing done) for other shapes."""
-    tr, norm = block.pair_transition, block.single_pair_logits_norm
-    proj = block.single_pair_logits_projection
+    tr, norm, proj = block.pair_transition, block.single_pair_logits_norm, nh.param(block, "single_pair_logits_projection")
+    names = ("transition1", "transition2")
+    w1_src, w2_src, *tr_norm = nh.params(tr, names, ("input_layer_norm",))
     n, c = pair.shape[0], pair.shape[-1]
     if (pair.dtype != torch.bfloat16 or pair.dim() != 3 or pair.shape[1] != n or c != 128
-            or tr.transition2.weight.shape != (c, 512) or tr.transition1.weight.shape != (1024, c)
+            or w2_src.shape != (c, 512) or w1_src.shape != (1024, c)
             or tuple(norm.normalized_shape) != (c,) or tuple(tr.input_layer_norm.normalized_shape) != (c,)
-            or proj.weight.shape[0] > 16 or n > nh.attention_max_keys()
-            or nh.compute_dtype(pair, tr.transition1.weight, tr.transition2.weight, proj.weight) != torch.bfloat16):
+            or proj.shape[0] > 16 or n > nh.attention_max_keys()):
+        return None
+    sources = [w1_src, w2_src, proj, *tr_norm, norm.weight, norm.bias]
+    # Not this dtype: None, and the general path builds its own copies.
+    dtype, values = nh.gather(
+        block, "transition_pair_bias", sources, 3, pair,
+        lambda dt: None if dt != torch.bfloat16 else (
+            nh.linear_weight(tr, "transition1", dt, "glu"), nh.linear_weight(tr, "transition2", dt),
+            nh.linear_weight(block, "single_pair_logits_projection", dt), *nh.norm_params(tr, "input_layer_norm"),
+            *nh.norm_params(block, "single_pair_logits_norm")))
+    if values is None:
         return None
     nh.check_gpu_inference(pair)
     nh.check_module(tr)
-    w1 = nh.linear_weight(tr, "transition1", torch.bfloat16, "glu")
-    w2 = nh.linear_weight(tr, "transition2", torch.bfloat16)
-    nw = nh.fp32_param(tr, "norm_w", tr.input_layer_norm.weight)
-    nb = nh.fp32_param(tr, "norm_b", tr.input_layer_norm.bias)
-    wb = nh.linear_weight(block, "single_pair_logits_projection", torch.bfloat16)
-    bw = nh.fp32_param(norm, "ln_weight", norm.weight)
-    bb = nh.fp32_param(norm, "ln_bias", norm.bias)
+    w1, w2, wb, nw, nb, bw, bb = values
     heads = wb.shape[0]
     packed = torch.empty((heads, n, (n + 63) // 64 * 64), dtype=torch.float32, device=pair.device)
     nh.call("xfh_transition_pair_bias", nh.ptr(pair), n, c, 512, nh.ptr(nw), nh.ptr(nb),
             float(tr.input_layer_norm.eps), nh.ptr(w1), nh.ptr(w2), nh.ptr(bw), nh.ptr(bb), float(norm.eps),
-            nh.ptr(wb.contiguous()), heads, nh.ptr(packed), nh.stream_of(pair.device))
+            nh.ptr(wb), heads, nh.ptr(packed), nh.stream_of(pair.device))
     return ops.PackedBias(packed)
 
 
@@ -86,6 +94,8 @@ def pairformer_block_hip(block: nn.Module, pair: torch.Tensor, pair_mask: torch.
         _pair_updates_hip(block, pair, pair_mask)
         return pair
     _pair_updates_hip(block, pair, pair_mask, transition=False)
+    if FUSE_TRANSITION_AND_LOGITS and _single_track_hip(block, pair, single, seq_mask):
+        return pair, single
     logits = _transition_with_logits_hip(block, pair) if FUSE_TRANSITION_AND_LOGITS else None
     if logits is None:
         transition_hip(block.pair_transition, pair, accumulate_into=pair)
@@ -96,14 +106,129 @@ def pairformer_block_hip(block: nn.Module, pair: torch.Tensor, pair_mask: torch.
     return pair, single
 
 
+def _single_track_hip(block: nn.Module, pair: torch.Tensor, single: torch.Tensor,
+                      seq_mask: Optional[torch.Tensor]) -> bool:
+    """The pair transition with its logits and the whole single track in one library call
+    (``xfh_pairformer_single``), where the operators' own bf16 paths take those shapes; False
+    (nothing done) otherwise."""
+    m = block._modules
+    tr, norm, att, str_ = (m[name] for name in ("pair_transition", "single_pair_logits_norm", "single_attention_",
+                                                "single_transition"))
+    proj = nh.param(block, "single_pair_logits_projection")
+    aln, zero = att._modules["adaptive_layernorm"], att._modules["adaptive_zero_init"]
+    n, heads, c = pair.shape[0], att.num_head, single.shape[-1]
+    if (pair.dtype != torch.bfloat16 or pair.dim() != 3 or tuple(pair.shape) != (n, n, 128) or heads > 16
+            or tuple(single.shape) != (n, c) or single.dtype not in (torch.float32, torch.bfloat16)
+            or c % 32 or c % heads or not ops.AttentionOperands.supported(n, heads, c // heads)
+            or aln.use_single_cond or zero.use_single_cond
+            or (seq_mask is not None and tuple(seq_mask.shape) != (n,))):
+        return False
+    names = ("transition1", "transition2")
+    tr_w, str_w, att_w = nh.params(tr, names), nh.params(str_, names), nh.params(att, _ATTENTION)
+    out_w = nh.param(zero, "transition2")
+    f = str_w[1].shape[1]
+    if (tr_w[0].shape != (1024, 128) or tr_w[1].shape != (128, 512) or proj.shape != (heads, 128)
+            or str_w[0].shape != (2 * f, c) or str_w[1].shape != (c, f) or out_w.shape != (c, c)
+            or any(w.shape != (c, c) for w in att_w)):
+        return False
+    norms = ((tr, "input_layer_norm", 128), (block, "single_pair_logits_norm", 128), (aln, "layer_norm", c),
+             (str_, "input_layer_norm", c))
+    if any(tuple(owner._modules[name].normalized_shape) != (size,) for owner, name, size in norms):
+        return False
+    nh.check_gpu_inference(pair, single, seq_mask)
+    nh.check_module(block)
+    norm_sources = []
+    for owner, name, _ in norms:
+        norm_sources += (nh.param(owner, name), nh.param(owner, name, "bias"))
+
+    def build(dt):
+        if dt != torch.bfloat16:
+            return None
+        n0, n1, n2, n3 = (nh.norm_params(owner, name) for owner, name, _ in norms)
+        return [*n0, nh.linear_weight(tr, "transition1", dt, "glu"), nh.linear_weight(tr, "transition2", dt),
+                *n1, nh.linear_weight(block, "single_pair_logits_projection", dt),
+                *n2, *qkvg_weights(att, dt), nh.linear_weight(zero, "transition2", dt),
+                *n3, nh.linear_weight(str_, "transition1", dt, "glu"), nh.linear_weight(str_, "transition2", dt)]
+    # The operators resolve the compute dtype from the pair or the single track and their own
+    # weights: one group when both have one dtype, else the general path.
+    if single.dtype != pair.dtype and not torch.is_autocast_enabled("cuda"):
+        return False
+    _, values = nh.gather(block, "single_track", [*tr_w, proj, *att_w, *str_w, out_w, nh.param(att, "q_projection", "bias"),
+                                                  *norm_sources], 9, pair, build, again=True)
+    if values is None:
+        return False
+    operands = ops.shared_attention_operands(1, n, heads, c // heads, single.device)
+    operands.set_mask(seq_mask)
+    eps = (ctypes.c_float * 4)(*(owner._modules[name].eps for owner, name, _ in norms))
+    lib = nh.load_library()
+    ws = nh.workspace(lib.xfh_pairformer_single_workspace_size(n, c, heads, f), pair.device)
+    nh.call("xfh_pairformer_single", nh.ptr(pair), nh.ptr(single), nh.dtype_code(single.dtype), n, c, heads, f,
+            nh.ptrs(values), eps, (c // heads) ** -0.5 * 1.4426950408889634, nh.ptr(operands.q), nh.ptr(operands.k),
+            nh.ptr(operands.vt), nh.ptr(operands.gate), nh.ptr(operands.words), nh.ptr(ws), ws.numel(),
+            nh.stream_of(pair.device))
+    return True
+
+
+_TRIANGLES = ("triangle_multiplication_outgoing", "triangle_multiplication_incoming")
+_GRIDS = ("pair_attention1", "pair_attention2")
+
+
 def _pair_updates_hip(block: nn.Module, pair: torch.Tensor, pair_mask: torch.Tensor,
                       transition: bool = True) -> None:
-    triangle_multiplication_hip(block.triangle_multiplication_outgoing, pair, pair_mask, accumulate_into=pair)
-    triangle_multiplication_hip(block.triangle_multiplication_incoming, pair, pair_mask, accumulate_into=pair)
-    grid_self_attention_hip(block.pair_attention1, pair, pair_mask, accumulate_into=pair)
-    grid_self_attention_hip(block.pair_attention2, pair, pair_mask, accumulate_into=pair)
-    if transition:
-        transition_hip(block.pair_transition, pair, accumulate_into=pair)
+    """The pair updates (``pairformer.py:96-100``), as one library call (``xfh_pair_updates``) when
+    the five modules agree in their widths."""
+    m = block._modules
+    triangles, grids = [m[name] for name in _TRIANGLES], [m[name] for name in _GRIDS]
+    tr = m["pair_transition"]
+    tr_w = nh.params(tr, ("transition1", "transition2"))
+    c, heads, f = pair.shape[-1], grids[0].num_head, tr_w[1].shape[1]
+
+    def one_by_one():
+        triangle_multiplication_hip(triangles[0], pair, pair_mask, accumulate_into=pair)
+        triangle_multiplication_hip(triangles[1], pair, pair_mask, accumulate_into=pair)
+        grid_self_attention_hip(grids[0], pair, pair_mask, accumulate_into=pair)
+        grid_self_attention_hip(grids[1], pair, pair_mask, accumulate_into=pair)
+        if transition:
+            transition_hip(tr, pair, accumulate_into=pair)
+    if (pair.dim() != 3 or pair.shape[0] != pair.shape[1] or pair_mask is None or heads != grids[1].num_head
+            or any(t.c_pair != c for t in triangles + grids) or tr_w[0].shape != (2 * f, c)):
+        return one_by_one()
+    nh.check_gpu_inference(pair, pair_mask)
+    nh.check_module(block)
+    n = pair.shape[0]
+    weights, norms = [], []
+    for t in triangles:
+        weights += nh.params(t, _TRIANGLE_WEIGHTS)
+        norms += nh.params(t, (), _TRIANGLE_NORMS)
+    for g in grids:
+        weights += nh.params(g, _GRID_WEIGHTS)
+        norms += nh.params(g, (), ("act_norm",))
+    norms += nh.params(tr, (), ("input_layer_norm",))
+
+    def build(dt):
+        out = []
+        for t in triangles:
+            out += (*nh.norm_params(t, _TRIANGLE_NORMS[0]), *nh.norm_params(t, _TRIANGLE_NORMS[1]))
+            out += (nh.linear_weight(t, name, dt) for name in _TRIANGLE_WEIGHTS)
+        for g in grids:
+            out += nh.norm_params(g, "act_norm")
+            out += (nh.linear_weight(g, name, dt) for name in _GRID_WEIGHTS)
+        out += nh.norm_params(tr, "input_layer_norm")
+        out += (nh.linear_weight(tr, "transition1", dt, "glu"), nh.linear_weight(tr, "transition2", dt))
+        return out
+    dtype, values = nh.gather(block, "pair_updates", weights + tr_w + norms, len(weights) + 2, pair, build, again=True)
+    if values is None:
+        return one_by_one()
+    mask_t, mask_code = nh.mask_arg(pair_mask, (n, n))
+    outgoing = (ctypes.c_int * 2)(*(t.equation == "cik,cjk->cij" for t in triangles))
+    transpose = (ctypes.c_int * 2)(*(bool(g.transpose) for g in grids))
+    eps = (ctypes.c_float * 7)(*(t._modules[name].eps for t in triangles for name in _TRIANGLE_NORMS),
+                               *(g.act_norm.eps for g in grids), tr.input_layer_norm.eps)
+    f_now = f if transition else 0
+    lib, code = nh.load_library(), nh.dtype_code(dtype)
+    ws = nh.workspace(lib.xfh_pair_updates_workspace_size(n, c, heads, f_now, code), pair.device)
+    nh.call("xfh_pair_updates", nh.ptr(pair), nh.dtype_code(pair.dtype), nh.ptr(mask_t), mask_code, n, c, heads, f_now,
+            outgoing, transpose, nh.ptrs(values), eps, code, nh.ptr(ws), ws.numel(), nh.stream_of(pair.device))
 
 
 def _require_hip_backends() -> None:

@@ -18,18 +18,17 @@ def transition_hip(module: nn.Module, x: torch.Tensor,
     """``transition2(GLU(LN(x), transition1.weight.T))`` (``xfold/nn/primitives.py:33-37``)."""
     nh.check_gpu_inference(x)
     nh.check_module(module)
-    dtype = nh.compute_dtype(x, module.transition1.weight, module.transition2.weight)
+    sources = nh.params(module, ("transition1", "transition2"), ("input_layer_norm",))
     c = x.shape[-1]
-    f = module.transition2.weight.shape[1]
-    if module.transition1.weight.shape != (2 * f, c):
+    f = sources[1].shape[1]
+    if sources[0].shape != (2 * f, c):
         raise ValueError("Transition weights do not match the input width.")
+    dtype, (w1, w2, nw, nb) = nh.gather(
+        module, "transition", sources, 2, x,
+        lambda dt: (nh.linear_weight(module, "transition1", dt, "glu"), nh.linear_weight(module, "transition2", dt),
+                    *nh.norm_params(module, "input_layer_norm")))
     x_c = x.contiguous()
     rows = x_c.numel() // c
-    w1 = nh.linear_weight(module, "transition1", dtype, "glu")
-    w2 = nh.linear_weight(module, "transition2", dtype)
-    norm = module.input_layer_norm
-    nw = nh.fp32_param(module, "norm_w", norm.weight)
-    nb = nh.fp32_param(module, "norm_b", norm.bias)
     if accumulate_into is not None:
         out, accumulate = accumulate_into, 1
         if not out.is_contiguous() or out.shape != x.shape:
@@ -39,7 +38,7 @@ def transition_hip(module: nn.Module, x: torch.Tensor,
     lib = nh.load_library()
     ws = nh.workspace(lib.xfh_transition_workspace_size(rows, c, f, nh.dtype_code(dtype)), x.device)
     nh.call("xfh_transition", nh.ptr(x_c), nh.dtype_code(x.dtype), rows, c, f, nh.ptr(nw), nh.ptr(nb),
-            float(norm.eps), nh.ptr(w1), nh.ptr(w2), nh.dtype_code(dtype), nh.ptr(out),
+            float(module.input_layer_norm.eps), nh.ptr(w1), nh.ptr(w2), nh.dtype_code(dtype), nh.ptr(out),
             nh.dtype_code(out.dtype), accumulate, nh.ptr(ws), ws.numel(), nh.stream_of(x.device))
     return out
 
@@ -77,19 +76,18 @@ def outer_product_mean_hip(module: nn.Module, msa: torch.Tensor, mask: torch.Ten
     ``epsilon + sum_s mask[s, i] mask[s, j]``."""
     nh.check_gpu_inference(msa, mask)
     nh.check_module(module)
-    dtype = nh.compute_dtype(msa, module.left_projection.weight, module.right_projection.weight)
+    projections = ("left_projection", "right_projection")
+    dtype, (proj, w_out, b_out, nw, nb) = nh.gather(
+        module, "outer_product_mean",
+        [*nh.params(module, projections, ("layer_norm_input",)), module.output_w, module.output_b], 2, msa,
+        lambda dt: (nh.fused_linear_weight(module, projections, dt), _opm_output_weight(module, dt),
+                    nh.fp32_param(module, "output_b", module.output_b), *nh.norm_params(module, "layer_norm_input")))
     if msa.dim() != 3 or msa.shape[-1] != module.c_msa:
         raise ValueError("OuterProductMean expects msa [S, N, c_msa].")
     rows, n, c_msa = msa.shape
     co, c_out = module.num_outer_channel, module.num_output_channel
     msa_c = msa.contiguous()
     mask_t, mask_code = nh.mask_arg(mask, (rows, n)) if mask is not None else (None, nh.BOOL)
-    proj = nh.fused_linear_weight(module, ("left_projection", "right_projection"), dtype)
-    w_out = _opm_output_weight(module, dtype)
-    b_out = nh.fp32_param(module, "output_b", module.output_b)
-    norm = module.layer_norm_input
-    nw = nh.fp32_param(module, "norm_w", norm.weight)
-    nb = nh.fp32_param(module, "norm_b", norm.bias)
     if accumulate_into is not None:
         out, accumulate = accumulate_into, 1
         if not out.is_contiguous() or tuple(out.shape) != (n, n, c_out):
@@ -100,7 +98,7 @@ def outer_product_mean_hip(module: nn.Module, msa: torch.Tensor, mask: torch.Ten
     ws = nh.workspace(lib.xfh_outer_product_mean_workspace_size(rows, n, c_msa, co, nh.dtype_code(dtype)),
                       msa.device)
     nh.call("xfh_outer_product_mean", nh.ptr(msa_c), nh.dtype_code(msa.dtype), nh.ptr(mask_t), mask_code,
-            rows, n, c_msa, co, c_out, nh.ptr(nw), nh.ptr(nb), float(norm.eps), nh.ptr(proj), nh.ptr(w_out),
+            rows, n, c_msa, co, c_out, nh.ptr(nw), nh.ptr(nb), float(module.layer_norm_input.eps), nh.ptr(proj), nh.ptr(w_out),
             nh.ptr(b_out), float(module.epsilon), nh.dtype_code(dtype), nh.ptr(out), nh.dtype_code(out.dtype),
             accumulate, nh.ptr(ws), ws.numel(), nh.stream_of(msa.device))
     return out

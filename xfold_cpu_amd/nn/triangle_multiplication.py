@@ -18,26 +18,26 @@ from ..fastnn import config as fastnn_config
 from ..fastnn import native_hip as nh
 
 
+_WEIGHTS = ("projection", "gate", "output_projection", "gating_linear")
+_NORMS = ("left_norm_input", "center_norm")
+
+
 def triangle_multiplication_hip(module: nn.Module, pair: torch.Tensor, mask: Optional[torch.Tensor],
                                 accumulate_into: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Update of ``xfold/nn/triangle_multiplication.py:71-105`` (or ``pair += update`` in
     place when ``accumulate_into`` is the contiguous pair tensor itself)."""
-    names = ("projection", "gate", "output_projection", "gating_linear")
     nh.check_gpu_inference(pair, mask)
     nh.check_module(module)
-    dtype = nh.compute_dtype(pair, *(getattr(module, n).weight for n in names))
+    dtype, (w_proj, w_gate, w_out, w_gating, lw, lb, cw, cb) = nh.gather(
+        module, "triangle_multiplication", nh.params(module, _WEIGHTS, _NORMS), 4, pair,
+        lambda dt: (*(nh.linear_weight(module, n, dt) for n in _WEIGHTS),
+                    *nh.norm_params(module, _NORMS[0]), *nh.norm_params(module, _NORMS[1])))
     if pair.dim() != 3 or pair.shape[0] != pair.shape[1] or pair.shape[2] != module.c_pair:
         raise ValueError("TriangleMultiplication expects pair [N, N, c_pair].")
     n, c = pair.shape[0], pair.shape[2]
     outgoing = module.equation == "cik,cjk->cij"
     pair_c = pair.contiguous()
     mask_t, mask_code = nh.mask_arg(mask, (n, n))
-    w = {name: nh.linear_weight(module, name, dtype) for name in names}
-    ln_in, ln_c = module.left_norm_input, module.center_norm
-    lw = nh.fp32_param(module, "left_w", ln_in.weight)
-    lb = nh.fp32_param(module, "left_b", ln_in.bias)
-    cw = nh.fp32_param(module, "center_w", ln_c.weight)
-    cb = nh.fp32_param(module, "center_b", ln_c.bias)
     if accumulate_into is not None:
         out, accumulate = accumulate_into, 1
         if not out.is_contiguous() or out.shape != pair.shape:
@@ -48,9 +48,9 @@ def triangle_multiplication_hip(module: nn.Module, pair: torch.Tensor, mask: Opt
     ws = nh.workspace(lib.xfh_triangle_multiplication_workspace_size(n, c, nh.dtype_code(dtype)),
                       pair.device)
     nh.call("xfh_triangle_multiplication", nh.ptr(pair_c), nh.dtype_code(pair.dtype), nh.ptr(mask_t),
-            mask_code, n, c, int(outgoing), nh.ptr(lw), nh.ptr(lb), float(ln_in.eps),
-            nh.ptr(w["projection"]), nh.ptr(w["gate"]), nh.ptr(cw), nh.ptr(cb), float(ln_c.eps),
-            nh.ptr(w["output_projection"]), nh.ptr(w["gating_linear"]), nh.dtype_code(dtype),
+            mask_code, n, c, int(outgoing), nh.ptr(lw), nh.ptr(lb), float(module.left_norm_input.eps),
+            nh.ptr(w_proj), nh.ptr(w_gate), nh.ptr(cw), nh.ptr(cb), float(module.center_norm.eps),
+            nh.ptr(w_out), nh.ptr(w_gating), nh.dtype_code(dtype),
             nh.ptr(out), nh.dtype_code(out.dtype), accumulate, nh.ptr(ws), ws.numel(),
             nh.stream_of(pair.device))
     return out
