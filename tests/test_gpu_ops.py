@@ -802,6 +802,39 @@ def test_gemm_ring_configurations(device, kind, m, k, n, batch, config):
     assert_parity_bf16(got, want, f"gemm_ring {config} {kind} {m}x{k}->{n}", floor=bf16_stored(want))
 
 
+# Each of the three k-split tiles on a 256-CU device: one row, rows and columns past a tile, k a
+# remainder of the wavefronts' rounds, the largest grid of one round.
+@pytest.mark.parametrize("m,k,n", [(1, 256, 136), (17, 288, 200), (96, 1536, 768), (200, 800, 776), (300, 768, 768),
+                                   (437, 1536, 768), (65, 768, 3072)])
+@pytest.mark.parametrize("kind", ["linear", "glu", "accumulate"])
+def test_gemm_direct(device, m, k, n, kind):
+    """Small outputs with k split over a workgroup's wavefronts, against an fp32 product of the
+    same bf16 operands (the bf16 store is the only rounding that differs)."""
+    announce("gemm_direct", m, k, n, kind)
+    g = torch.Generator().manual_seed(m + k + n)
+    x = torch.randn(m, k, generator=g).bfloat16()
+    w = (torch.randn(n, k, generator=g) / math.sqrt(k)).bfloat16()
+    nh.kernel_timing_read("gemm_direct")
+    nh.set_kernel_timing(True)
+    if kind == "glu":
+        f = n // 2
+        packed = nh._prepare(w[:2 * f].to(device), torch.bfloat16, "glu")
+        got, want = ops.gated_linear_unit(x.to(device), packed, f, torch.bfloat16), R.gated_linear_unit(x.float(), w[:2 * f].float().T)
+    elif kind == "linear":
+        bias = torch.randn(n, generator=g)
+        got, want = ops.linear(x.to(device), w.to(device), bias.to(device), torch.bfloat16), x.float() @ w.float().T + bias
+    else:
+        out, aux = torch.randn(m, n, generator=g), torch.randn(m, n, generator=g)
+        got = ops.linear(x.to(device), w.to(device), None, torch.bfloat16, out=out.to(device),
+                         epilogue=nh.EPI_MUL_SIGMOID_AUX_ACCUMULATE, aux=aux.to(device))
+        want = out + x.float() @ w.float().T * torch.sigmoid(aux)
+    torch.cuda.synchronize()
+    nh.set_kernel_timing(False)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert nh.kernel_timing_read("gemm_direct")[1] == 1
+    assert_parity_bf16(got, want, f"gemm_direct {kind} {m}x{k}->{n}", floor=bf16_stored(want))
+
+
 @pytest.mark.parametrize("profile", ["jump", "low", "ramp", "mixed"])
 @pytest.mark.parametrize("batch", [3, 8])
 def test_attention_logit_ranges(device, profile, batch):

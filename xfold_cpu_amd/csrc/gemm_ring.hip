@@ -427,6 +427,11 @@ __global__ __launch_bounds__(256, G::WGS) void gemm_ring_kernel(GemmArgs p) {
   }
 }
 
+}  // namespace
+}  // namespace xfh
+#include "gemm_direct.h"
+namespace xfh {
+namespace {
 bool aligned(const void *ptr, int bytes) { return reinterpret_cast<uintptr_t>(ptr) % bytes == 0; }
 
 }  // namespace
@@ -506,6 +511,23 @@ RingPick pick_ring(const GemmArgs &p, int64_t batch, bool glu, int cus) {
   return best;
 }
 
+// Outputs that one round of small k-split tiles covers (at most one workgroup per CU) take
+// gemm_direct: a second workgroup on a CU doubles its time (its loads share the CU's 64 bytes
+// per clock), and the ring is then as fast or faster. us per launch, direct against ring:
+// [96][768] k = 768 4.6 / 9.1, k = 1536 6.9 / 13.9, [437][768] k = 768 7.9 / 10.4, [96][3072] k = 768 6.9 / 8.8;
+// past the line [768][768] k = 768 12.9 / 9.9, [200][3072] 11.1 / 8.7. Below k = 256 the two are equal;
+// [512][128] k = 384 (4.7 / 5.3) stays with the ring: no operator here has such a shape.
+using Direct16 = Direct<1, 2, 8, 4>;      // 16 x 32 tile, k over 8 wavefronts
+using Direct32 = Direct<2, 2, 4, 4>;      // 32 x 32, 4
+using Direct64 = Direct<2, 4, 8, 2>;      // 32 x 64, 8
+enum class DirectPick { None, Rows16, Rows32, Cols64 };
+DirectPick pick_direct(const GemmArgs &p, int64_t batch, int cus) {
+  if (p.K < 256 || (p.N <= 128 && p.K < 512)) return DirectPick::None;
+  auto fits = [&](int bm, int bn) { return ceil_div(p.M, bm) * ceil_div(p.N, bn) * batch <= cus; };
+  return fits(16, 32) ? DirectPick::Rows16 : fits(32, 32) ? DirectPick::Rows32 : fits(32, 64) ? DirectPick::Cols64
+                                                                                               : DirectPick::None;
+}
+
 bool gemm_ring_supported(const GemmArgs &p, int out_dtype) {
   const int ob = out_dtype == XFH_BF16 ? 2 : 4;
   if (p.pair_blk && (p.pair_blk % 4 || !aligned(p.C, 4 * ob) || p.sC % 4)) return false;
@@ -519,6 +541,15 @@ int gemm_ring(const GemmArgs &p, int64_t batch, int out_dtype, bool glu, hipStre
   int cus = 0;
   XFH_TRY(device_cu_count(&cus));
   KernelTimer timer("gemm_ring", s, 2.0 * double(p.M) * double(p.N) * double(p.K) * double(batch), true);
+  const DirectPick direct = pick_direct(p, batch, cus);
+  if (direct != DirectPick::None) {
+    KernelTimer config_timer("gemm_direct", s);
+    switch (direct) {
+      case DirectPick::Rows16: return launch_direct<Direct16>(p, batch, out_dtype, glu, s, timer);
+      case DirectPick::Rows32: return launch_direct<Direct32>(p, batch, out_dtype, glu, s, timer);
+      default: return launch_direct<Direct64>(p, batch, out_dtype, glu, s, timer);
+    }
+  }
   const RingPick pick = pick_ring(p, batch, glu, cus);
   const int bn = pick == RingPick::XWide ? 192 : pick == RingPick::Shallow ? 128 : pick == RingPick::Mid ? 96 : 64;
   // Per-XCD row runs when row blocks span several tiles, the whole B operand fits comfortably
