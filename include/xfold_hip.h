@@ -195,6 +195,33 @@ int xfh_attention_operands(const void *q, const void *k, const void *vt, const u
                            const void *bias, int bias_dtype, const void *gate, void *out, int64_t B, int64_t T,
                            int64_t H, int64_t Dh, void *stream);
 
+/* Weights of xfh_cross_attention (host struct): [128][128] bf16 matrices, fp32 vectors (biases and
+ * LayerNorm parameters may be NULL). */
+typedef struct XfhCrossWeights {
+  const float *q_cond_w, *q_cond_b;                /* q_adaptive_layernorm */
+  const void *q_scale, *q_shift;
+  const float *q_scale_b;
+  const float *k_cond_w, *k_cond_b;                /* k_adaptive_layernorm */
+  const void *k_scale, *k_shift;
+  const float *k_scale_b;
+  const void *q;
+  const float *q_b;
+  const void *k, *v, *gating, *zero;               /* zero: adaptive_zero_cond */
+  const float *zero_b;
+  const void *output;                              /* transition2 */
+} XfhCrossWeights;
+
+/* CrossAttention.forward (xfold/nn/diffusion_transformer.py:304-350), bf16 compute, 128 channels and 4
+ * heads of 32: x_q, cond_q [subsets][nq][128], x_k, cond_k [subsets][nk][128] (one dtype), masks
+ * [subsets][nq] and [subsets][nk], logits element (b, h, q, k) at logit_strides (or NULL),
+ * 1 <= nk <= 128; out [subsets][nq][128] stored or accumulated. eps: q condition, x_q, k condition, x_k. */
+int64_t xfh_cross_attention_workspace_size(int64_t subsets, int64_t nq, int64_t nk);
+int xfh_cross_attention(const void *x_q, const void *x_k, const void *cond_q, const void *cond_k, int x_dtype,
+                        const void *mask_q, int mask_q_dtype, const void *mask_k, int mask_k_dtype,
+                        const void *logits, int logit_dtype, const int64_t *logit_strides, int64_t subsets, int64_t nq,
+                        int64_t nk, const XfhCrossWeights *weights, const float *eps, float scale, void *out,
+                        int out_dtype, int accumulate, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* Weights of xfh_pair_updates (host struct of device pointers, as the single entry points take them). */
 typedef struct XfhPairWeights {
   struct {

@@ -62,3 +62,34 @@ def test_cross_attention_broadcast_pair_logits_and_bool_masks(device):
     with torch.inference_mode():
         got = hip(*(t.to(device) for t in (x_q, x_k, mask_q > 0, mask_k > 0, pair, cond_q, cond_k)))
     assert_parity(got, want, TOL_FP32, "cross_attention broadcast")
+
+
+@pytest.mark.parametrize("nq,nk", [(32, 128), (5, 7), (33, 97), (64, 32), (1, 1), (40, 129)])
+@pytest.mark.parametrize("logits", ["head_minor", "contiguous", "odd", None])
+def test_cross_attention_atom_widths(device, nq, nk, logits):
+    """128 channels and 4 heads in bf16 (the three fused kernels up to 128 keys, the composed path
+    beyond): query and key counts off their tiles, logits heads innermost, contiguous, in rows
+    no four of which are aligned, and absent; the result stored and accumulated."""
+    announce("cross_attention atom", nq, nk, logits)
+    ref, hip = pair_of("CrossAttention", dict(key_dim=128, value_dim=128, c_single_cond=128, num_head=4), seed=nq + nk)
+    x_q, x_k, mask_q, mask_k, pair, cond_q, cond_k = cross_inputs(5, nq, nk, 128, 4, seed=nq * nk)
+    mask_k[..., 0] = 1.0                             # no masked query without an unmasked key's subset: 1e9 swamps fp32
+    mask_q[:] = 1.0
+    mask_q[0, -1] = 0.0
+    x_q, x_k, cond_q, cond_k = (t.bfloat16() for t in (x_q, x_k, cond_q, cond_k))
+    pair = None if logits is None else pair.bfloat16()
+    on_gpu = None if pair is None else pair.to(device)
+    if logits == "head_minor":
+        base = torch.randn(5, nq, nk, 12).bfloat16().to(device)
+        base[..., 4:8] = on_gpu.permute(0, 2, 3, 1)
+        on_gpu = base[..., 4:8].permute(0, 3, 1, 2)
+    elif logits == "odd":
+        base = torch.zeros(5, 4, nq, nk + 1, dtype=torch.bfloat16, device=device)
+        base[..., 1:] = on_gpu
+        on_gpu = base[..., 1:]
+    f32 = lambda t: None if t is None else t.float()
+    dev = lambda t: None if t is None else t.to(device)
+    check_module(ref, hip, hnn.cross_attention_hip,
+                 (f32(x_q), f32(x_k), mask_q, mask_k, f32(pair), f32(cond_q), f32(cond_k)),
+                 (dev(x_q), dev(x_k), dev(mask_q), dev(mask_k), on_gpu, dev(cond_q), dev(cond_k)), True,
+                 "cross_attention atom")

@@ -564,6 +564,10 @@ def cross_attention_hip(module: nn.Module, x_q: torch.Tensor, x_k: torch.Tensor,
     if accumulate_into is not None and (not accumulate_into.is_contiguous() or
                                         tuple(accumulate_into.shape) != lead + (nq, vd)):
         raise ValueError("accumulate_into must be a contiguous [..., Q, value_dim] tensor")
+    fused = _cross_attention_fused(module, x_q, x_k, mask_q, mask_k, pair_logits, single_cond_q, single_cond_k, dtype,
+                                   lead, batch, accumulate_into)
+    if fused is not None:
+        return fused
     xq = _adaptive_layer_norm(module.q_adaptive_layernorm, x_q, single_cond_q, dtype)
     xk = _adaptive_layer_norm(module.k_adaptive_layernorm, x_k, single_cond_k, dtype)
     q = ops.linear(xq, w_q, nh.param(module, "q_projection", "bias"), dtype)
@@ -588,6 +592,84 @@ def cross_attention_hip(module: nn.Module, x_q: torch.Tensor, x_k: torch.Tensor,
     ops.attention(q4, k4, v4, None, bias, out=o_view, scale=module.q_scale)
     ops.linear(xq, w_gate, None, dtype, out=o, epilogue=nh.EPI_SIGMOID_MUL_AUX, aux=o)
     return _ada_ln_zero(module.adaptive_zero_init, o, single_cond_q, dtype, accumulate_into)
+
+
+def _cross_sources(module: nn.Module):
+    """Parameters of a conditioned CrossAttention: the matrices, then biases and LayerNorms."""
+    m = module._modules
+    alns, zero = (m["q_adaptive_layernorm"], m["k_adaptive_layernorm"]), m["adaptive_zero_init"]
+    matrices = [nh.param(a, n) for a in alns for n in ("single_cond_scale", "single_cond_bias")]
+    matrices += nh.params(module, _QKV + ("gating_query",)) + nh.params(zero, ("adaptive_zero_cond", "transition2"))
+    rest = [nh.param(module, "q_projection", "bias"), nh.param(zero, "adaptive_zero_cond", "bias")]
+    for a in alns:
+        rest += (nh.param(a, "single_cond_scale", "bias"), nh.param(a, "single_cond_layer_norm"),
+                 nh.param(a, "single_cond_layer_norm", "bias"))
+    return matrices, rest
+
+
+def _cross_values(module: nn.Module, dtype: torch.dtype):
+    """The prepared weights in ``XfhCrossWeights`` order."""
+    m = module._modules
+    alns, zero = (m["q_adaptive_layernorm"], m["k_adaptive_layernorm"]), m["adaptive_zero_init"]
+    out = []
+    for a in alns:
+        out += (*nh.norm_params(a, "single_cond_layer_norm"), nh.linear_weight(a, "single_cond_scale", dtype),
+                nh.linear_weight(a, "single_cond_bias", dtype),
+                nh.fp32_param(a, "single_cond_scale.bias", nh.param(a, "single_cond_scale", "bias")))
+    out += (nh.linear_weight(module, "q_projection", dtype),
+            nh.fp32_param(module, "q_projection.bias", nh.param(module, "q_projection", "bias")))
+    out += (nh.linear_weight(module, n, dtype) for n in ("k_projection", "v_projection", "gating_query"))
+    out += (nh.linear_weight(zero, "adaptive_zero_cond", dtype),
+            nh.fp32_param(zero, "adaptive_zero_cond.bias", nh.param(zero, "adaptive_zero_cond", "bias")),
+            nh.linear_weight(zero, "transition2", dtype))
+    return out
+
+
+def _cross_attention_fused(module: nn.Module, x_q, x_k, mask_q, mask_k, pair_logits, cond_q, cond_k,
+                           dtype: torch.dtype, lead: tuple, batch: int, accumulate_into) -> Optional[torch.Tensor]:
+    """The call in three launches (``xfh_cross_attention``) at the atom attention's widths: bf16
+    compute, 128 channels, 4 heads, at most 128 keys, one activation dtype, every condition
+    given; None otherwise. With the subsets' logits broadcast over outer leading dims the
+    general path's one copy of them stays."""
+    alns = (module.q_adaptive_layernorm, module.k_adaptive_layernorm)
+    zero = module.adaptive_zero_init
+    nq, nk = x_q.shape[-2], x_k.shape[-2]
+    acts = (x_q, x_k, cond_q, cond_k)
+    if (dtype != torch.bfloat16 or module.num_head != 4 or module.key_dim != 128 or module.value_dim != 128
+            or cond_q is None or cond_k is None or not zero.use_single_cond
+            or not all(a.use_single_cond for a in alns) or not 1 <= nk <= 128 or nq == 0
+            or any(t.dtype != x_q.dtype for t in acts) or x_q.dtype not in (torch.float32, torch.bfloat16)
+            or tuple(x_q.shape) != lead + (nq, 128) or tuple(x_k.shape) != lead + (nk, 128)
+            or cond_q.shape != x_q.shape or cond_k.shape != x_k.shape
+            or any(tuple(a.single_cond_layer_norm.normalized_shape) != (128,)
+                   or tuple(a.layer_norm.normalized_shape) != (128,) for a in alns)):
+        return None
+    matrices, rest = _cross_sources(module)
+    if any(tuple(w.shape) != (128, 128) for w in matrices) or any(nh.param(a, "single_cond_bias", "bias") is not None
+                                                                  for a in alns):
+        return None
+    logits, code, strides = None, nh.F32, None
+    if pair_logits is not None:
+        if pair_logits.dtype not in (torch.float32, torch.bfloat16):
+            raise ValueError("CrossAttention: pair_logits must be fp32 or bf16")
+        logits = pair_logits.expand(*lead, 4, nq, nk).reshape(batch, 4, nq, nk)
+        code, strides = nh.dtype_code(logits.dtype), (ctypes.c_int64 * 4)(*logits.stride())
+    _, values = nh.gather(module, "fused", matrices + rest, 0, x_q, lambda dt: _cross_values(module, dt), dtype)
+    mq, mq_code = nh.mask_arg(mask_q, lead + (nq,))
+    mk, mk_code = nh.mask_arg(mask_k, lead + (nk,))
+    acts = [t.contiguous() for t in acts]
+    out = accumulate_into
+    if out is None:
+        out = torch.empty(lead + (nq, 128), dtype=dtype, device=x_q.device)
+    if any(t.data_ptr() % 16 for t in (*acts, out)):
+        return None
+    eps = (ctypes.c_float * 4)(*(e for a in alns for e in (a.single_cond_layer_norm.eps, a.layer_norm.eps)))
+    lib = nh.load_library()
+    ws = nh.workspace(lib.xfh_cross_attention_workspace_size(batch, nq, nk), x_q.device)
+    nh.call("xfh_cross_attention", *map(nh.ptr, acts), nh.dtype_code(x_q.dtype), nh.ptr(mq), mq_code, nh.ptr(mk), mk_code,
+            nh.ptr(logits), code, strides, batch, nq, nk, nh.ptrs(values), eps, float(module.q_scale), nh.ptr(out),
+            nh.dtype_code(out.dtype), int(accumulate_into is not None), nh.ptr(ws), ws.numel(), nh.stream_of(x_q.device))
+    return out
 
 
 class CrossAttention(nn.Module):
