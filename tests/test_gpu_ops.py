@@ -435,6 +435,32 @@ def test_triangle_multiplication_other_widths(device, c, n, bf16):
                  (pair.to(device), mask.to(device)), bf16, f"trimul c={c}")
 
 
+@pytest.mark.parametrize("n", [1, 31, 65, 130])
+def test_pair_operators_at_64_channels(device, n):
+    """The fused kernels at 64 channels (4 heads of 16; 128 and 256 hidden features) around the ends of
+    their 16- and 32-position units, for a bf16 and an fp32 pair; a pair whose rows are not
+    16-byte aligned takes the general kernels and gives the same update."""
+    announce("64 channels", n)
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(n, n, 64, generator=g).bfloat16()
+    mask = torch.ones(n, n)
+    mask[:, n // 2:n // 2 + 1] = 0 if n > 1 else 1
+    cases = [("TriangleMultiplication", dict(c_pair=64, _outgoing=o), hnn.triangle_multiplication_hip) for o in (True, False)]
+    cases += [("GridSelfAttention", dict(c_pair=64, num_head=4, transpose=t), hnn.grid_self_attention_hip) for t in (False, True)]
+    cases += [("Transition", dict(c_x=64, num_intermediate_factor=f), hnn.transition_hip) for f in (2, 4)]
+    for name, args, fn in cases:
+        ref, hip = pair_of(name, args, seed=n + len(name))
+        extra = () if name == "Transition" else (mask,)
+        dev = tuple(t.to(device) for t in extra)
+        check_module(ref, hip, fn, (x.float(), *extra), (x.to(device), *dev), True, f"{name} c=64")
+        want, floor = ref(x.float(), *extra), floor_of(lambda: ref(x.float(), *extra))
+        odd = torch.zeros(n * n * 64 + 1, dtype=torch.bfloat16, device=device)[1:].view(n, n, 64)
+        odd.copy_(x)
+        with torch.inference_mode(), autocast(True):
+            assert_parity_bf16(hip(x.float().to(device), *dev), want, f"{name} c=64 fp32 pair", floor=bf16_stored(floor))
+            assert_parity_bf16(hip(odd, *dev), want, f"{name} c=64 unaligned", floor=bf16_stored(floor))
+
+
 # n = 520: enough 32-position units (520 x 17) for the 32-position projection path on a
 # 256-CU device; the smaller sizes take the 16-position path.
 @pytest.mark.parametrize("n,mask_dtype", [(33, torch.float32), (96, torch.bfloat16), (45, torch.bool),

@@ -1,8 +1,10 @@
 // C ABI of libxfold_hip.so: validation, workspace carving and kernel sequencing.
 // Declarations and their reference counterparts are in include/xfold_hip.h.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -120,13 +122,17 @@ struct TriMulPlan {
   void *normed, *proj, *gate, *left, *right, *contracted, *centered, *gating;
 };
 
-static bool trimul_fast_path(int64_t c, int dtype) { return dtype == XFH_BF16 && c == 128; }
+static bool trimul_fast_path(int64_t c, int dtype) { return dtype == XFH_BF16 && (c == 128 || c == 64); }
+static bool aligned16(std::initializer_list<const void *> ptrs) {
+  for (const void *p : ptrs)
+    if (reinterpret_cast<uintptr_t>(p) % 16) return false;
+  return true;
+}
 
-
-static int64_t trimul_carve(Carver &cv, TriMulPlan &p, int64_t n, int64_t c, int dtype, int out_dtype) {
+static int64_t trimul_carve(Carver &cv, TriMulPlan &p, int64_t n, int64_t c, int dtype, int out_dtype, bool fast) {
   const int64_t es = dsize(dtype), plane = n * n;
   std::memset(&p, 0, sizeof(p));
-  if (trimul_fast_path(c, dtype)) {
+  if (fast) {
     p.left = cv.take(contraction_operand_elems(n, c) * es);
     p.right = cv.take(contraction_operand_elems(n, c) * es);
     p.contracted = cv.take(contraction_result_elems(n, c) * es);
@@ -156,13 +162,13 @@ struct GridPlan {
 };
 
 static bool grid_fast_path(int64_t n, int64_t c, int64_t heads, int dtype) {
-  return dtype == XFH_BF16 && c == 128 && heads == 4 && n <= grid_attention_max_n();
+  return dtype == XFH_BF16 && (c == 128 || c == 64) && heads == 4 && n <= grid_attention_max_n();
 }
 
-static int64_t grid_carve(Carver &cv, GridPlan &p, int64_t n, int64_t c, int64_t heads, int dtype) {
+static int64_t grid_carve(Carver &cv, GridPlan &p, int64_t n, int64_t c, int64_t heads, int dtype, bool fast) {
   const int64_t es = dsize(dtype), plane = n * n;
   std::memset(&p, 0, sizeof(p));
-  if (grid_fast_path(n, c, heads, dtype)) {
+  if (fast) {
     const int64_t npad = grid_attention_pad(n);
     p.qh = cv.take(plane * c * es);
     p.kh = cv.take(n * c * npad * es);
@@ -513,9 +519,15 @@ int xfh_pair_attention_bias(const void *pair, int pair_dtype, int64_t n, int64_t
 
 int64_t xfh_triangle_multiplication_workspace_size(int64_t n, int64_t c, int dtype) {
   if (n < 0 || c < 0 || !float_dtype(dtype)) return -1;
-  Carver cv(nullptr, 0);
-  TriMulPlan p;
-  return trimul_carve(cv, p, n, c, dtype, XFH_F32) + 256;
+  // At 64 channels the general path still takes operands that are not 16-byte aligned: room for both.
+  int64_t most = 0;
+  for (int fast = 0; fast < 2; ++fast) {
+    if (fast ? !trimul_fast_path(c, dtype) : c == 128 && trimul_fast_path(c, dtype)) continue;
+    Carver cv(nullptr, 0);
+    TriMulPlan p;
+    most = std::max(most, trimul_carve(cv, p, n, c, dtype, XFH_F32, fast != 0));
+  }
+  return most + 256;
 }
 
 int xfh_triangle_multiplication(const void *pair, int pair_dtype, const void *mask, int mask_dtype,
@@ -535,19 +547,21 @@ int xfh_triangle_multiplication(const void *pair, int pair_dtype, const void *ma
   XFH_REQUIRE(pair && out && proj_w && gate_w && out_w && gating_w, "triangle_multiplication: null tensor");
   Carver cv(workspace, workspace_bytes);
   TriMulPlan p;
-  const int64_t need = trimul_carve(cv, p, n, c, dtype, out_dtype);
+  const bool fast = trimul_fast_path(c, dtype) &&
+                    (c == 128 || aligned16({pair, out, proj_w, gate_w, out_w, gating_w}));
+  const int64_t need = trimul_carve(cv, p, n, c, dtype, out_dtype, fast);
   if (!workspace || need > workspace_bytes)
     return fail(XFH_EWORKSPACE, "triangle_multiplication: workspace too small (need " +
                                     std::to_string(need) + " bytes)");
   hipStream_t s = as_stream(stream);
   const int64_t plane = n * n;
-  if (trimul_fast_path(c, dtype)) {
+  if (fast) {
     TriProjectArgs pa;
     pa.pair = pair; pa.mask = mask; pa.mask_dtype = mask_dtype;
     pa.ln_w = left_w; pa.ln_b = left_b; pa.eps = left_eps;
     pa.w_proj = static_cast<const bf16 *>(proj_w); pa.w_gate = static_cast<const bf16 *>(gate_w);
     pa.left = static_cast<bf16 *>(p.left); pa.right = static_cast<bf16 *>(p.right);
-    pa.n = int(n); pa.ld = int(contraction_ld(n)); pa.outgoing = outgoing;
+    pa.n = int(n); pa.ld = int(contraction_ld(n)); pa.outgoing = outgoing; pa.c = int(c);
     XFH_TRY(trimul_project(pa, pair_dtype, s));
     ContractionArgs ca;
     ca.left = static_cast<const bf16 *>(p.left);
@@ -560,7 +574,7 @@ int xfh_triangle_multiplication(const void *pair, int pair_dtype, const void *ma
     oa.ln_in_w = left_w; oa.ln_in_b = left_b; oa.eps_in = left_eps;
     oa.ln_c_w = center_w; oa.ln_c_b = center_b; oa.eps_c = center_eps;
     oa.w_gating = static_cast<const bf16 *>(gating_w); oa.w_out = static_cast<const bf16 *>(out_w);
-    oa.out = out; oa.accumulate = accumulate; oa.n = int(n);
+    oa.out = out; oa.accumulate = accumulate; oa.n = int(n); oa.c = int(c);
     return trimul_output(oa, pair_dtype, out_dtype, s);
   }
   XFH_TRY(layer_norm_rows(pair, pair_dtype, plane, c, left_w, left_b, left_eps, p.normed, dtype, s));
@@ -585,9 +599,14 @@ int xfh_triangle_multiplication(const void *pair, int pair_dtype, const void *ma
 
 int64_t xfh_grid_self_attention_workspace_size(int64_t n, int64_t c, int64_t heads, int dtype) {
   if (n < 0 || c < 0 || heads <= 0 || !float_dtype(dtype)) return -1;
-  Carver cv(nullptr, 0);
-  GridPlan p;
-  return grid_carve(cv, p, n, c, heads, dtype) + 256;
+  int64_t most = 0;
+  for (int fast = 0; fast < 2; ++fast) {                // (both at 64 channels, as for the triangle multiplication)
+    if (fast ? !grid_fast_path(n, c, heads, dtype) : c == 128 && grid_fast_path(n, c, heads, dtype)) continue;
+    Carver cv(nullptr, 0);
+    GridPlan p;
+    most = std::max(most, grid_carve(cv, p, n, c, heads, dtype, fast != 0));
+  }
+  return most + 256;
 }
 
 int xfh_grid_self_attention(const void *pair, int pair_dtype, const void *mask, int mask_dtype,
@@ -607,7 +626,9 @@ int xfh_grid_self_attention(const void *pair, int pair_dtype, const void *mask, 
               "grid_self_attention: null tensor");
   Carver cv(workspace, workspace_bytes);
   GridPlan p;
-  const int64_t need = grid_carve(cv, p, n, c, heads, dtype);
+  const bool fast = grid_fast_path(n, c, heads, dtype) &&
+                    (c == 128 || aligned16({pair, out, bias_w, q_w, k_w, v_w, gating_w, out_w}));
+  const int64_t need = grid_carve(cv, p, n, c, heads, dtype, fast);
   if (!workspace || need > workspace_bytes)
     return fail(XFH_EWORKSPACE, "grid_self_attention: workspace too small (need " +
                                     std::to_string(need) + " bytes)");
@@ -616,7 +637,7 @@ int xfh_grid_self_attention(const void *pair, int pair_dtype, const void *mask, 
   // Batch row b, position t of the (optionally transposed) grid lives at pair row
   // b*n + t (starting node) or t*n + b (ending node); the output keeps pair rows.
   const int64_t row_b = transpose ? 1 : n, row_t = transpose ? n : 1;
-  if (grid_fast_path(n, c, heads, dtype)) {
+  if (fast) {
     const int64_t npad = grid_attention_pad(n);
     GridProjectArgs pa;
     pa.pair = pair; pa.n = int(n); pa.heads = int(heads); pa.transpose = transpose;
@@ -626,7 +647,7 @@ int xfh_grid_self_attention(const void *pair, int pair_dtype, const void *mask, 
     pa.mask = mask; pa.mask_dtype = mask_dtype; pa.maskbits = p.maskbits;
     pa.qscale = kLog2e / std::sqrt(float(dh));
     pa.q = static_cast<bf16 *>(p.qh); pa.k = static_cast<bf16 *>(p.kh); pa.vt = static_cast<bf16 *>(p.vt);
-    pa.bias = p.bias_t; pa.npad = int(npad);
+    pa.bias = p.bias_t; pa.npad = int(npad); pa.c = int(c);
     XFH_TRY(grid_project(pa, pair_dtype, s));
     GridAttentionArgs ga;
     ga.q = static_cast<const bf16 *>(p.qh);
@@ -643,12 +664,13 @@ int xfh_grid_self_attention(const void *pair, int pair_dtype, const void *mask, 
     ga.Nblk = ga.Npad / 64;
     ga.mbs = ga.Nblk;
     ga.Dv = int(dh);
-    XFH_TRY(grid_attention(ga, s));
+    if (c == 128) XFH_TRY(grid_attention(ga, s));
+    else XFH_TRY(mha_attention(ga, int(dh), s));
     GridOutputArgs oa;
     oa.pair = pair; oa.attn = static_cast<const bf16 *>(p.attn);
     oa.ln_w = norm_w; oa.ln_b = norm_b; oa.eps = eps;
     oa.w_gating = static_cast<const bf16 *>(gating_w); oa.w_out = static_cast<const bf16 *>(out_w);
-    oa.out = out; oa.accumulate = accumulate; oa.n = int(n);
+    oa.out = out; oa.accumulate = accumulate; oa.n = int(n); oa.c = int(c);
     return grid_output(oa, pair_dtype, out_dtype, s);
   }
   XFH_TRY(layer_norm_rows(pair, pair_dtype, plane, c, norm_w, norm_b, eps, p.normed, dtype, s));
@@ -742,11 +764,13 @@ int xfh_transition(const void *x, int x_dtype, int64_t rows, int64_t c, int64_t 
               "transition: dtypes must be f32/bf16");
   if (rows == 0) return XFH_OK;
   XFH_REQUIRE(x && out && w1_packed && w2, "transition: null tensor");
-  if (dtype == XFH_BF16 && c == 128 && f == 512) {
+  const bool narrow = c == 64 && (f == 128 || f == 256) && aligned16({x, out, w1_packed, w2});
+  if (dtype == XFH_BF16 && ((c == 128 && f == 512) || narrow)) {
     TransitionArgs ta;
     ta.x = x; ta.rows = rows; ta.ln_w = norm_w; ta.ln_b = norm_b; ta.eps = eps;
     ta.w1 = static_cast<const bf16 *>(w1_packed); ta.w2 = static_cast<const bf16 *>(w2);
     ta.out = out; ta.accumulate = accumulate;
+    if (narrow) return transition_rows(ta, int(f), x_dtype, out_dtype, as_stream(stream));
     return transition_fused(ta, x_dtype, out_dtype, as_stream(stream));
   }
   Carver cv(workspace, workspace_bytes);

@@ -21,8 +21,10 @@ namespace {
 
 using namespace panel;
 
-constexpr int HD = 32;                 // head dim
-constexpr int QKV_ROWS = 3 * K;        // q, k, v weight rows in LDS, then the bias rows
+// Channels K = 128 in 4 heads of 32, or 64 in 4 heads of 16 (the template stack), where the
+// weights and registers leave room for two workgroups per CU.
+constexpr int GRID_HEADS = 4;
+constexpr int wgs_per_cu(int k) { return k == 64 ? 2 : 1; }
 
 // grid_project, one wavefront per unit of 32 attention positions t0 .. t0 + 31 of one batch
 // row b (t0 a multiple of 32, t up to npad so the pad rows and columns come out as zeros),
@@ -36,14 +38,15 @@ constexpr int QKV_ROWS = 3 * K;        // q, k, v weight rows in LDS, then the b
 //          (tile 1): exactly the 8 keys of positions t0 + 8 g .. + 7 of the permuted layout;
 //   bias:  out = x W^T, 4 consecutive keys per lane (starting node) or one value per
 //          (query t, key b) (ending node).
-constexpr int W_ROWS = QKV_ROWS + 16;  // q, k, v, then one tile of bias rows (heads <= 16)
-
-template <typename TIN>
-__global__ __launch_bounds__(512, 1) void grid_project_kernel(GridProjectArgs a) {
+template <typename TIN, int K>
+__global__ __launch_bounds__(512, wgs_per_cu(K)) void grid_project_kernel(GridProjectArgs a) {
+  constexpr int KS = K / 32, HD = K / GRID_HEADS;
+  constexpr int QKV_ROWS = 3 * K;      // q, k, v weight rows in LDS, then the bias rows
+  constexpr int W_ROWS = QKV_ROWS + 16;  // one tile of bias rows (heads <= 16)
   __shared__ __attribute__((aligned(16))) bf16 w_lds[W_ROWS * K];
   __shared__ __attribute__((aligned(16))) float lnw[K], lnb[K];
-  rowstep::WeightStage<W_ROWS, 512> sw;
-  rowstep::LnStage sl;
+  rowstep::WeightStage<W_ROWS, 512, K> sw;
+  rowstep::LnStageOf<K> sl;
   sw.load([&](int r) -> const bf16 * {
     const int blk = r / K, rr = r % K;              // q, k, v, bias
     if (blk < 2) {                                  // q, k: rows permuted inside each head
@@ -80,7 +83,7 @@ __global__ __launch_bounds__(512, 1) void grid_project_kernel(GridProjectArgs a)
   // Pair row of attention position (b, t): b*n + t (starting node) or t*n + b (ending node).
   auto pos_of = [&](int b, int t) -> int64_t { return a.transpose ? int64_t(t) * n + b : int64_t(b) * n + t; };
   struct Unit {
-    rowstep::Raw4<TIN> z[2][8];
+    rowstep::Raw4<TIN> z[2][K / 16];
   };
   auto fetch = [&](int u, Unit &w) {
     const int b = u / upr, t0 = (u - b * upr) * 32;
@@ -99,10 +102,10 @@ __global__ __launch_bounds__(512, 1) void grid_project_kernel(GridProjectArgs a)
   for (; u < units; u += waves) {
     Unit next;
     if (u + waves < units) fetch(u + waves, next);
-    bf16x8 xa[2][4];
+    bf16x8 xa[2][KS];
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
-      float v[32];
+      float v[K / 4];
       rowstep::k_to_float(cur.z[rt], v);
       rowstep::ln_k(v, lnw, lnb, a.eps, xa[rt]);
     }
@@ -116,17 +119,17 @@ __global__ __launch_bounds__(512, 1) void grid_project_kernel(GridProjectArgs a)
       const int rows = blk == 0 ? n : npad;
       bf16 *dst_base = blk == 0 ? a.q : a.k;
 #pragma unroll 1
-      for (int s = 0; s < H; ++s) {
+      for (int s = 0; s < KS; ++s) {           // 32 channels: one head, or two of 16
         f32x4 acc[2][2];
 #pragma unroll
         for (int p = 0; p < 2; ++p)
 #pragma unroll
           for (int rt = 0; rt < 2; ++rt) acc[p][rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
           for (int p = 0; p < 2; ++p) {
-            const bf16x8 wf = rowstep::weight_frag(wb, 2 * s + p, ks);
+            const bf16x8 wf = rowstep::weight_frag<K>(wb, 2 * s + p, ks);
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt) acc[p][rt] = mfma16(wf, xa[rt][ks], acc[p][rt]);
           }
@@ -141,7 +144,8 @@ __global__ __launch_bounds__(512, 1) void grid_project_kernel(GridProjectArgs a)
             v[4 + e] = bf16(acc[1][rt][e] * scale);
           }
           if (t >= n) v = bf16x8{};
-          *reinterpret_cast<bf16x8 *>(dst_base + ((int64_t(b) * H + s) * rows + t) * HD + 8 * g) = v;
+          const int c0 = 32 * s + 8 * g, h = c0 / HD, d = c0 % HD;
+          *reinterpret_cast<bf16x8 *>(dst_base + ((int64_t(b) * H + h) * rows + t) * HD + d) = v;
         }
       }
     }
@@ -153,8 +157,8 @@ __global__ __launch_bounds__(512, 1) void grid_project_kernel(GridProjectArgs a)
       for (int tile = 0; tile < K / 16; ++tile) {
         f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          const bf16x8 wf = rowstep::weight_frag(wv, tile, ks);
+        for (int ks = 0; ks < KS; ++ks) {
+          const bf16x8 wf = rowstep::weight_frag<K>(wv, tile, ks);
 #pragma unroll
           for (int rt = 0; rt < 2; ++rt) acc[rt] = mfma16(xa[rt][ks], wf, acc[rt]);
         }
@@ -175,8 +179,8 @@ __global__ __launch_bounds__(512, 1) void grid_project_kernel(GridProjectArgs a)
       const bf16 *wbias = w_lds + QKV_ROWS * K;
       f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const bf16x8 wf = rowstep::weight_frag(wbias, 0, ks);
+      for (int ks = 0; ks < KS; ++ks) {
+        const bf16x8 wf = rowstep::weight_frag<K>(wbias, 0, ks);
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) acc[rt] = mfma16(xa[rt][ks], wf, acc[rt]);
       }
@@ -215,13 +219,14 @@ __global__ __launch_bounds__(512, 1) void grid_project_kernel(GridProjectArgs a)
 //   u^T    = Wout . y^T                (y is the k operand as it stands, Wout in kperm order)
 //   z     += bf16(u)                   (bf16 pair updated in place: the residual is the z
 //                                       already loaded, moved to O-layout the same way)
-template <typename TIN, typename TOUT>
-__global__ __launch_bounds__(512, 1) void grid_output_kernel(GridOutputArgs a) {
-  __shared__ __attribute__((aligned(16))) bf16 w_gate[rowstep::W_ELEMS];
-  __shared__ __attribute__((aligned(16))) bf16 w_out[rowstep::W_ELEMS];
+template <typename TIN, typename TOUT, int K>
+__global__ __launch_bounds__(512, wgs_per_cu(K)) void grid_output_kernel(GridOutputArgs a) {
+  constexpr int KS = K / 32, NT = K / 16;
+  __shared__ __attribute__((aligned(16))) bf16 w_gate[K * K];
+  __shared__ __attribute__((aligned(16))) bf16 w_out[K * K];
   __shared__ __attribute__((aligned(16))) float lnw[K], lnb[K];
-  rowstep::WeightStage<K, 512> sg, so;
-  rowstep::LnStage sl;
+  rowstep::WeightStage<K, 512, K> sg, so;
+  rowstep::LnStageOf<K> sl;
   sg.load([&](int row) { return a.w_gating + row * K; }, false);
   so.load([&](int row) { return a.w_out + row * K; }, true);
   sl.load(a.ln_w, a.ln_b);
@@ -240,15 +245,15 @@ __global__ __launch_bounds__(512, 1) void grid_output_kernel(GridOutputArgs a) {
   rowstep::identity_frags(id);
 
   struct Rows {
-    rowstep::Raw4<TIN> z[8];                       // K-layout
-    bf16x8 att[4];                                 // K-layout
-    rowstep::Raw4<TOUT> res[8];                    // O-layout (only when not derived from z)
+    rowstep::Raw4<TIN> z[NT];                       // K-layout
+    bf16x8 att[KS];                                 // K-layout
+    rowstep::Raw4<TOUT> res[NT];                    // O-layout (only when not derived from z)
   };
   auto fetch = [&](int64_t st, Rows &rw) {
     const int64_t pos = st * 16 + r, pc = pos < npos ? pos : npos - 1;
     rowstep::load_k<TIN>(z + pc * K, rw.z);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) rw.att[ks] = *reinterpret_cast<const bf16x8 *>(a.attn + pc * K + 32 * ks + 8 * g);
+    for (int ks = 0; ks < KS; ++ks) rw.att[ks] = *reinterpret_cast<const bf16x8 *>(a.attn + pc * K + 32 * ks + 8 * g);
     if (res_load) rowstep::load_o<TOUT>(out + pc * K, rw.res);
   };
   // Rows of the next step are loaded while this one is computed.
@@ -262,33 +267,33 @@ __global__ __launch_bounds__(512, 1) void grid_output_kernel(GridOutputArgs a) {
   for (; st < steps; st += waves) {
     Rows next;
     if (st + waves < steps) fetch(st + waves, next);
-    bf16x8 x[4];
+    bf16x8 x[KS];
     {
-      float v[32];
+      float v[K / 4];
       rowstep::k_to_float(cur.z, v);
       rowstep::ln_k(v, lnw, lnb, a.eps, x);
     }
-    f32x4 acc[8];
+    f32x4 acc[NT];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     rowstep::gemm_t(w_gate, x, acc);
-    f32x4 att[8];
+    f32x4 att[NT];
     rowstep::k_to_o(id, cur.att, att);
-    float y[8][4];
+    float y[NT][4];
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[t][e] = sigmoidf_(acc[t][e]) * att[t][e];
     rowstep::o_to_operand(y, x);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     rowstep::gemm_t(w_out, x, acc);
-    f32x4 res[8];
+    f32x4 res[NT];
     if (res_from_z) {
       if constexpr (kBf16) {
-        bf16x8 zk[4];
+        bf16x8 zk[KS];
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             zk[ks][e] = cur.z[2 * ks].v[e];
@@ -298,14 +303,14 @@ __global__ __launch_bounds__(512, 1) void grid_output_kernel(GridOutputArgs a) {
       }
     } else {
 #pragma unroll
-      for (int t = 0; t < 8; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) res[t][e] = res_load ? cur.res[t][e] : 0.f;
     }
     const int64_t pos = st * 16 + r;
     if (pos < npos) {
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
+      for (int t = 0; t < NT; ++t) {
         float o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = res[t][e] + static_cast<float>(bf16(acc[t][e]));  // bf16 update
@@ -318,36 +323,44 @@ __global__ __launch_bounds__(512, 1) void grid_output_kernel(GridOutputArgs a) {
 
 }  // namespace
 
-int grid_project(const GridProjectArgs &a, int pair_dtype, hipStream_t s) {
-  if (a.npad % 64 != 0 || a.npad < a.n || a.heads > 16 || a.heads * HD != K)
-    return fail(XFH_EINVAL, "grid_project: npad must be a multiple of 64 >= n, heads * 32 == 128");
+template <int K> static int launch_project(const GridProjectArgs &a, int pair_dtype, hipStream_t s) {
   const int64_t units = int64_t(a.n) * (a.npad / 32);
   int cus = 0;
   XFH_TRY(device_cu_count(&cus));
-  const dim3 grid(unsigned(balanced_grid(units, 8, cus)));
+  const dim3 grid(unsigned(balanced_grid(units, 8, cus * wgs_per_cu(K))));
   KernelTimer timer("grid_project", s, 0.0, true);
   if (pair_dtype == XFH_BF16)
-    timer.launch(grid_project_kernel<bf16>, dim3(grid), dim3(512), 0, a);
+    timer.launch(grid_project_kernel<bf16, K>, dim3(grid), dim3(512), 0, a);
   else
-    timer.launch(grid_project_kernel<float>, dim3(grid), dim3(512), 0, a);
+    timer.launch(grid_project_kernel<float, K>, dim3(grid), dim3(512), 0, a);
   return check_launch("grid_project");
 }
 
-int grid_output(const GridOutputArgs &a, int pair_dtype, int out_dtype, hipStream_t s) {
+template <int K> static int launch_output(const GridOutputArgs &a, int pair_dtype, int out_dtype, hipStream_t s) {
   const int64_t steps = ceil_div(int64_t(a.n) * a.n, 16);
   int cus = 0;
   XFH_TRY(device_cu_count(&cus));
-  const dim3 grid(unsigned(balanced_grid(steps, 8, cus)));
+  const dim3 grid(unsigned(balanced_grid(steps, 8, cus * wgs_per_cu(K))));
   KernelTimer timer("grid_output", s, 0.0, true);
   if (pair_dtype == XFH_BF16 && out_dtype == XFH_BF16)
-    timer.launch(grid_output_kernel<bf16, bf16>, dim3(grid), dim3(512), 0, a);
+    timer.launch(grid_output_kernel<bf16, bf16, K>, dim3(grid), dim3(512), 0, a);
   else if (pair_dtype == XFH_BF16 && out_dtype == XFH_F32)
-    timer.launch(grid_output_kernel<bf16, float>, dim3(grid), dim3(512), 0, a);
+    timer.launch(grid_output_kernel<bf16, float, K>, dim3(grid), dim3(512), 0, a);
   else if (pair_dtype == XFH_F32 && out_dtype == XFH_F32)
-    timer.launch(grid_output_kernel<float, float>, dim3(grid), dim3(512), 0, a);
+    timer.launch(grid_output_kernel<float, float, K>, dim3(grid), dim3(512), 0, a);
   else
-    timer.launch(grid_output_kernel<float, bf16>, dim3(grid), dim3(512), 0, a);
+    timer.launch(grid_output_kernel<float, bf16, K>, dim3(grid), dim3(512), 0, a);
   return check_launch("grid_output");
+}
+
+int grid_project(const GridProjectArgs &a, int pair_dtype, hipStream_t s) {
+  if (a.npad % 64 != 0 || a.npad < a.n || a.heads != GRID_HEADS || (a.c != 128 && a.c != 64))
+    return fail(XFH_EINVAL, "grid_project: npad must be a multiple of 64 >= n, 4 heads, 128 or 64 channels");
+  return a.c == 64 ? launch_project<64>(a, pair_dtype, s) : launch_project<128>(a, pair_dtype, s);
+}
+
+int grid_output(const GridOutputArgs &a, int pair_dtype, int out_dtype, hipStream_t s) {
+  return a.c == 64 ? launch_output<64>(a, pair_dtype, out_dtype, s) : launch_output<128>(a, pair_dtype, out_dtype, s);
 }
 
 }  // namespace xfh

@@ -128,7 +128,7 @@ struct GridAttentionArgs {
   const bf16 *gate = nullptr;
   int bias_bf16 = 0;
 };
-// Fused grid-attention projection / output (grid_fused.hip), bf16, c = 128, 4 x 32 heads.
+// Fused grid-attention projection / output (grid_fused.hip), bf16, c = 128 or 64 in 4 heads.
 struct GridProjectArgs {
   const void *pair;
   int n, heads, transpose;
@@ -141,7 +141,7 @@ struct GridProjectArgs {
   float qscale;              // d^-0.5 * log2(e)
   bf16 *q, *k, *vt;
   float *bias;
-  int npad;
+  int npad, c;
 };
 struct GridOutputArgs {
   const void *pair;
@@ -150,7 +150,7 @@ struct GridOutputArgs {
   float eps;
   const bf16 *w_gating, *w_out;
   void *out;
-  int accumulate, n;
+  int accumulate, n, c;
 };
 // One launch: the packed [q | k | v | bias] weight of grid_project and the 64-bit
 // kept-key words of the attention kernel (bit s of word b*nblk + s/64 set iff key s < n of
@@ -167,7 +167,7 @@ int qkv_repack(const bf16 *qkv, int64_t ld, int64_t B, int64_t T, int64_t H, int
 int64_t grid_attention_max_n();
 int grid_attention(const GridAttentionArgs &a, hipStream_t s);
 
-// Fused triangle multiplication, bf16 compute, c = 128 (trimul_fused.hip).
+// Fused triangle multiplication, bf16 compute, c = 128 or 64 (trimul_fused.hip).
 struct TriProjectArgs {
   const void *pair;
   const void *mask;
@@ -176,7 +176,7 @@ struct TriProjectArgs {
   float eps;
   const bf16 *w_proj, *w_gate;  // [2c][c] each (nn.Linear layout)
   bf16 *left, *right;        // contraction operands in the blocked operand layout, zero-padded
-  int n, ld, outgoing;
+  int n, ld, outgoing, c;    // c: 128 or 64 channels
 };
 struct TriOutputArgs {
   const void *pair;
@@ -187,7 +187,7 @@ struct TriOutputArgs {
   float eps_c;
   const bf16 *w_gating, *w_out;
   void *out;
-  int accumulate, n;
+  int accumulate, n, c;
 };
 // Fused pair transition (transition_fused.hip), bf16 compute, c = 128, hidden 512.
 struct TransitionArgs {
@@ -201,6 +201,9 @@ struct TransitionArgs {
   int accumulate;
 };
 int transition_fused(const TransitionArgs &a, int x_dtype, int out_dtype, hipStream_t s);
+// The same at c = 64 with f = 128 or 256 hidden features (transition_rows.hip): w1 [2f][64] packed, w2
+// [64][f]; 16-byte aligned pointers.
+int transition_rows(const TransitionArgs &a, int f, int x_dtype, int out_dtype, hipStream_t s);
 // The in-place bf16 pair transition (a.x == a.out, accumulating) followed by the attention
 // bias Linear(LayerNorm(pair)) of the updated pair, computed in the transition's epilogue
 // from the values it stores: the result equals transition_fused then pair_bias (fp32 times

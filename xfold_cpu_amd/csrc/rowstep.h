@@ -1,5 +1,6 @@
 // Register-resident building blocks for the pair-stack kernels whose inputs and outputs
-// are [positions][128 channels] rows (bf16 compute, K = 128).
+// are [positions][128 or 64 channels] rows (bf16 compute). The channel count CC follows from the
+// sizes of the register arrays (KS = CC / 32 k-steps, CC / 16 tiles); the text below is for 128.
 //
 // A wavefront works on 16 positions at a time ("step") with no LDS traffic for its
 // activations and no barriers: lane l handles position l % 16 and channel group
@@ -23,7 +24,7 @@
 namespace xfh {
 namespace rowstep {
 
-constexpr int C = 128;                  // channels
+constexpr int C = 128;                  // channels (default)
 constexpr int W_ELEMS = C * C;          // one weight matrix in LDS (bf16, 32 KB)
 
 // Input channel of MFMA k-slot (ks, g, j) when the operand is an O-layout register set.
@@ -31,22 +32,27 @@ __host__ __device__ constexpr int kperm(int ks, int g, int j) {
   return j < 4 ? 32 * ks + 4 * g + j : 32 * ks + 16 + 4 * g + (j - 4);
 }
 
+// Chunk c of row n sits at c ^ (n & swizzle_mask(CC)).
+__host__ __device__ constexpr int swizzle_mask(int cc) { return (cc / 8 < 16 ? cc / 8 : 16) - 1; }
+
 // Weight rows ([rows][128] bf16, row-major) on their way into LDS with the chunk swizzle:
 // load() issues every global load of the calling thread, store() writes them, so the copy
 // costs one memory round trip (a loop that stores each chunk before loading the next pays
 // one per iteration). Work is spread over T threads (the workgroup size); `src(row)` gives
 // the row's source, or nullptr for a row of zeros; `permuted` reorders each row's input
 // channels to kperm order.
-template <int ROWS, int T> struct WeightStage {
-  static constexpr int N = (ROWS * 16 + T - 1) / T;   // chunks per thread
+template <int ROWS, int T, int CC = C> struct WeightStage {
+  static constexpr int CPR = CC / 8;                  // 16-byte chunks per row
+  static constexpr int SWZ = swizzle_mask(CC);
+  static constexpr int N = (ROWS * CPR + T - 1) / T;  // chunks per thread
   bf16x8 v[N];
   template <class Src> __device__ __forceinline__ void load(Src src, bool permuted) {
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       const int i = int(threadIdx.x) + j * T;
       v[j] = bf16x8{};
-      if (i >= ROWS * 16) continue;
-      const int n = i >> 4, c = i & 15;             // row, logical chunk
+      if (i >= ROWS * CPR) continue;
+      const int n = i / CPR, c = i % CPR;           // row, logical chunk
       const bf16 *w = src(n);
       if (!w) continue;
       if (permuted) {
@@ -67,36 +73,38 @@ template <int ROWS, int T> struct WeightStage {
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       const int i = int(threadIdx.x) + j * T;
-      if (i >= ROWS * 16) continue;
-      const int n = i >> 4, c = i & 15;
-      *reinterpret_cast<bf16x8 *>(dst + n * C + ((c ^ (n & 15)) * 8)) = v[j];
+      if (i >= ROWS * CPR) continue;
+      const int n = i / CPR, c = i % CPR;
+      *reinterpret_cast<bf16x8 *>(dst + n * CC + ((c ^ (n & SWZ)) * 8)) = v[j];
     }
   }
 };
 
 // Fragment of W for output tile t, k-step ks (lane: row 16 t + l % 16, chunk 4 ks + g):
 // the A operand of out^T = W . x^T, or the B operand of out = x . W^T (same lane layout).
-__device__ __forceinline__ bf16x8 weight_frag(const bf16 *w_lds, int t, int ks) {
+template <int CC = C> __device__ __forceinline__ bf16x8 weight_frag(const bf16 *w_lds, int t, int ks) {
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int n = 16 * t + r;
-  return *reinterpret_cast<const bf16x8 *>(w_lds + n * C + (((4 * ks + g) ^ r) * 8));
+  return *reinterpret_cast<const bf16x8 *>(w_lds + n * CC + (((4 * ks + g) ^ (r & swizzle_mask(CC))) * 8));
 }
 
 // out^T tiles: acc[t] (+)= sum_ks W(t, ks) . x[ks]; x is a K-layout (or, with a permuted W,
 // an O-layout) bf16 operand.
-__device__ __forceinline__ void gemm_t(const bf16 *w_lds, const bf16x8 (&x)[4], f32x4 (&acc)[8]) {
+template <int KS, int NT>
+__device__ __forceinline__ void gemm_t(const bf16 *w_lds, const bf16x8 (&x)[KS], f32x4 (&acc)[NT]) {
 #pragma unroll
-  for (int t = 0; t < 8; ++t)
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) acc[t] = mfma16(weight_frag(w_lds, t, ks), x[ks], acc[t]);
+    for (int ks = 0; ks < KS; ++ks) acc[t] = mfma16(weight_frag<32 * KS>(w_lds, t, ks), x[ks], acc[t]);
 }
 
 // out tile: acc (+)= sum_ks x[ks] . W(t, ks) — rows are positions, columns the 16 output
 // channels of tile t; a lane ends up with 4 consecutive positions (4 g .. +3) of channel
 // 16 t + l % 16.
-__device__ __forceinline__ void gemm_n(const bf16 *w_lds, int t, const bf16x8 (&x)[4], f32x4 &acc) {
+template <int KS>
+__device__ __forceinline__ void gemm_n(const bf16 *w_lds, int t, const bf16x8 (&x)[KS], f32x4 &acc) {
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) acc = mfma16(x[ks], weight_frag(w_lds, t, ks), acc);
+  for (int ks = 0; ks < KS; ++ks) acc = mfma16(x[ks], weight_frag<32 * KS>(w_lds, t, ks), acc);
 }
 
 // Sum over the four lanes of one position (l, l ^ 16, l ^ 32, l ^ 48). The swap results
@@ -115,19 +123,20 @@ __device__ __forceinline__ float position_sum(float x) {
   return __builtin_bit_cast(float, q0) + __builtin_bit_cast(float, q1);
 }
 
-// LayerNorm statistics of a position from this lane's 32 channels (fp32, two passes).
-__device__ __forceinline__ void ln_stats(const float (&v)[32], float eps, float &mean, float &rstd) {
+// LayerNorm statistics of a position from this lane's V = CC / 4 channels (fp32, two passes).
+template <int V>
+__device__ __forceinline__ void ln_stats(const float (&v)[V], float eps, float &mean, float &rstd) {
   float s = 0.f;
 #pragma unroll
-  for (int i = 0; i < 32; ++i) s += v[i];
-  mean = position_sum(s) * (1.0f / C);
+  for (int i = 0; i < V; ++i) s += v[i];
+  mean = position_sum(s) * (1.0f / (4 * V));
   float q = 0.f;
 #pragma unroll
-  for (int i = 0; i < 32; ++i) {
+  for (int i = 0; i < V; ++i) {
     const float d = v[i] - mean;
     q += d * d;
   }
-  rstd = rsqrtf(position_sum(q) * (1.0f / C) + eps);
+  rstd = rsqrtf(position_sum(q) * (1.0f / (4 * V)) + eps);
 }
 
 // Loads 8 consecutive channels of a row as floats.
@@ -178,35 +187,36 @@ template <> struct Raw4<float> {
 };
 
 // K-layout row as loaded: r[2 ks + h] = channels 32 ks + 8 g + 4 h .. +3.
-template <typename T> __device__ __forceinline__ void load_k(const T *row, Raw4<T> (&r)[8]) {
+template <typename T, int R> __device__ __forceinline__ void load_k(const T *row, Raw4<T> (&r)[R]) {
   const int g = (threadIdx.x & 63) >> 4;
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
+  for (int ks = 0; ks < R / 2; ++ks) {
     r[2 * ks].load(row + 32 * ks + 8 * g);
     r[2 * ks + 1].load(row + 32 * ks + 8 * g + 4);
   }
 }
-template <typename T> __device__ __forceinline__ void k_to_float(const Raw4<T> (&r)[8], float (&v)[32]) {
+template <typename T, int R> __device__ __forceinline__ void k_to_float(const Raw4<T> (&r)[R], float (&v)[4 * R]) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < R; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[4 * i + e] = r[i][e];
 }
 // O-layout row as loaded: r[t] = channels 16 t + 4 g .. +3.
-template <typename T> __device__ __forceinline__ void load_o(const T *row, Raw4<T> (&r)[8]) {
+template <typename T, int R> __device__ __forceinline__ void load_o(const T *row, Raw4<T> (&r)[R]) {
   const int g = (threadIdx.x & 63) >> 4;
 #pragma unroll
-  for (int t = 0; t < 8; ++t) r[t].load(row + 16 * t + 4 * g);
+  for (int t = 0; t < R; ++t) r[t].load(row + 16 * t + 4 * g);
 }
 
 // LayerNorm of a K-layout position (affine parameters from LDS, fp32) to bf16 operands.
-__device__ __forceinline__ void ln_k(float (&v)[32], const float *lnw, const float *lnb, float eps,
-                                     bf16x8 (&x)[4]) {
+template <int KS>
+__device__ __forceinline__ void ln_k(float (&v)[8 * KS], const float *lnw, const float *lnb, float eps,
+                                     bf16x8 (&x)[KS]) {
   const int g = (threadIdx.x & 63) >> 4;
   float mean, rstd;
   ln_stats(v, eps, mean, rstd);
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
+  for (int ks = 0; ks < KS; ++ks) {
     const float4 w0 = *reinterpret_cast<const float4 *>(lnw + 32 * ks + 8 * g);
     const float4 w1 = *reinterpret_cast<const float4 *>(lnw + 32 * ks + 8 * g + 4);
     const float4 b0 = *reinterpret_cast<const float4 *>(lnb + 32 * ks + 8 * g);
@@ -219,25 +229,26 @@ __device__ __forceinline__ void ln_k(float (&v)[32], const float *lnw, const flo
 }
 
 // Optional LayerNorm affine parameters (fp32[128], nullptr: 1 / 0) on their way into LDS,
-// split like WeightStage; the workgroup has at least 128 threads.
-struct LnStage {
+// split like WeightStage; the workgroup has at least CC threads.
+template <int CC> struct LnStageOf {
   float w, b;
   __device__ __forceinline__ void load(const float *wp, const float *bp) {
     const int i = int(threadIdx.x);
     w = 1.f;
     b = 0.f;
-    if (i < C) {
+    if (i < CC) {
       if (wp) w = wp[i];
       if (bp) b = bp[i];
     }
   }
   __device__ __forceinline__ void store(float *w_lds, float *b_lds) const {
-    if (threadIdx.x < C) {
+    if (threadIdx.x < CC) {
       w_lds[threadIdx.x] = w;
       b_lds[threadIdx.x] = b;
     }
   }
 };
+using LnStage = LnStageOf<C>;
 
 // Identity fragments: as the A operand with a K-layout operand x[ks] as B, half h
 // (0 or 1) gives O-layout tile t = 2 ks + h exactly (one nonzero product per output), so
@@ -249,17 +260,19 @@ __device__ __forceinline__ void identity_frags(bf16x8 (&id)[2]) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) id[h][j] = (8 * g + j == m + 16 * h) ? bf16(1.0f) : bf16(0.0f);
 }
-__device__ __forceinline__ void k_to_o(const bf16x8 (&id)[2], const bf16x8 (&x)[4], f32x4 (&o)[8]) {
+template <int KS>
+__device__ __forceinline__ void k_to_o(const bf16x8 (&id)[2], const bf16x8 (&x)[KS], f32x4 (&o)[2 * KS]) {
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
+  for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
     for (int h = 0; h < 2; ++h) o[2 * ks + h] = mfma16(id[h], x[ks], f32x4{0.f, 0.f, 0.f, 0.f});
 }
 
 // Pairs the O-layout values of tiles 2 ks and 2 ks + 1 into k-operand ks (kperm order).
-__device__ __forceinline__ void o_to_operand(const float (&y)[8][4], bf16x8 (&x)[4]) {
+template <int KS>
+__device__ __forceinline__ void o_to_operand(const float (&y)[2 * KS][4], bf16x8 (&x)[KS]) {
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
+  for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       x[ks][e] = bf16(y[2 * ks][e]);

@@ -1,4 +1,4 @@
-// Fused triangle-multiplication kernels (bf16 compute, c = 128), around the per-channel
+// Fused triangle-multiplication kernels (bf16 compute, c = 128 or 64), around the per-channel
 // contraction (xfold/nn/triangle_multiplication.py:71-105):
 //
 //   trimul_project: LN_in(z) -> [projection | gate] (one GEMM over both weights' rows) ->
@@ -36,10 +36,12 @@ using namespace panel;
 // lines x of one row group and the 32 positions of a k-slice of all channels form one block.
 // RT = 1 (row m = position y0 + m, 8-byte stores) halves the unit for grids too small to
 // give every wavefront several 32-position units.
-constexpr int PROJ = 2 * K;          // projection (and gate) output channels
+// At c = 64 the weights take 32 KB and a row half the registers: two workgroups per CU.
+constexpr int wgs_per_cu(int k) { return k == 64 ? 2 : 1; }
 
-template <typename TIN, int RT>
-__global__ __launch_bounds__(512, 1) void trimul_project_kernel(TriProjectArgs a) {
+template <typename TIN, int RT, int K>
+__global__ __launch_bounds__(512, wgs_per_cu(K)) void trimul_project_kernel(TriProjectArgs a) {
+  constexpr int PROJ = 2 * K, KS = K / 32;          // projection (and gate) output channels, k-steps
   constexpr int UP = 16 * RT;                       // positions per unit
   // Position offset (in the unit) of row m of row tile rt, and of output element i < 4 RT
   // of a lane in channel-tile group g.
@@ -47,8 +49,8 @@ __global__ __launch_bounds__(512, 1) void trimul_project_kernel(TriProjectArgs a
   __shared__ __attribute__((aligned(16))) bf16 w_proj[PROJ * K];
   __shared__ __attribute__((aligned(16))) bf16 w_gate[PROJ * K];
   __shared__ __attribute__((aligned(16))) float lnw[K], lnb[K];
-  rowstep::WeightStage<PROJ, 512> sp, sg;
-  rowstep::LnStage sl;
+  rowstep::WeightStage<PROJ, 512, K> sp, sg;
+  rowstep::LnStageOf<K> sl;
   sp.load([&](int row) { return a.w_proj + row * K; }, false);
   sg.load([&](int row) { return a.w_gate + row * K; }, false);
   sl.load(a.ln_w, a.ln_b);
@@ -65,7 +67,7 @@ __global__ __launch_bounds__(512, 1) void trimul_project_kernel(TriProjectArgs a
   auto pos_of = [&](int x, int y) -> int64_t { return a.outgoing ? int64_t(x) * n + y : int64_t(y) * n + x; };
 
   struct Unit {
-    rowstep::Raw4<TIN> z[RT][8];                    // K-layout rows of the row tiles
+    rowstep::Raw4<TIN> z[RT][K / 16];                    // K-layout rows of the row tiles
     float mrow[RT];                                 // mask of those rows (0 for y >= n)
   };
   auto fetch = [&](int u, Unit &w) {
@@ -88,10 +90,10 @@ __global__ __launch_bounds__(512, 1) void trimul_project_kernel(TriProjectArgs a
   for (; u < units; u += waves) {
     Unit next;
     if (u + waves < units) fetch(u + waves, next);
-    bf16x8 xa[RT][4];
+    bf16x8 xa[RT][KS];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      float v[32];
+      float v[K / 4];
       rowstep::k_to_float(cur.z[rt], v);
       rowstep::ln_k(v, lnw, lnb, a.eps, xa[rt]);
     }
@@ -112,8 +114,8 @@ __global__ __launch_bounds__(512, 1) void trimul_project_kernel(TriProjectArgs a
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) ap[rt] = ag[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const bf16x8 wp = rowstep::weight_frag(w_proj, t, ks), wg = rowstep::weight_frag(w_gate, t, ks);
+      for (int ks = 0; ks < KS; ++ks) {
+        const bf16x8 wp = rowstep::weight_frag<K>(w_proj, t, ks), wg = rowstep::weight_frag<K>(w_gate, t, ks);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           ap[rt] = mfma16(xa[rt][ks], wp, ap[rt]);
@@ -149,13 +151,14 @@ __global__ __launch_bounds__(512, 1) void trimul_project_kernel(TriProjectArgs a
 //   y      = bf16(LN_c(c))                    (statistics over the 4 lanes of a position)
 //   u^T    = Wout . y^T                       (Wout in kperm order)
 //   z     += bf16(u * sigmoid(gate))
-template <typename TIN, typename TOUT>
-__global__ __launch_bounds__(512, 1) void trimul_output_kernel(TriOutputArgs a) {
-  __shared__ __attribute__((aligned(16))) bf16 w_gate[rowstep::W_ELEMS];
-  __shared__ __attribute__((aligned(16))) bf16 w_out[rowstep::W_ELEMS];
+template <typename TIN, typename TOUT, int K>
+__global__ __launch_bounds__(512, wgs_per_cu(K)) void trimul_output_kernel(TriOutputArgs a) {
+  constexpr int KS = K / 32, NT = K / 16;
+  __shared__ __attribute__((aligned(16))) bf16 w_gate[K * K];
+  __shared__ __attribute__((aligned(16))) bf16 w_out[K * K];
   __shared__ __attribute__((aligned(16))) float lnw_in[K], lnb_in[K], lnw_c[K], lnb_c[K];
-  rowstep::WeightStage<K, 512> sg, so;
-  rowstep::LnStage sl_in, sl_c;
+  rowstep::WeightStage<K, 512, K> sg, so;
+  rowstep::LnStageOf<K> sl_in, sl_c;
   sg.load([&](int row) { return a.w_gating + row * K; }, false);
   so.load([&](int row) { return a.w_out + row * K; }, true);
   sl_in.load(a.ln_in_w, a.ln_in_b);
@@ -176,19 +179,19 @@ __global__ __launch_bounds__(512, 1) void trimul_output_kernel(TriOutputArgs a) 
   rowstep::identity_frags(id);
 
   struct Rows {
-    rowstep::Raw4<TIN> z[8];                       // K-layout
-    bf16x8 c[4];                                   // see fetch
-    rowstep::Raw4<TOUT> res[8];                    // O-layout (only when not derived from z)
+    rowstep::Raw4<TIN> z[NT];                       // K-layout
+    bf16x8 c[KS];                                  // see fetch
+    rowstep::Raw4<TOUT> res[NT];                    // O-layout (only when not derived from z)
   };
   auto fetch = [&](int st, Rows &rw) {
     const int i = st / row_blocks, j = (st - i * row_blocks) * 16 + r;
     const int64_t pc = int64_t(i) * n + (j < n ? j : n - 1);
     rowstep::load_k<TIN>(z + pc * K, rw.z);
-    // c[q]: channel 16 q + r (g < 2) or 16 (q + 4) + r (g >= 2), positions 8 (g % 2) .. +7
-    // of the step: k = 8 g + j of an A fragment whose k-halves hold tiles q and q + 4.
-    const bf16 *src = a.contracted + st * res_block_stride(K) + (64 * (g >> 1) + r) * 16 + 8 * (g & 1);
+    // c[q]: channel 16 q + r (g < 2) or 16 (q + KS) + r (g >= 2), positions 8 (g % 2) .. +7
+    // of the step: k = 8 g + j of an A fragment whose k-halves hold tiles q and q + KS.
+    const bf16 *src = a.contracted + st * res_block_stride(K) + (K / 2 * (g >> 1) + r) * 16 + 8 * (g & 1);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) rw.c[q] = *reinterpret_cast<const bf16x8 *>(src + q * 256);
+    for (int q = 0; q < KS; ++q) rw.c[q] = *reinterpret_cast<const bf16x8 *>(src + q * 256);
     if (res_load) rowstep::load_o<TOUT>(out + pc * K, rw.res);
   };
 
@@ -204,40 +207,40 @@ __global__ __launch_bounds__(512, 1) void trimul_output_kernel(TriOutputArgs a) 
     Rows next;
     if (st + waves < steps) fetch(st + waves, next);
     // gate = sigmoid(Wg . LN_in(z))
-    float sig[8][4];
+    float sig[NT][4];
     {
-      bf16x8 x[4];
-      float v[32];
+      bf16x8 x[KS];
+      float v[K / 4];
       rowstep::k_to_float(cur.z, v);
       rowstep::ln_k(v, lnw_in, lnb_in, a.eps_in, x);
-      f32x4 acc[8];
+      f32x4 acc[NT];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
       rowstep::gemm_t(w_gate, x, acc);
 #pragma unroll
-      for (int t = 0; t < 8; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) sig[t][e] = sigmoidf_(acc[t][e]);
     }
     // y = LN_c(c), O-layout
-    bf16x8 y[4];
+    bf16x8 y[KS];
     {
-      f32x4 co[8];
+      f32x4 co[NT];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q < KS; ++q) {
         co[q] = mfma16(cur.c[q], id[0], f32x4{0.f, 0.f, 0.f, 0.f});
-        co[q + 4] = mfma16(cur.c[q], id[1], f32x4{0.f, 0.f, 0.f, 0.f});
+        co[q + KS] = mfma16(cur.c[q], id[1], f32x4{0.f, 0.f, 0.f, 0.f});
       }
-      float v[32];
+      float v[K / 4];
 #pragma unroll
-      for (int t = 0; t < 8; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[4 * t + e] = co[t][e];
       float mean, rstd;
       rowstep::ln_stats(v, a.eps_c, mean, rstd);
-      float yo[8][4];
+      float yo[NT][4];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
+      for (int t = 0; t < NT; ++t) {
         const float4 w = *reinterpret_cast<const float4 *>(lnw_c + 16 * t + 4 * g);
         const float4 b = *reinterpret_cast<const float4 *>(lnb_c + 16 * t + 4 * g);
         const float wv[4] = {w.x, w.y, w.z, w.w}, bv[4] = {b.x, b.y, b.z, b.w};
@@ -246,16 +249,16 @@ __global__ __launch_bounds__(512, 1) void trimul_output_kernel(TriOutputArgs a) 
       }
       rowstep::o_to_operand(yo, y);
     }
-    f32x4 acc[8];
+    f32x4 acc[NT];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     rowstep::gemm_t(w_out, y, acc);
-    f32x4 res[8];
+    f32x4 res[NT];
     if (res_from_z) {
       if constexpr (kBf16) {
-        bf16x8 zk[4];
+        bf16x8 zk[KS];
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             zk[ks][e] = cur.z[2 * ks].v[e];
@@ -265,7 +268,7 @@ __global__ __launch_bounds__(512, 1) void trimul_output_kernel(TriOutputArgs a) 
       }
     } else {
 #pragma unroll
-      for (int t = 0; t < 8; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) res[t][e] = res_load ? cur.res[t][e] : 0.f;
     }
@@ -273,7 +276,7 @@ __global__ __launch_bounds__(512, 1) void trimul_output_kernel(TriOutputArgs a) 
     if (j < n) {
       const int64_t pos = int64_t(i) * n + j;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
+      for (int t = 0; t < NT; ++t) {
         float o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = res[t][e] + static_cast<float>(bf16(acc[t][e] * sig[t][e]));
@@ -286,13 +289,13 @@ __global__ __launch_bounds__(512, 1) void trimul_output_kernel(TriOutputArgs a) 
 
 }  // namespace
 
-int trimul_project(const TriProjectArgs &a, int pair_dtype, hipStream_t s) {
-  if (a.ld != contraction_ld(a.n)) return fail(XFH_EINVAL, "trimul_project: ld must be contraction_ld(n)");
+template <int K> static int launch_project(const TriProjectArgs &a, int pair_dtype, hipStream_t s) {
   int cus = 0;
   XFH_TRY(device_cu_count(&cus));
+  cus *= wgs_per_cu(K);
   // 32-position units take 1.75 times a 16-position unit's time (the weight fragments are read
   // once for both row tiles), so they win unless 16-position units need few enough more
-  // rounds: n = 509 59.3 us (32) against 69.2 (16), 900 168 / 301, 256 18.3 / 18.8; 160 19.8 / 16.3,
+  // rounds (c = 128): n = 509 59.3 us (32) against 69.2 (16), 900 168 / 301, 256 18.3 / 18.8; 160 19.8 / 16.3,
   // 384 37.3 / 35.5.
   const int64_t units32 = int64_t(a.n) * (a.ld / 32);
   const int64_t slots = int64_t(cus) * 8;
@@ -301,30 +304,40 @@ int trimul_project(const TriProjectArgs &a, int pair_dtype, hipStream_t s) {
   const dim3 grid(unsigned(balanced_grid(units, 8, cus)));
   KernelTimer timer("trimul_project", s, 0.0, true);
   if (pair_dtype == XFH_BF16) {
-    if (wide) timer.launch(trimul_project_kernel<bf16, 2>, dim3(grid), dim3(512), 0, a);
-    else timer.launch(trimul_project_kernel<bf16, 1>, dim3(grid), dim3(512), 0, a);
+    if (wide) timer.launch(trimul_project_kernel<bf16, 2, K>, dim3(grid), dim3(512), 0, a);
+    else timer.launch(trimul_project_kernel<bf16, 1, K>, dim3(grid), dim3(512), 0, a);
   } else {
-    if (wide) timer.launch(trimul_project_kernel<float, 2>, dim3(grid), dim3(512), 0, a);
-    else timer.launch(trimul_project_kernel<float, 1>, dim3(grid), dim3(512), 0, a);
+    if (wide) timer.launch(trimul_project_kernel<float, 2, K>, dim3(grid), dim3(512), 0, a);
+    else timer.launch(trimul_project_kernel<float, 1, K>, dim3(grid), dim3(512), 0, a);
   }
   return check_launch("trimul_project");
 }
 
-int trimul_output(const TriOutputArgs &a, int pair_dtype, int out_dtype, hipStream_t s) {
+template <int K>
+static int launch_output(const TriOutputArgs &a, int pair_dtype, int out_dtype, hipStream_t s) {
   const int64_t steps = int64_t(a.n) * res_row_blocks(a.n);
   int cus = 0;
   XFH_TRY(device_cu_count(&cus));
-  const dim3 grid(unsigned(balanced_grid(steps, 8, cus)));
+  const dim3 grid(unsigned(balanced_grid(steps, 8, cus * wgs_per_cu(K))));
   KernelTimer timer("trimul_output", s, 0.0, true);
   if (pair_dtype == XFH_BF16 && out_dtype == XFH_BF16)
-    timer.launch(trimul_output_kernel<bf16, bf16>, dim3(grid), dim3(512), 0, a);
+    timer.launch(trimul_output_kernel<bf16, bf16, K>, dim3(grid), dim3(512), 0, a);
   else if (pair_dtype == XFH_BF16 && out_dtype == XFH_F32)
-    timer.launch(trimul_output_kernel<bf16, float>, dim3(grid), dim3(512), 0, a);
+    timer.launch(trimul_output_kernel<bf16, float, K>, dim3(grid), dim3(512), 0, a);
   else if (pair_dtype == XFH_F32 && out_dtype == XFH_F32)
-    timer.launch(trimul_output_kernel<float, float>, dim3(grid), dim3(512), 0, a);
+    timer.launch(trimul_output_kernel<float, float, K>, dim3(grid), dim3(512), 0, a);
   else
-    timer.launch(trimul_output_kernel<float, bf16>, dim3(grid), dim3(512), 0, a);
+    timer.launch(trimul_output_kernel<float, bf16, K>, dim3(grid), dim3(512), 0, a);
   return check_launch("trimul_output");
+}
+
+int trimul_project(const TriProjectArgs &a, int pair_dtype, hipStream_t s) {
+  if (a.ld != contraction_ld(a.n)) return fail(XFH_EINVAL, "trimul_project: ld must be contraction_ld(n)");
+  return a.c == 64 ? launch_project<64>(a, pair_dtype, s) : launch_project<128>(a, pair_dtype, s);
+}
+
+int trimul_output(const TriOutputArgs &a, int pair_dtype, int out_dtype, hipStream_t s) {
+  return a.c == 64 ? launch_output<64>(a, pair_dtype, out_dtype, s) : launch_output<128>(a, pair_dtype, out_dtype, s);
 }
 
 }  // namespace xfh
