@@ -122,6 +122,28 @@ def test_msa_attention_mask_values(device, kind, c_pair):
     assert_parity(got, want, TOL_FP32, f"msa_attention {kind} mask")
 
 
+@pytest.mark.parametrize("rows,n", [(1, 1), (17, 65), (32, 31), (16, 64)])
+def test_msa_operators_fp32_rows_and_unaligned(device, rows, n):
+    """64 MSA channels in bf16 compute around the 16-sequence and 32-position units, from fp32 rows and
+    from bf16 rows that are not 16-byte aligned (the general kernels)."""
+    announce("msa units", rows, n)
+    torch.manual_seed(rows + n)
+    msa, pair = torch.randn(rows, n, 64).bfloat16(), torch.randn(n, n, 128).bfloat16()
+    mask = msa_mask(rows, n, seed=n, kind="fractional") if rows > 1 else torch.ones(rows, n)
+    odd = torch.zeros(msa.numel() + 1, dtype=torch.bfloat16, device=device)[1:].view(msa.shape)
+    odd.copy_(msa)
+    d = [t.to(device) for t in (mask, pair)]
+    for name, args, extra in (("MSAAttention", dict(c_msa=64, c_pair=128, num_head=8), (mask, pair.float())),
+                              ("OuterProductMean", dict(c_msa=64, num_output_channel=128, num_outer_channel=32), (mask,))):
+        ref, hip = pair_of(name, args, seed=n)
+        with torch.no_grad():
+            want = ref(msa.float(), *extra)
+        floor = bf16_stored(floor_of(lambda: ref(msa.float(), *extra)))
+        with torch.inference_mode(), autocast(True):
+            for x in (msa.float().to(device), odd):
+                assert_parity_bf16(hip(x, *d[:len(extra)]), want, f"{name} {x.dtype}", floor=floor)
+
+
 def test_msa_attention_fully_masked(device):
     """Every key masked: the reference's logits all get -1e9 and the softmax is uniform
     over the keys (fp32 cannot hold the -1e9-shifted logits' differences)."""

@@ -10,7 +10,10 @@
 //     1e9 (max_s mask[s,k] - 1) (msa_key_term_kernel, msa_softmax_kernel), shared by every
 //     MSA row -> v^T per head (GEMM) -> weights x v per head (GEMM over keys) -> rows back to
 //     [s][q][h, c] (msa_gather_kernel) -> sigmoid(gating) x (GEMM epilogue) -> output GEMM.
+// At 64 MSA channels in bf16 (32 outer channels) the steps around those GEMMs are msa_fused.hip's.
+#include <algorithm>
 #include <cstring>
+#include <initializer_list>
 #include <string>
 
 #include "common.h"
@@ -158,9 +161,28 @@ struct MsaPlan {
   float *kt;
 };
 
+// The fused kernels' shapes (msa_fused.hip): 64 MSA channels in bf16, 16-byte aligned operands.
+bool fused_width(int64_t c_msa, int dtype) { return dtype == XFH_BF16 && c_msa == 64; }
+bool aligned16(std::initializer_list<const void *> ptrs) {
+  for (const void *p : ptrs)
+    if (reinterpret_cast<uintptr_t>(p) % 16) return false;
+  return true;
+}
+
 int64_t msa_carve(Carver &cv, MsaPlan &p, int64_t rows, int64_t n, int64_t c_msa, int64_t c_pair, int64_t heads,
-                  int dtype, bool packed) {
+                  int dtype, bool packed, bool fused) {
   const int64_t es = esize(dtype), npad = align_up(n, int64_t(64));
+  if (fused) {
+    const int64_t rpad = align_up(rows, int64_t(16));
+    std::memset(&p, 0, sizeof(p));
+    p.pair_normed = packed ? nullptr : cv.take(n * n * c_pair * es);
+    p.logits = packed ? cv.take(heads * n * npad * 4) : cv.take(n * n * heads * es);
+    p.kt = static_cast<float *>(cv.take(npad * 4));
+    p.weights = cv.take(heads * n * npad * es);
+    p.vt = cv.take(rpad * npad * c_msa * es);
+    p.avg_t = cv.take(rpad * n * c_msa * es);
+    return cv.used;
+  }
   p.normed = cv.take(rows * n * c_msa * es);
   p.pair_normed = packed ? nullptr : cv.take(n * n * c_pair * es);
   p.logits = packed ? cv.take(heads * n * npad * 4) : cv.take(n * n * heads * es);
@@ -215,13 +237,26 @@ int xfh_outer_product_mean(const void *msa, int msa_dtype, const void *mask, int
     return fail(XFH_EWORKSPACE, "outer_product_mean: workspace too small (need " + std::to_string(need) + " bytes)");
   hipStream_t s = as_stream(stream);
   const int64_t spad = align_up(rows, int64_t(kOpmTile)), co = c_outer;
-  XFH_TRY(layer_norm_rows(msa, msa_dtype, rows * n, c_msa, ln_w, ln_b, ln_eps, p.normed, dtype, s));
-  {
+  const bool fused = fused_width(c_msa, dtype) && co == 32 && aligned16({msa, proj_w});
+  if (fused) {
+    MsaProjectArgs pa;
+    std::memset(&pa, 0, sizeof(pa));
+    pa.x = msa; pa.mask = mask; pa.mask_dtype = mask_dtype; pa.ln_w = ln_w; pa.ln_b = ln_b; pa.eps = ln_eps;
+    pa.w = static_cast<const bf16 *>(proj_w);
+    pa.lines = pa.lines_pad = int(n); pa.t_len = int(rows); pa.t_pad = int(spad);
+    pa.line_rows = 1; pa.t_rows = n;
+    pa.out0 = static_cast<bf16 *>(p.lt); pa.out1 = static_cast<bf16 *>(p.rt); pa.split = 32;
+    pa.ch_stride = spad; pa.line_stride = 32 * spad;
+    pa.mask_out = static_cast<bf16 *>(p.mt);
+    XFH_TRY(msa_project(pa, msa_dtype, s));
+  }
+  if (!fused) XFH_TRY(layer_norm_rows(msa, msa_dtype, rows * n, c_msa, ln_w, ln_b, ln_eps, p.normed, dtype, s));
+  if (!fused) {
     GemmArgs g = plain_gemm(p.normed, c_msa, proj_w, c_msa, p.lr, 2 * co, rows * n, 2 * co, c_msa);
     XFH_TRY(gemm_nt(g, 1, dtype, dtype, false, s));
   }
   const dim3 grid(unsigned(spad / kOpmTile), unsigned(n));
-  {
+  if (!fused) {
     if (dtype == XFH_BF16)
       opm_operands_kernel<bf16><<<grid, 256, 0, s>>>(static_cast<const bf16 *>(p.lr), mask, mask_dtype, int(rows),
                                                       int(n), int(co), int(spad), static_cast<bf16 *>(p.lt),
@@ -253,9 +288,14 @@ int xfh_outer_product_mean(const void *msa, int msa_dtype, const void *mask, int
 int64_t xfh_msa_attention_workspace_size(int64_t rows, int64_t n, int64_t c_msa, int64_t c_pair, int64_t heads,
                                          int dtype) {
   if (rows < 0 || n < 0 || c_msa < 0 || c_pair < 0 || heads <= 0 || !fdtype(dtype)) return -1;
-  Carver cv(nullptr, 0);
-  MsaPlan p;
-  return msa_carve(cv, p, rows, n, c_msa, c_pair, heads, dtype, msa_packed_logits(n, c_pair, heads, dtype)) + 256;
+  int64_t most = 0;                                  // (unaligned operands at 64 channels: the general path)
+  for (int fused = 0; fused <= (fused_width(c_msa, dtype) ? 1 : 0); ++fused) {
+    Carver cv(nullptr, 0);
+    MsaPlan p;
+    most = std::max(most, msa_carve(cv, p, rows, n, c_msa, c_pair, heads, dtype,
+                                    msa_packed_logits(n, c_pair, heads, dtype), fused != 0));
+  }
+  return most + 256;
 }
 
 int xfh_msa_attention(const void *msa, int msa_dtype, const void *mask, int mask_dtype, const void *pair,
@@ -279,12 +319,13 @@ int xfh_msa_attention(const void *msa, int msa_dtype, const void *mask, int mask
   const bool packed = msa_packed_logits(n, c_pair, heads, dtype);
   Carver cv(workspace, workspace_bytes);
   MsaPlan p;
-  const int64_t need = msa_carve(cv, p, rows, n, c_msa, c_pair, heads, dtype, packed);
+  const bool fused = fused_width(c_msa, dtype) && aligned16({msa, out, v_w, gating_w, out_w});
+  const int64_t need = msa_carve(cv, p, rows, n, c_msa, c_pair, heads, dtype, packed, fused);
   if (!workspace || need > workspace_bytes)
     return fail(XFH_EWORKSPACE, "msa_attention: workspace too small (need " + std::to_string(need) + " bytes)");
   hipStream_t s = as_stream(stream);
   const int64_t npad = align_up(n, int64_t(64));
-  XFH_TRY(layer_norm_rows(msa, msa_dtype, rows * n, c_msa, ln_w, ln_b, ln_eps, p.normed, dtype, s));
+  if (!fused) XFH_TRY(layer_norm_rows(msa, msa_dtype, rows * n, c_msa, ln_w, ln_b, ln_eps, p.normed, dtype, s));
   // logits(h, q, k) = Linear(LN(pair))[q][k][h]
   int logit_dtype;
   int64_t sh, sq, sk;
@@ -316,10 +357,30 @@ int xfh_msa_attention(const void *msa, int msa_dtype, const void *mask, int mask
     msa_softmax_kernel<float><<<sgrid, 256, 0, s>>>(p.logits, logit_dtype, sh, sq, sk, scale, p.kt, int(heads),
                                                     int(n), int(npad), static_cast<float *>(p.weights));
   XFH_TRY(check_launch("msa_softmax"));
-  // vt[h][c][s n + k] = v_w[h dv + c] . LN(msa)[s][k]
-  GemmArgs g = plain_gemm(v_w, c_msa, p.normed, c_msa, p.vt, rows * n, dv, rows * n, c_msa);
-  g.sA = dv * c_msa; g.sB = 0; g.sC = dv * rows * n;
-  XFH_TRY(gemm_nt(g, heads, dtype, dtype, false, s));
+  if (fused) {
+    // vt[h][c][s][k] = v_w[h dv + c] . LN(msa)[s][k], key rows padded to npad and sequences to rpad
+    // (zeros), so every n runs the pipelined GEMM; then avg_t[h][q][c][s] and the fused tail.
+    const int64_t rpad = align_up(rows, int64_t(16));
+    MsaProjectArgs pa;
+    std::memset(&pa, 0, sizeof(pa));
+    pa.x = msa; pa.ln_w = ln_w; pa.ln_b = ln_b; pa.eps = ln_eps; pa.w = static_cast<const bf16 *>(v_w);
+    pa.lines = int(rows); pa.lines_pad = int(rpad); pa.t_len = int(n); pa.t_pad = int(npad);
+    pa.line_rows = n; pa.t_rows = 1;
+    pa.out0 = static_cast<bf16 *>(p.vt); pa.split = 64;
+    pa.ch_stride = rpad * npad; pa.line_stride = npad;
+    XFH_TRY(msa_project(pa, msa_dtype, s));
+    GemmArgs g = plain_gemm(p.weights, npad, p.vt, npad, p.avg_t, dv * rpad, n, dv * rpad, npad);
+    g.sA = n * npad; g.sB = dv * rpad * npad; g.sC = n * dv * rpad;
+    XFH_TRY(gemm_nt(g, heads, dtype, dtype, false, s));
+    MsaOutputArgs oa;
+    oa.x = msa; oa.avg_t = static_cast<const bf16 *>(p.avg_t); oa.ln_w = ln_w; oa.ln_b = ln_b; oa.eps = ln_eps;
+    oa.w_gating = static_cast<const bf16 *>(gating_w); oa.w_out = static_cast<const bf16 *>(out_w);
+    oa.out = out; oa.accumulate = accumulate; oa.rows = int(rows); oa.rows_pad = int(rpad); oa.n = int(n); oa.dv = int(dv);
+    return msa_output(oa, msa_dtype, out_dtype, s);
+  }
+  // vt[h][c][s n + k] = v_w[h dv + c] . LN(msa)[s][k] (all heads' rows in one product)
+  GemmArgs g = plain_gemm(v_w, c_msa, p.normed, c_msa, p.vt, rows * n, c_msa, rows * n, c_msa);
+  XFH_TRY(gemm_nt(g, 1, dtype, dtype, false, s));
   // avg_t[h][q][c rows + s] = sum_k weights[h][q][k] vt[h][c][s n + k]
   g = plain_gemm(p.weights, npad, p.vt, n, p.avg_t, dv * rows, n, dv * rows, n);
   g.sA = n * npad; g.sB = dv * rows * n; g.sC = n * dv * rows;
