@@ -861,6 +861,30 @@ def test_gemm_direct(device, m, k, n, kind):
     assert_parity_bf16(got, want, f"gemm_direct {kind} {m}x{k}->{n}", floor=bf16_stored(want))
 
 
+# fp32: both k-split tiles and the 64 x 64 one on a 256-CU device, off their edges; n % 4 != 0 and k % 32 != 0
+# take the scalar forms.
+@pytest.mark.parametrize("m,k,n", [(1, 32, 4), (33, 160, 36), (250, 512, 128), (1000, 96, 260), (4096, 128, 132),
+                                   (9000, 64, 300), (70, 40, 50), (129, 128, 130)])
+@pytest.mark.parametrize("kind", ["linear", "glu", "accumulate"])
+def test_gemm_fp32(device, m, k, n, kind):
+    announce("gemm fp32", m, k, n, kind)
+    g = torch.Generator().manual_seed(m + k + n)
+    x, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g) / math.sqrt(k)
+    if kind == "glu":
+        f = n // 2
+        packed = nh._prepare(w[:2 * f].to(device), torch.float32, "glu")
+        got, want = ops.gated_linear_unit(x.to(device), packed, f, torch.float32), R.gated_linear_unit(x, w[:2 * f].T)
+    elif kind == "linear":
+        bias = torch.randn(n, generator=g)
+        got, want = ops.linear(x.to(device), w.to(device), bias.to(device), torch.float32), x @ w.T + bias
+    else:
+        out, aux = torch.randn(m, n, generator=g), torch.randn(m, n, generator=g)
+        got = ops.linear(x.to(device), w.to(device), None, torch.float32, out=out.to(device),
+                         epilogue=nh.EPI_MUL_SIGMOID_AUX_ACCUMULATE, aux=aux.to(device))
+        want = out + x @ w.T * torch.sigmoid(aux)
+    assert_parity(got, want, TOL_FP32, f"gemm fp32 {kind} {m}x{k}->{n}")
+
+
 @pytest.mark.parametrize("profile", ["jump", "low", "ramp", "mixed"])
 @pytest.mark.parametrize("batch", [3, 8])
 def test_attention_logit_ranges(device, profile, batch):

@@ -168,6 +168,25 @@ __device__ __forceinline__ f32x4 mfma16(const f32x8 &a, const f32x8 &b, f32x4 c)
   return c;
 }
 
+// acc[x][y] += a[x] . b[y] over a grid of tiles. fp32: the eight 16x16x4 products of a tile depend on
+// one another, so the tiles take turns.
+template <int X, int Y>
+__device__ __forceinline__ void mfma_tiles(const bf16x8 (&a)[X], const bf16x8 (&b)[Y], f32x4 (&acc)[X][Y]) {
+#pragma unroll
+  for (int x = 0; x < X; ++x)
+#pragma unroll
+    for (int y = 0; y < Y; ++y) acc[x][y] = mfma16(a[x], b[y], acc[x][y]);
+}
+template <int X, int Y>
+__device__ __forceinline__ void mfma_tiles(const f32x8 (&a)[X], const f32x8 (&b)[Y], f32x4 (&acc)[X][Y]) {
+#pragma unroll
+  for (int s = 0; s < 8; ++s)
+#pragma unroll
+    for (int x = 0; x < X; ++x)
+#pragma unroll
+      for (int y = 0; y < Y; ++y) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x].v[s], b[y].v[s], acc[x][y], 0, 0, 0);
+}
+
 template <typename T> struct Frag;
 template <> struct Frag<bf16> { typedef bf16x8 type; };
 template <> struct Frag<float> { typedef f32x8 type; };

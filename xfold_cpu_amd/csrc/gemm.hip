@@ -7,19 +7,24 @@
 // Tiling: 128 x 128 block tile, k-step 32, 256 threads = 4 wavefronts in a 2 x 2 grid,
 // each owning a 64 x 64 sub-tile = 4 x 4 MFMA 16x16 tiles (bf16: v_mfma_f32_16x16x32_bf16;
 // fp32: 8 x v_mfma_f32_16x16x4f32 per k-step). Problems with fewer 128 x 128 tiles than two
-// per CU take 64 x 64 tiles (32 x 32 per wavefront) instead, four times as many workgroups. Global -> register prefetch of the next
+// per CU, and fp32, take 64 x 64 tiles (32 x 32 per wavefront) instead, four times as many workgroups. Global -> register prefetch of the next
 // k-step overlaps the MFMAs of the current one; LDS rows are padded by 16 bytes so the
-// 16 rows a fragment read touches fall in distinct banks.
+// 16 rows a fragment read touches fall in distinct banks. Aligned operands (VEC) take the vector
+// epilogue of gemm_epilogue.h: the per-element one, with its divisions and its switch, is ten
+// times the main loop's code and cost 2 us a launch.
+#include <type_traits>
+
 #include "common.h"
+#include "gemm_epilogue.h"
 #include "kernels.h"
 
 namespace xfh {
 
 namespace {
 
-constexpr int BK = 32, THREADS = 256;
+constexpr int THREADS = 256;
 
-template <typename T, int BT> struct GemmSmem {
+template <typename T, int BT, int BK> struct GemmSmem {
   static constexpr int kChunk = 16 / sizeof(T);      // elements per 16-byte vector
   static constexpr int kPitch = BK + kChunk;          // padded LDS row (elements)
   T a[BT * kPitch];
@@ -70,10 +75,10 @@ __device__ __forceinline__ float apply_epilogue(int epi, float acc, TO *c, const
 }
 
 // BT x BT block tile (BT = 128 or 64), each wavefront BT/2 x BT/2 = TW x TW MFMA tiles.
-template <typename T, typename TO, bool VEC, bool GLU, int BT>
+template <typename T, typename TO, bool VEC, bool GLU, int BT, int BK = 32>
 __global__ __launch_bounds__(THREADS) void gemm_nt_kernel(GemmArgs p) {
   constexpr int BM = BT, BN = BT, WT = BT / 2, TW = WT / 16;
-  typedef GemmSmem<T, BT> Smem;
+  typedef GemmSmem<T, BT, BK> Smem;
   constexpr int kChunk = Smem::kChunk;
   constexpr int kPitch = Smem::kPitch;
   constexpr int kChunksPerRow = BK / kChunk;
@@ -91,11 +96,13 @@ __global__ __launch_bounds__(THREADS) void gemm_nt_kernel(GemmArgs p) {
   const T *B = static_cast<const T *>(p.B) + batch * p.sB + int64_t(n0) * p.ldb;
   const int rowsA = p.M - m0, rowsB = p.N - n0;
 
+  // acc[j][i]: output tile (row tile i, column tile j); with VEC a lane holds four consecutive
+  // columns of a row (the B rows as the MFMA's A operand), else four rows of a column.
   f32x4 acc[TW][TW];
 #pragma unroll
   for (int i = 0; i < TW; ++i)
 #pragma unroll
-    for (int j = 0; j < TW; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < TW; ++j) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   uint4 ra[kLoads], rb[kLoads];
   auto fetch = [&](int k0) {
@@ -124,18 +131,53 @@ __global__ __launch_bounds__(THREADS) void gemm_nt_kernel(GemmArgs p) {
     stash();
     __syncthreads();
     if (k0 + BK < p.K) fetch(k0 + BK);
-    typename Frag<T>::type fa[TW], fb[TW];
 #pragma unroll
-    for (int i = 0; i < TW; ++i) fa[i] = read_frag<T>(&smem.a[(wm * WT + i * 16 + fr) * kPitch + fk]);
+    for (int ks = 0; ks < BK; ks += 32) {
+      typename Frag<T>::type fa[TW], fb[TW];
 #pragma unroll
-    for (int j = 0; j < TW; ++j) fb[j] = read_frag<T>(&smem.b[(wn * WT + j * 16 + fr) * kPitch + fk]);
+      for (int i = 0; i < TW; ++i) fa[i] = read_frag<T>(&smem.a[(wm * WT + i * 16 + fr) * kPitch + ks + fk]);
 #pragma unroll
-    for (int i = 0; i < TW; ++i)
+      for (int j = 0; j < TW; ++j) fb[j] = read_frag<T>(&smem.b[(wn * WT + j * 16 + fr) * kPitch + ks + fk]);
+      if constexpr (VEC) {
+        mfma_tiles(fb, fa, acc);
+      } else {
 #pragma unroll
-      for (int j = 0; j < TW; ++j) acc[i][j] = mfma16(fa[i], fb[j], acc[i][j]);
+        for (int i = 0; i < TW; ++i)
+#pragma unroll
+          for (int j = 0; j < TW; ++j) acc[j][i] = mfma16(fa[i], fb[j], acc[j][i]);
+      }
+    }
   }
 
   TO *C = static_cast<TO *>(p.C) + batch * p.sC;
+  if constexpr (VEC) {
+    const int mw = m0 + wm * WT, nw = n0 + wn * WT, col = lane & 15, grp = lane >> 4;
+    if constexpr (GLU) {
+#pragma unroll
+      for (int q = 0; q < TW / 2; ++q) {
+        const int f = nw / 2 + q * 16 + grp * 4;
+#pragma unroll
+        for (int i = 0; i < TW; ++i) {
+          const int m = mw + i * 16 + col;
+          if (m >= p.M) continue;
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = siluf_(acc[2 * q][i][e]) * acc[2 * q + 1][i][e];
+          TO *dst = C + int64_t(m) * p.ldc + f;
+          if (f + 4 <= p.glu_f) {
+            Vec4<TO>::store(dst, v);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (f + e < p.glu_f) dst[e] = from_f32<TO>(v[e]);
+          }
+        }
+      }
+    } else {
+      store_any<TO>(p, acc, batch, mw, nw, col, grp);
+    }
+    return;
+  }
   const TO *aux = static_cast<const TO *>(p.aux);
   const int col_lane = lane & 15, row_lane = (lane >> 4) * 4;
   if (GLU) {
@@ -151,7 +193,7 @@ __global__ __launch_bounds__(THREADS) void gemm_nt_kernel(GemmArgs p) {
         for (int e = 0; e < 4; ++e) {
           const int m = m0 + wm * WT + i * 16 + row_lane + e;
           if (m >= p.M) continue;
-          const float g = acc[i][2 * q][e], v = acc[i][2 * q + 1][e];
+          const float g = acc[2 * q][i][e], v = acc[2 * q + 1][i][e];
           C[int64_t(m) * p.ldc + f] = from_f32<TO>(siluf_(g) * v);
         }
     }
@@ -174,7 +216,7 @@ __global__ __launch_bounds__(THREADS) void gemm_nt_kernel(GemmArgs p) {
           const int64_t ar = p.aux_rows > 0 ? (m % p.aux_rows) : m;
           a = aux + batch * p.sAux + ar * p.ldaux + n;
         }
-        float v = acc[i][j][e] + bias;
+        float v = acc[j][i][e] + bias;
         if (p.row_div) v /= p.row_div_eps + p.row_div[m];
         *c = from_f32<TO>(apply_epilogue<TO>(p.epi, v, c, a));
       }
@@ -187,10 +229,13 @@ int launch_typed(const GemmArgs &p, int64_t batch, bool glu, hipStream_t s) {
   const bool vec = (p.K % kChunk == 0) && (p.lda % kChunk == 0) && (p.ldb % kChunk == 0) &&
                    (p.sA % kChunk == 0) && (p.sB % kChunk == 0) &&
                    (reinterpret_cast<uintptr_t>(p.A) % 16 == 0) &&
-                   (reinterpret_cast<uintptr_t>(p.B) % 16 == 0);
+                   (reinterpret_cast<uintptr_t>(p.B) % 16 == 0) && vector_output(p, sizeof(TO));
   int cus = 0;
   XFH_TRY(device_cu_count(&cus));
-  const bool small = ceil_div(p.N, int64_t(128)) * ceil_div(p.M, int64_t(128)) * batch < 2 * int64_t(cus);
+  // fp32 always takes 64 x 64 tiles: a 128 x 128 tile's fragments leave one wavefront per SIMD
+  // ([25600][384] k = 128 91 -> 37 us, [589824][128] 478 -> 291).
+  const bool small = std::is_same<T, float>::value ||
+                     ceil_div(p.N, int64_t(128)) * ceil_div(p.M, int64_t(128)) * batch < 2 * int64_t(cus);
   if (small) {
     dim3 grid(ceil_div(p.N, 64), ceil_div(p.M, 64), batch);
     if (glu) {
@@ -202,13 +247,15 @@ int launch_typed(const GemmArgs &p, int64_t batch, bool glu, hipStream_t s) {
     }
     return check_launch("gemm_nt");
   }
-  dim3 grid(ceil_div(p.N, 128), ceil_div(p.M, 128), batch);
-  if (glu) {
-    if (vec) gemm_nt_kernel<T, TO, true, true, 128><<<grid, THREADS, 0, s>>>(p);
-    else gemm_nt_kernel<T, TO, false, true, 128><<<grid, THREADS, 0, s>>>(p);
-  } else {
-    if (vec) gemm_nt_kernel<T, TO, true, false, 128><<<grid, THREADS, 0, s>>>(p);
-    else gemm_nt_kernel<T, TO, false, false, 128><<<grid, THREADS, 0, s>>>(p);
+  if constexpr (!std::is_same<T, float>::value) {
+    dim3 grid(ceil_div(p.N, 128), ceil_div(p.M, 128), batch);
+    if (glu) {
+      if (vec) gemm_nt_kernel<T, TO, true, true, 128><<<grid, THREADS, 0, s>>>(p);
+      else gemm_nt_kernel<T, TO, false, true, 128><<<grid, THREADS, 0, s>>>(p);
+    } else {
+      if (vec) gemm_nt_kernel<T, TO, true, false, 128><<<grid, THREADS, 0, s>>>(p);
+      else gemm_nt_kernel<T, TO, false, false, 128><<<grid, THREADS, 0, s>>>(p);
+    }
   }
   return check_launch("gemm_nt");
 }
@@ -234,6 +281,11 @@ int gemm_nt(const GemmArgs &p, int64_t batch, int dtype, int out_dtype, bool glu
     return gemm_ring(p, batch, out_dtype, glu, s);
   if (dtype == XFH_BF16 && out_dtype == XFH_BF16) return launch_typed<bf16, bf16>(p, batch, glu, s);
   if (dtype == XFH_BF16 && out_dtype == XFH_F32) return launch_typed<bf16, float>(p, batch, glu, s);
+  if (dtype == XFH_F32 && out_dtype == XFH_F32) {
+    bool taken = false;
+    XFH_TRY(gemm_direct_f32(p, batch, glu, s, &taken));
+    if (taken) return XFH_OK;
+  }
   if (dtype == XFH_F32 && out_dtype == XFH_F32) return launch_typed<float, float>(p, batch, glu, s);
   if (dtype == XFH_F32 && out_dtype == XFH_BF16) return launch_typed<float, bf16>(p, batch, glu, s);
   return fail(XFH_EUNSUPPORTED, "gemm: dtype must be f32 or bf16");

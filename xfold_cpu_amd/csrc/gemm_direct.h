@@ -20,7 +20,17 @@ template <int TM_, int TN_, int KW_, int U_> struct Direct {
   static_assert(TN % 2 == 0, "GLU pairs two 16-column tiles");
 };
 
-template <typename TO, bool GLU, class G, bool ATTN>
+template <typename T> __device__ __forceinline__ typename Frag<T>::type direct_frag(const T *p);
+template <> __device__ __forceinline__ bf16x8 direct_frag<bf16>(const bf16 *p) { return *reinterpret_cast<const bf16x8 *>(p); }
+template <> __device__ __forceinline__ f32x8 direct_frag<float>(const float *p) {
+  f32x8 f;
+  const float4 lo = reinterpret_cast<const float4 *>(p)[0], hi = reinterpret_cast<const float4 *>(p)[1];
+  f.v[0] = lo.x; f.v[1] = lo.y; f.v[2] = lo.z; f.v[3] = lo.w;
+  f.v[4] = hi.x; f.v[5] = hi.y; f.v[6] = hi.z; f.v[7] = hi.w;
+  return f;
+}
+
+template <typename T, typename TO, bool GLU, class G, bool ATTN>
 __global__ __launch_bounds__(64 * G::KW) void gemm_direct_kernel(GemmArgs p) {
   constexpr int TM = G::TM, TN = G::TN, KW = G::KW, U = G::U, TILES = G::TILES;
   __shared__ __attribute__((aligned(16))) f32x4 part[KW][TILES][64];
@@ -29,16 +39,16 @@ __global__ __launch_bounds__(64 * G::KW) void gemm_direct_kernel(GemmArgs p) {
   const int m0 = blockIdx.y * G::BM, n0 = blockIdx.x * G::BN;
   const int64_t batch = blockIdx.z;
   // Rows past M or N read the last row (their results are never stored).
-  const bf16 *a[TM], *b[TN];
+  const T *a[TM], *b[TN];
 #pragma unroll
   for (int y = 0; y < TM; ++y) {
     const int m = m0 + 16 * y + col;
-    a[y] = static_cast<const bf16 *>(p.A) + batch * p.sA + int64_t(m < p.M ? m : p.M - 1) * p.lda + grp * 8;
+    a[y] = static_cast<const T *>(p.A) + batch * p.sA + int64_t(m < p.M ? m : p.M - 1) * p.lda + grp * 8;
   }
 #pragma unroll
   for (int x = 0; x < TN; ++x) {
     const int n = n0 + 16 * x + col;
-    b[x] = static_cast<const bf16 *>(p.B) + batch * p.sB + int64_t(n < p.N ? n : p.N - 1) * p.ldb + grp * 8;
+    b[x] = static_cast<const T *>(p.B) + batch * p.sB + int64_t(n < p.N ? n : p.N - 1) * p.ldb + grp * 8;
   }
   f32x4 acc[TN][TM];
 #pragma unroll
@@ -47,7 +57,7 @@ __global__ __launch_bounds__(64 * G::KW) void gemm_direct_kernel(GemmArgs p) {
     for (int y = 0; y < TM; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int steps = p.K / 32;
   struct Frags {
-    bf16x8 a[U][TM], b[U][TN];
+    typename Frag<T>::type a[U][TM], b[U][TN];
   };
   auto load = [&](Frags &f, int s0) {
 #pragma unroll
@@ -55,19 +65,16 @@ __global__ __launch_bounds__(64 * G::KW) void gemm_direct_kernel(GemmArgs p) {
       const int s = s0 + u * KW;
       if (s >= steps) break;                              // (uniform over the wavefront)
 #pragma unroll
-      for (int y = 0; y < TM; ++y) f.a[u][y] = *reinterpret_cast<const bf16x8 *>(a[y] + s * 32);
+      for (int y = 0; y < TM; ++y) f.a[u][y] = direct_frag<T>(a[y] + s * 32);
 #pragma unroll
-      for (int x = 0; x < TN; ++x) f.b[u][x] = *reinterpret_cast<const bf16x8 *>(b[x] + s * 32);
+      for (int x = 0; x < TN; ++x) f.b[u][x] = direct_frag<T>(b[x] + s * 32);
     }
   };
   auto multiply = [&](const Frags &f, int s0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (s0 + u * KW >= steps) break;
-#pragma unroll
-      for (int x = 0; x < TN; ++x)
-#pragma unroll
-        for (int y = 0; y < TM; ++y) acc[x][y] = mfma16(f.b[u][x], f.a[u][y], acc[x][y]);
+      mfma_tiles(f.b[u], f.a[u], acc);
     }
   };
   Frags f0, f1;
@@ -116,15 +123,7 @@ __global__ __launch_bounds__(64 * G::KW) void gemm_direct_kernel(GemmArgs p) {
       if constexpr (ATTN) {
         store_attn<1, 1>(p, t, mw, nw, col, grp);
       } else {
-        switch (p.epi) {
-          case XFH_EPI_MUL_SIGMOID_AUX: store_tile<XFH_EPI_MUL_SIGMOID_AUX, TO, 1>(p, t, batch, mw, nw, col, grp); break;
-          case XFH_EPI_SIGMOID_MUL_AUX: store_tile<XFH_EPI_SIGMOID_MUL_AUX, TO, 1>(p, t, batch, mw, nw, col, grp); break;
-          case XFH_EPI_ACCUMULATE: store_tile<XFH_EPI_ACCUMULATE, TO, 1>(p, t, batch, mw, nw, col, grp); break;
-          case XFH_EPI_MUL_SIGMOID_AUX_ACCUMULATE:
-            store_tile<XFH_EPI_MUL_SIGMOID_AUX_ACCUMULATE, TO, 1>(p, t, batch, mw, nw, col, grp);
-            break;
-          default: store_tile<XFH_EPI_STORE, TO, 1>(p, t, batch, mw, nw, col, grp);
-        }
+        store_any<TO>(p, t, batch, mw, nw, col, grp);
       }
     }
   }
@@ -136,16 +135,24 @@ int launch_direct(const GemmArgs &p, int64_t batch, int out_dtype, bool glu, hip
   const dim3 block(64 * G::KW);
   const bool b16 = out_dtype == XFH_BF16;
   if (glu) {
-    if (b16) timer.launch(gemm_direct_kernel<bf16, true, G, false>, grid, block, 0, p);
-    else timer.launch(gemm_direct_kernel<float, true, G, false>, grid, block, 0, p);
+    if (b16) timer.launch(gemm_direct_kernel<bf16, bf16, true, G, false>, grid, block, 0, p);
+    else timer.launch(gemm_direct_kernel<bf16, float, true, G, false>, grid, block, 0, p);
   } else if (p.attn.q) {
     if (!b16) return fail(XFH_EUNSUPPORTED, "gemm_direct: the attention layouts are bf16");
-    timer.launch(gemm_direct_kernel<bf16, false, G, true>, grid, block, 0, p);
+    timer.launch(gemm_direct_kernel<bf16, bf16, false, G, true>, grid, block, 0, p);
   } else {
-    if (b16) timer.launch(gemm_direct_kernel<bf16, false, G, false>, grid, block, 0, p);
-    else timer.launch(gemm_direct_kernel<float, false, G, false>, grid, block, 0, p);
+    if (b16) timer.launch(gemm_direct_kernel<bf16, bf16, false, G, false>, grid, block, 0, p);
+    else timer.launch(gemm_direct_kernel<bf16, float, false, G, false>, grid, block, 0, p);
   }
   return check_launch("gemm_direct");
+}
+
+template <class G> int launch_direct_f32(const GemmArgs &p, int64_t batch, bool glu, hipStream_t s, KernelTimer &timer) {
+  const dim3 grid(unsigned(ceil_div(p.N, G::BN)), unsigned(ceil_div(p.M, G::BM)), unsigned(batch));
+  const dim3 block(64 * G::KW);
+  if (glu) timer.launch(gemm_direct_kernel<float, float, true, G, false>, grid, block, 0, p);
+  else timer.launch(gemm_direct_kernel<float, float, false, G, false>, grid, block, 0, p);
+  return check_launch("gemm_direct_f32");
 }
 
 }  // namespace

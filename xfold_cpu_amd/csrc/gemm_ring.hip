@@ -18,6 +18,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_epilogue.h"
 #include "kernels.h"
 
 namespace xfh {
@@ -45,125 +46,6 @@ template <int BN_, int TK_, int SLOTS_, int WGS_, int BM_ = 128> struct Ring {
 
 template <int N> __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-template <typename TO> struct Vec4;
-template <> struct Vec4<bf16> {
-  __device__ static void load(const bf16 *p, float (&v)[4]) {
-    const bf16x4 x = *reinterpret_cast<const bf16x4 *>(p);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = static_cast<float>(x[e]);
-  }
-  __device__ static void store(bf16 *p, const float (&v)[4]) {
-    bf16x4 x;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = bf16(v[e]);
-    *reinterpret_cast<bf16x4 *>(p) = x;
-  }
-};
-template <> struct Vec4<float> {
-  __device__ static void load(const float *p, float (&v)[4]) {
-    const float4 x = *reinterpret_cast<const float4 *>(p);
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-  }
-  __device__ static void store(float *p, const float (&v)[4]) {
-    *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
-  }
-};
-
-template <int EPI> __device__ __forceinline__ float epilogue(float acc, float c, float aux) {
-  if constexpr (EPI == XFH_EPI_MUL_SIGMOID_AUX) return acc * sigmoidf_(aux);
-  else if constexpr (EPI == XFH_EPI_SIGMOID_MUL_AUX) return sigmoidf_(acc) * aux;
-  else if constexpr (EPI == XFH_EPI_ACCUMULATE) return c + acc;
-  else if constexpr (EPI == XFH_EPI_MUL_SIGMOID_AUX_ACCUMULATE) return c + acc * sigmoidf_(aux);
-  else return acc;
-}
-
-// Stores one wavefront's 64 x (16 NT) sub-tile (rows mw + 16 y + col, columns nw + 16 x +
-// 4 grp + e) through epilogue EPI. The epilogue kind is a template parameter and the row
-// quantities (row divisor, auxiliary row) are taken once per row: a runtime switch per
-// element made this code ~10x larger than the main loop, and its instruction-cache misses
-// cost ~10 us per launch whatever the grid.
-template <int EPI, typename TO, int NT, int MT>
-__device__ __forceinline__ void store_tile(const GemmArgs &p, const f32x4 (&acc)[NT][MT], int64_t batch, int mw,
-                                           int nw, int col, int grp) {
-  constexpr bool READS_C = EPI == XFH_EPI_ACCUMULATE || EPI == XFH_EPI_MUL_SIGMOID_AUX_ACCUMULATE;
-  constexpr bool AUX = EPI == XFH_EPI_MUL_SIGMOID_AUX || EPI == XFH_EPI_SIGMOID_MUL_AUX ||
-                       EPI == XFH_EPI_MUL_SIGMOID_AUX_ACCUMULATE;
-  TO *C = static_cast<TO *>(p.C) + batch * p.sC;
-  int m[MT];
-  float rs[MT];
-  const TO *arow[MT];
-#pragma unroll
-  for (int y = 0; y < MT; ++y) {
-    m[y] = mw + y * 16 + col;
-    rs[y] = p.row_div && m[y] < p.M ? 1.0f / (p.row_div_eps + p.row_div[m[y]]) : 1.0f;
-    arow[y] = nullptr;
-    if constexpr (AUX) {
-      const int ar = p.aux_rows > 0 ? m[y] % int(p.aux_rows) : m[y];
-      arow[y] = static_cast<const TO *>(p.aux) + batch * p.sAux + int64_t(ar) * p.ldaux;
-    }
-  }
-  if (p.pair_blk == 0 && mw + 16 * MT <= p.M && nw + 16 * NT <= p.N) {
-    // Interior sub-tile (every tile of the usual shapes): straight-line code, no per-element
-    // bounds, row-major addresses.
-#pragma unroll
-    for (int x = 0; x < NT; ++x) {
-      const int n = nw + x * 16 + grp * 4;
-      float bias[4] = {0.f, 0.f, 0.f, 0.f};
-      if (p.bias)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bias[e] = p.bias[batch * p.sBias + n + e];
-#pragma unroll
-      for (int y = 0; y < MT; ++y) {
-        TO *c = C + int64_t(m[y]) * p.ldc + n;
-        float cv[4] = {0.f, 0.f, 0.f, 0.f}, av[4] = {0.f, 0.f, 0.f, 0.f}, out[4];
-        if constexpr (READS_C) Vec4<TO>::load(c, cv);
-        if constexpr (AUX) Vec4<TO>::load(arow[y] + n, av);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) out[e] = epilogue<EPI>((acc[x][y][e] + bias[e]) * rs[y], cv[e], av[e]);
-        Vec4<TO>::store(c, out);
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int x = 0; x < NT; ++x) {
-    const int n = nw + x * 16 + grp * 4;
-    if (n >= p.N) continue;
-    const bool full = n + 4 <= p.N;
-    float bias[4] = {0.f, 0.f, 0.f, 0.f};
-    if (p.bias)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) bias[e] = n + e < p.N ? p.bias[batch * p.sBias + n + e] : 0.f;
-#pragma unroll
-    for (int y = 0; y < MT; ++y) {
-      if (m[y] >= p.M) continue;
-      TO *c = c_element(p, C, m[y], n);
-      float cv[4] = {0.f, 0.f, 0.f, 0.f}, av[4] = {0.f, 0.f, 0.f, 0.f}, out[4];
-      if (full) {
-        if constexpr (READS_C) Vec4<TO>::load(c, cv);
-        if constexpr (AUX) Vec4<TO>::load(arow[y] + n, av);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (n + e >= p.N) continue;
-          if constexpr (READS_C) cv[e] = to_f32(c[e]);
-          if constexpr (AUX) av[e] = to_f32(arow[y][n + e]);
-        }
-      }
-      // (acc + bias) * 1.0f is exact, so rows without a divisor keep acc + bias.
-#pragma unroll
-      for (int e = 0; e < 4; ++e) out[e] = epilogue<EPI>((acc[x][y][e] + bias[e]) * rs[y], cv[e], av[e]);
-      if (full) {
-        Vec4<TO>::store(c, out);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (n + e < p.N) c[e] = from_f32<TO>(out[e]);
-      }
-    }
-  }
 }
 
 // Position of key t inside the attention kernel's V^T rows: within each run of 32 keys,
@@ -409,22 +291,7 @@ __global__ __launch_bounds__(256, G::WGS) void gemm_ring_kernel(GemmArgs p) {
     store_attn(p, acc, mw, nw, col, grp);
     return;
   }
-  switch (p.epi) {
-    case XFH_EPI_MUL_SIGMOID_AUX:
-      store_tile<XFH_EPI_MUL_SIGMOID_AUX, TO, NT>(p, acc, batch, mw, nw, col, grp);
-      break;
-    case XFH_EPI_SIGMOID_MUL_AUX:
-      store_tile<XFH_EPI_SIGMOID_MUL_AUX, TO, NT>(p, acc, batch, mw, nw, col, grp);
-      break;
-    case XFH_EPI_ACCUMULATE:
-      store_tile<XFH_EPI_ACCUMULATE, TO, NT>(p, acc, batch, mw, nw, col, grp);
-      break;
-    case XFH_EPI_MUL_SIGMOID_AUX_ACCUMULATE:
-      store_tile<XFH_EPI_MUL_SIGMOID_AUX_ACCUMULATE, TO, NT>(p, acc, batch, mw, nw, col, grp);
-      break;
-    default:
-      store_tile<XFH_EPI_STORE, TO, NT>(p, acc, batch, mw, nw, col, grp);
-  }
+  store_any<TO>(p, acc, batch, mw, nw, col, grp);
 }
 
 }  // namespace
@@ -529,12 +396,8 @@ DirectPick pick_direct(const GemmArgs &p, int64_t batch, int cus) {
 }
 
 bool gemm_ring_supported(const GemmArgs &p, int out_dtype) {
-  const int ob = out_dtype == XFH_BF16 ? 2 : 4;
-  if (p.pair_blk && (p.pair_blk % 4 || !aligned(p.C, 4 * ob) || p.sC % 4)) return false;
-  const bool vec_out = p.ldc % 4 == 0 && p.sC % 4 == 0 && aligned(p.C, 4 * ob) &&
-                       (!p.aux || (p.ldaux % 4 == 0 && p.sAux % 4 == 0 && aligned(p.aux, 4 * ob)));
-  return p.K > 0 && p.K % 32 == 0 && p.aux_rows <= INT32_MAX && p.lda % 8 == 0 && p.ldb % 8 == 0 && p.sA % 8 == 0 &&
-         p.sB % 8 == 0 && aligned(p.A, 16) && aligned(p.B, 16) && vec_out;
+  return p.K > 0 && p.K % 32 == 0 && p.lda % 8 == 0 && p.ldb % 8 == 0 && p.sA % 8 == 0 && p.sB % 8 == 0 &&
+         aligned(p.A, 16) && aligned(p.B, 16) && vector_output(p, out_dtype == XFH_BF16 ? 2 : 4);
 }
 
 int gemm_ring(const GemmArgs &p, int64_t batch, int out_dtype, bool glu, hipStream_t s) {
@@ -574,6 +437,27 @@ int gemm_ring(const GemmArgs &p, int64_t batch, int out_dtype, bool glu, hipStre
     case RingPick::Shallow: return launch_ring<RingShallow>(q, batch, out_dtype, glu, s, timer);
     default: return launch_ring<RingShallowNarrow>(q, batch, out_dtype, glu, s, timer);
   }
+}
+
+// fp32: 32 x 32 tiles while they leave a CU to each, 32 x 64 up to twice as many tiles as CUs, then
+// gemm_nt's 64 x 64. us per launch, direct against gemm_nt: [256][128] k = 128 4.1 / 8.6, k = 512 7.3 / 20, k = 1536
+// ([256][384]) 14 / 49; [4096][128] k = 128 5.4 / 9.3, k = 512 10.6 / 20.7; [16384][4] (the pair bias) 4.3 / 8.8; past the
+// line [16384][128] 13.3 / 12.6, [4096][384] 11.3 / 12.6. The error against 64 bits is half of gemm_nt's (four
+// partial sums of a quarter of the terms).
+int gemm_direct_f32(const GemmArgs &p, int64_t batch, bool glu, hipStream_t s, bool *taken) {
+  *taken = false;
+  if (p.K < 32 || p.K % 32 || p.lda % 4 || p.ldb % 4 || p.sA % 4 || p.sB % 4 || !aligned(p.A, 16) || !aligned(p.B, 16) ||
+      !vector_output(p, 4) || batch > 65535)
+    return XFH_OK;
+  int cus = 0;
+  XFH_TRY(device_cu_count(&cus));
+  const int64_t small = ceil_div(p.M, 32) * ceil_div(p.N, 32) * batch;
+  const int64_t wide = ceil_div(p.M, 32) * ceil_div(p.N, 64) * batch;
+  if (small > cus && wide > 2 * int64_t(cus)) return XFH_OK;
+  *taken = true;
+  KernelTimer timer("gemm_direct_f32", s, 2.0 * double(p.M) * double(p.N) * double(p.K) * double(batch), true);
+  return small <= cus ? launch_direct_f32<Direct<2, 2, 4, 2>>(p, batch, glu, s, timer)
+                      : launch_direct_f32<Direct<2, 4, 4, 1>>(p, batch, glu, s, timer);
 }
 
 }  // namespace xfh

@@ -61,6 +61,9 @@ int stack_rows(void *dst, const void *const src[4], const int64_t rows[4], int64
 // gemm_ring_supported (k a multiple of 32, 16-byte aligned operand rows, 4-aligned output).
 bool gemm_ring_supported(const GemmArgs &p, int out_dtype);
 int gemm_ring(const GemmArgs &p, int64_t batch, int out_dtype, bool glu, hipStream_t s);
+// fp32 GEMM with k split over a workgroup's wavefronts (gemm_direct.h), for outputs of few tiles;
+// *taken says whether it ran.
+int gemm_direct_f32(const GemmArgs &p, int64_t batch, bool glu, hipStream_t s, bool *taken);
 int glu_pack(const void *w, int64_t f, int64_t k, int dtype, void *packed, hipStream_t s);
 
 int layer_norm_rows(const void *x, int xd, int64_t rows, int64_t C, const float *w, const float *b,
@@ -252,6 +255,35 @@ int64_t contraction_result_elems(int64_t n, int64_t channels);
 int contraction(const ContractionArgs &a, hipStream_t s);
 int trimul_project(const TriProjectArgs &a, int pair_dtype, hipStream_t s);
 int trimul_output(const TriOutputArgs &a, int pair_dtype, int out_dtype, hipStream_t s);
+
+// MSA stack at 64 channels (msa_fused.hip).
+struct MsaProjectArgs {
+  const void *x;             // msa rows [.][64]
+  const void *mask;          // one value per row, or null
+  int mask_dtype;
+  const float *ln_w, *ln_b;
+  float eps;
+  const bf16 *w;             // [64][64]
+  // Row of (line, t): line * line_rows + t * t_rows, t < t_len, line < lines; zeros up to t_pad, lines_pad.
+  int lines, lines_pad, t_len, t_pad;
+  int64_t line_rows, t_rows;
+  // Channel p, line, t at (p < split ? out0 : out1) + (p % split) ch_stride + line * line_stride + t.
+  bf16 *out0, *out1;
+  int split;
+  int64_t ch_stride, line_stride;
+  bf16 *mask_out;            // [lines_pad][t_pad], or null
+};
+struct MsaOutputArgs {
+  const void *x;             // msa [rows][n][64]
+  const bf16 *avg_t;         // [heads][n][dv][rows_pad]
+  const float *ln_w, *ln_b;
+  float eps;
+  const bf16 *w_gating, *w_out;
+  void *out;
+  int accumulate, rows, rows_pad, n, dv;
+};
+int msa_project(const MsaProjectArgs &a, int x_dtype, hipStream_t s);
+int msa_output(const MsaOutputArgs &a, int x_dtype, int out_dtype, hipStream_t s);
 
 // Triangle multiplication helpers.
 int trimul_gate(const void *proj, const void *gate, int dtype, const void *mask, int mask_dtype,
