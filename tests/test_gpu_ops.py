@@ -885,6 +885,31 @@ def test_gemm_fp32(device, m, k, n, kind):
     assert_parity(got, want, TOL_FP32, f"gemm fp32 {kind} {m}x{k}->{n}")
 
 
+@pytest.mark.parametrize("n", [3, 64, 68, 130])
+@pytest.mark.parametrize("layout", ["planes", "head_minor", "odd"])
+@pytest.mark.parametrize("mask", ["keys", "query", None])
+def test_attention_fp32_bias_and_mask_forms(device, n, layout, mask):
+    """The general kernel's four-key bias reads and per-block key mask against its element reads:
+    biases contiguous along the keys, with the heads innermost and in unaligned rows, masks per key
+    and per (query, key)."""
+    announce("attention fp32 forms", n, layout, mask)
+    g = torch.Generator().manual_seed(n)
+    b, h, d = 2, 4, 32
+    q, k, v = (torch.randn(b, h, n, d, generator=g) for _ in range(3))
+    bias = torch.randn(1, h, n, n, generator=g)
+    on_gpu = bias.to(device)
+    if layout == "head_minor":
+        on_gpu = bias.permute(0, 2, 3, 1).contiguous().to(device).permute(0, 3, 1, 2)
+    elif layout == "odd":
+        base = torch.zeros(1, h, n, n + 1, device=device)
+        base[..., 1:] = on_gpu
+        on_gpu = base[..., 1:]
+    m = None if mask is None else torch.rand((b, n) if mask == "keys" else (b, 1, n, n), generator=g) > 0.3
+    want = R.dot_product_attention(q, k, v, m, bias.clone())
+    got = ops.attention(q.to(device), k.to(device), v.to(device), None if m is None else m.to(device), on_gpu)
+    assert_parity(got, want, TOL_FP32, "attention fp32 forms")
+
+
 @pytest.mark.parametrize("profile", ["jump", "low", "ramp", "mixed"])
 @pytest.mark.parametrize("batch", [3, 8])
 def test_attention_logit_ranges(device, profile, batch):

@@ -674,7 +674,11 @@ int xfh_grid_self_attention(const void *pair, int pair_dtype, const void *mask, 
     return grid_output(oa, pair_dtype, out_dtype, s);
   }
   XFH_TRY(layer_norm_rows(pair, pair_dtype, plane, c, norm_w, norm_b, eps, p.normed, dtype, s));
-  GemmArgs g = gemm_args(p.normed, c, bias_w, c, p.bias, heads, plane, heads, c);
+  // fp32: the bias as [h][i][j] (the weight's rows as the product's rows), so the attention reads four
+  // keys at a time; bf16 keeps the heads innermost for attention_bias_pack.
+  const bool bias_planes = dtype == XFH_F32;
+  GemmArgs g = bias_planes ? gemm_args(bias_w, c, p.normed, c, p.bias, plane, heads, plane, c)
+                           : gemm_args(p.normed, c, bias_w, c, p.bias, heads, plane, heads, c);
   XFH_TRY(gemm_nt(g, 1, dtype, dtype, false, s));
   // [q | k | v] = LN(z) [Wq; Wk; Wv]^T in one GEMM: the normalised pair is read once for the
   // three projections (each output column is the same dot product as in a GEMM of its own).
@@ -705,7 +709,8 @@ int xfh_grid_self_attention(const void *pair, int pair_dtype, const void *mask, 
   a.mask = mask; a.mask_dtype = mask_dtype;
   a.ms[0] = n; a.ms[1] = 0; a.ms[2] = 0; a.ms[3] = 1;
   a.bias = p.bias; a.bias_dtype = dtype;
-  a.bs[0] = 0; a.bs[1] = 1; a.bs[2] = n * heads; a.bs[3] = heads;
+  a.bs[0] = 0;
+  a.bs[1] = bias_planes ? plane : 1; a.bs[2] = bias_planes ? n : n * heads; a.bs[3] = bias_planes ? 1 : heads;
   a.scale = 1.0f / std::sqrt(float(dh));
   // bf16: the pipelined attention kernel on operands repacked from the projections: whole
   // projection rows through LDS (qkv_repack) where the width allows, else mha_prepare's

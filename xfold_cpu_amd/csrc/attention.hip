@@ -23,6 +23,10 @@ constexpr int KB = 64;    // keys per block
 
 template <typename T> struct AttnSmemPitch { static constexpr int kPad = 16 / sizeof(T); };
 
+// A bias that is contiguous along aligned groups of four keys is read four at a time, and a mask that
+// does not depend on the query once per key block, into LDS: the fp32 grid attention at n = 128
+// (4 heads of 32) 44 us with element reads of both, 33 now. (16-byte reads of q, k and v took 254
+// registers and 56 us, 35 held to two wavefronts per SIMD.)
 template <typename T, typename TO, int DP, int DVT>
 __global__ __launch_bounds__(256) void attention_kernel(AttentionArgs a) {
   constexpr int kPad = AttnSmemPitch<T>::kPad;
@@ -30,6 +34,7 @@ __global__ __launch_bounds__(256) void attention_kernel(AttentionArgs a) {
   constexpr int VP = KB + kPad;          // V^T tile pitch
   __shared__ T ks[KB * KP];
   __shared__ T vt[DVT * 16 * VP];
+  __shared__ float keep[KB];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t b = blockIdx.z, h = blockIdx.y;
@@ -60,6 +65,10 @@ __global__ __launch_bounds__(256) void attention_kernel(AttentionArgs a) {
   const char *biasb = static_cast<const char *>(a.bias);
   const uint8_t *maskb = static_cast<const uint8_t *>(a.mask);
 
+  const bool key_mask = maskb && a.ms[2] == 0;
+  const int64_t bias_row = b * a.bs[0] + h * a.bs[1] + query * a.bs[2];
+  const bool bias_quads = a.bias && a.bs[3] == 1 && a.bs[0] % 4 == 0 && a.bs[1] % 4 == 0 && a.bs[2] % 4 == 0 &&
+                          reinterpret_cast<uintptr_t>(a.bias) % (a.bias_dtype == XFH_F32 ? 16 : 8) == 0;
   float m_run = -INFINITY;
   float l_part = 0.f;
   f32x4 o[DVT];
@@ -80,6 +89,8 @@ __global__ __launch_bounds__(256) void attention_kernel(AttentionArgs a) {
       const int64_t key = kb0 + r;
       vt[d * VP + r] = (key < a.K && d < a.Dv) ? vp[key * a.vs[2] + d] : T(0);
     }
+    if (key_mask && tid < KB && kb0 + tid < a.K)
+      keep[tid] = load_any(maskb, a.mask_dtype, b * a.ms[0] + h * a.ms[1] + (kb0 + tid) * a.ms[3]);
     __syncthreads();
 
     // S^T for 4 tiles of 16 keys: lane holds keys kt*16 + 4*grp + e of query `col`.
@@ -100,22 +111,38 @@ __global__ __launch_bounds__(256) void attention_kernel(AttentionArgs a) {
 
     float bmax = -INFINITY;
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
+    for (int kt = 0; kt < 4; ++kt) {
+      const int64_t key0 = kb0 + kt * 16 + grp * 4;
+      float bq[4] = {0.f, 0.f, 0.f, 0.f};
+      if (qvalid && bias_quads && key0 + 4 <= a.K) {
+        if (a.bias_dtype == XFH_F32) {
+          const float4 x = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(biasb) + bias_row + key0);
+          bq[0] = x.x; bq[1] = x.y; bq[2] = x.z; bq[3] = x.w;
+        } else {
+          const bf16x4 x = *reinterpret_cast<const bf16x4 *>(reinterpret_cast<const bf16 *>(biasb) + bias_row + key0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) bq[e] = static_cast<float>(x[e]);
+        }
+      } else if (qvalid && a.bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (key0 + e < a.K) {
+            const int64_t off = bias_row + (key0 + e) * a.bs[3];
+            bq[e] = a.bias_dtype == XFH_F32 ? reinterpret_cast<const float *>(biasb)[off]
+                                            : static_cast<float>(reinterpret_cast<const bf16 *>(biasb)[off]);
+          }
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int64_t key = kb0 + kt * 16 + grp * 4 + e;
+        const int64_t key = key0 + e;
         float v = sv[kt][e];
         if (key >= a.K) {
           v = -INFINITY;
         } else if (qvalid) {
-          if (a.bias) {
-            const int64_t off = b * a.bs[0] + h * a.bs[1] + query * a.bs[2] + key * a.bs[3];
-            const float bv = a.bias_dtype == XFH_F32
-                                 ? reinterpret_cast<const float *>(biasb)[off]
-                                 : static_cast<float>(reinterpret_cast<const bf16 *>(biasb)[off]);
-            v += bv * kLog2e;
-          }
-          if (maskb) {
+          if (a.bias) v += bq[e] * kLog2e;
+          if (key_mask) {
+            if (keep[kt * 16 + grp * 4 + e] == 0.f) v = masked_logit;
+          } else if (maskb) {
             const int64_t off = b * a.ms[0] + h * a.ms[1] + query * a.ms[2] + key * a.ms[3];
             if (load_any(maskb, a.mask_dtype, off) == 0.f) v = masked_logit;
           }
@@ -123,6 +150,7 @@ __global__ __launch_bounds__(256) void attention_kernel(AttentionArgs a) {
         sv[kt][e] = v;
         bmax = fmaxf(bmax, v);
       }
+    }
     bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
     bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
     const float m_new = fmaxf(m_run, bmax);
