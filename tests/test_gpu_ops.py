@@ -885,6 +885,16 @@ def test_gemm_fp32(device, m, k, n, kind):
     assert_parity(got, want, TOL_FP32, f"gemm fp32 {kind} {m}x{k}->{n}")
 
 
+def test_gemm_fp32_more_rows_than_a_grid_of_small_tiles(device):
+    """65535 tiles of 64 rows and one more: the 128 x 128 tiles take over."""
+    m = 65535 * 64 + 1
+    announce("gemm fp32 rows", m)
+    g = torch.Generator().manual_seed(0)
+    x, w = torch.randn(m, 4, generator=g), torch.randn(4, 4, generator=g)
+    got = ops.linear(x.to(device), w.to(device), None, torch.float32)
+    assert_parity(got, x @ w.T, TOL_FP32, f"gemm fp32 {m} rows")
+
+
 @pytest.mark.parametrize("n", [3, 64, 68, 130])
 @pytest.mark.parametrize("layout", ["planes", "head_minor", "odd"])
 @pytest.mark.parametrize("mask", ["keys", "query", None])

@@ -7,9 +7,10 @@
 // Tiling: 128 x 128 block tile, k-step 32, 256 threads = 4 wavefronts in a 2 x 2 grid,
 // each owning a 64 x 64 sub-tile = 4 x 4 MFMA 16x16 tiles (bf16: v_mfma_f32_16x16x32_bf16;
 // fp32: 8 x v_mfma_f32_16x16x4f32 per k-step). Problems with fewer 128 x 128 tiles than two
-// per CU, and fp32, take 64 x 64 tiles (32 x 32 per wavefront) instead, four times as many workgroups. Global -> register prefetch of the next
-// k-step overlaps the MFMAs of the current one; LDS rows are padded by 16 bytes so the
-// 16 rows a fragment read touches fall in distinct banks. Aligned operands (VEC) take the vector
+// per CU, and fp32, take 64 x 64 tiles (32 x 32 per wavefront) instead, four times as many
+// workgroups. Global -> register prefetch of the next k-step overlaps the MFMAs of the current
+// one; LDS rows are padded by 16 bytes so the 16 rows a fragment read touches fall in distinct
+// banks. Aligned operands (VEC) take the vector
 // epilogue of gemm_epilogue.h: the per-element one, with its divisions and its switch, is ten
 // times the main loop's code and cost 2 us a launch.
 #include <type_traits>
@@ -23,8 +24,9 @@ namespace xfh {
 namespace {
 
 constexpr int THREADS = 256;
+constexpr int BK = 32;  // k-step
 
-template <typename T, int BT, int BK> struct GemmSmem {
+template <typename T, int BT> struct GemmSmem {
   static constexpr int kChunk = 16 / sizeof(T);      // elements per 16-byte vector
   static constexpr int kPitch = BK + kChunk;          // padded LDS row (elements)
   T a[BT * kPitch];
@@ -75,10 +77,10 @@ __device__ __forceinline__ float apply_epilogue(int epi, float acc, TO *c, const
 }
 
 // BT x BT block tile (BT = 128 or 64), each wavefront BT/2 x BT/2 = TW x TW MFMA tiles.
-template <typename T, typename TO, bool VEC, bool GLU, int BT, int BK = 32>
+template <typename T, typename TO, bool VEC, bool GLU, int BT>
 __global__ __launch_bounds__(THREADS) void gemm_nt_kernel(GemmArgs p) {
   constexpr int BM = BT, BN = BT, WT = BT / 2, TW = WT / 16;
-  typedef GemmSmem<T, BT, BK> Smem;
+  typedef GemmSmem<T, BT> Smem;
   constexpr int kChunk = Smem::kChunk;
   constexpr int kPitch = Smem::kPitch;
   constexpr int kChunksPerRow = BK / kChunk;
@@ -232,9 +234,10 @@ int launch_typed(const GemmArgs &p, int64_t batch, bool glu, hipStream_t s) {
                    (reinterpret_cast<uintptr_t>(p.B) % 16 == 0) && vector_output(p, sizeof(TO));
   int cus = 0;
   XFH_TRY(device_cu_count(&cus));
-  // fp32 always takes 64 x 64 tiles: a 128 x 128 tile's fragments leave one wavefront per SIMD
-  // ([25600][384] k = 128 91 -> 37 us, [589824][128] 478 -> 291).
-  const bool small = std::is_same<T, float>::value ||
+  // fp32 takes 64 x 64 tiles: a 128 x 128 tile's fragments leave one wavefront per SIMD
+  // ([25600][384] k = 128 91 -> 37 us, [589824][128] 478 -> 291). Only more rows than a grid of
+  // 64-row tiles can hold (M > 4194240) keep the larger ones.
+  const bool small = (std::is_same<T, float>::value && ceil_div(p.M, int64_t(64)) <= 65535) ||
                      ceil_div(p.N, int64_t(128)) * ceil_div(p.M, int64_t(128)) * batch < 2 * int64_t(cus);
   if (small) {
     dim3 grid(ceil_div(p.N, 64), ceil_div(p.M, 64), batch);
@@ -247,15 +250,13 @@ int launch_typed(const GemmArgs &p, int64_t batch, bool glu, hipStream_t s) {
     }
     return check_launch("gemm_nt");
   }
-  if constexpr (!std::is_same<T, float>::value) {
-    dim3 grid(ceil_div(p.N, 128), ceil_div(p.M, 128), batch);
-    if (glu) {
-      if (vec) gemm_nt_kernel<T, TO, true, true, 128><<<grid, THREADS, 0, s>>>(p);
-      else gemm_nt_kernel<T, TO, false, true, 128><<<grid, THREADS, 0, s>>>(p);
-    } else {
-      if (vec) gemm_nt_kernel<T, TO, true, false, 128><<<grid, THREADS, 0, s>>>(p);
-      else gemm_nt_kernel<T, TO, false, false, 128><<<grid, THREADS, 0, s>>>(p);
-    }
+  dim3 grid(ceil_div(p.N, 128), ceil_div(p.M, 128), batch);
+  if (glu) {
+    if (vec) gemm_nt_kernel<T, TO, true, true, 128><<<grid, THREADS, 0, s>>>(p);
+    else gemm_nt_kernel<T, TO, false, true, 128><<<grid, THREADS, 0, s>>>(p);
+  } else {
+    if (vec) gemm_nt_kernel<T, TO, true, false, 128><<<grid, THREADS, 0, s>>>(p);
+    else gemm_nt_kernel<T, TO, false, false, 128><<<grid, THREADS, 0, s>>>(p);
   }
   return check_launch("gemm_nt");
 }
