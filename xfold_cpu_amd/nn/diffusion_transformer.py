@@ -383,10 +383,11 @@ def diffusion_transformer_hip(module: nn.Module, act: torch.Tensor, mask: torch.
     # host time than the two batched GEMMs they would save.
     conds = weights = None
     if _conditioned_alike(single_cond, alns, zeros):
-        block_weights, rest = _block_sources(att, tr, alns, zeros)
-        _, weights = nh.gather(
-            module, "blocks", block_weights + projs + rest, len(block_weights), act,
-            lambda dt: _block_weights(module, att, tr, alns, zeros, projs, dt), again=True)
+        if not nh.first_pass(module, "blocks"):
+            block_weights, rest = _block_sources(att, tr, alns, zeros)
+            _, weights = nh.gather(
+                module, "blocks", block_weights + projs + rest, len(block_weights), act,
+                lambda dt: _block_weights(module, att, tr, alns, zeros, projs, dt), again=True)
         conds = _block_conditioning(single_cond, alns, dtype, act.dtype,
                                     weights["conditioning"] if weights is not None else
                                     _conditioning_weights(module, alns, zeros, dtype))

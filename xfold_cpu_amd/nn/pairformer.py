@@ -111,6 +111,8 @@ def _single_track_hip(block: nn.Module, pair: torch.Tensor, single: torch.Tensor
     """The pair transition with its logits and the whole single track in one library call
     (``xfh_pairformer_single``), where the operators' own bf16 paths take those shapes; False
     (nothing done) otherwise."""
+    if nh.first_pass(block, "single_track"):
+        return False
     m = block._modules
     tr, norm, att, str_ = (m[name] for name in ("pair_transition", "single_pair_logits_norm", "single_attention_",
                                                 "single_transition"))
@@ -180,8 +182,6 @@ def _pair_updates_hip(block: nn.Module, pair: torch.Tensor, pair_mask: torch.Ten
     m = block._modules
     triangles, grids = [m[name] for name in _TRIANGLES], [m[name] for name in _GRIDS]
     tr = m["pair_transition"]
-    tr_w = nh.params(tr, ("transition1", "transition2"))
-    c, heads, f = pair.shape[-1], grids[0].num_head, tr_w[1].shape[1]
 
     def one_by_one():
         triangle_multiplication_hip(triangles[0], pair, pair_mask, accumulate_into=pair)
@@ -190,6 +190,10 @@ def _pair_updates_hip(block: nn.Module, pair: torch.Tensor, pair_mask: torch.Ten
         grid_self_attention_hip(grids[1], pair, pair_mask, accumulate_into=pair)
         if transition:
             transition_hip(tr, pair, accumulate_into=pair)
+    if nh.first_pass(block, "pair_updates"):
+        return one_by_one()
+    tr_w = nh.params(tr, ("transition1", "transition2"))
+    c, heads, f = pair.shape[-1], grids[0].num_head, tr_w[1].shape[1]
     if (pair.dim() != 3 or pair.shape[0] != pair.shape[1] or pair_mask is None or heads != grids[1].num_head
             or any(t.c_pair != c for t in triangles + grids) or tr_w[0].shape != (2 * f, c)):
         return one_by_one()
