@@ -214,6 +214,68 @@ def test_gathered_weights_follow_every_change_of_a_source():
         assert not torch.equal(get()[1], got)             # no version counter: never kept
 
 
+def _two_swaps(p):
+    """New values in ``p`` through two ``.data`` swaps (offload and reload): the allocator may hand the
+    second storage the first one's address, and ``_version`` does not move."""
+    shape = p.shape
+    p.data = torch.empty(8)
+    p.data = torch.randn(shape)
+
+
+def test_kept_weights_notice_a_reused_address():
+    """Every cache of prepared weights tells a new storage at an old address from the old one."""
+    import copy
+    module = torch.nn.Module()
+    module.lin = torch.nn.Linear(64, 64, bias=False)
+    module.fused = torch.nn.Linear(64, 64, bias=False)
+    x, bf16 = torch.zeros(1), torch.bfloat16
+    kinds = (lambda m: nh.gather(m, "t", nh.params(m, ("lin",)), 0, x, lambda dt: m.lin.weight.detach().to(dt), bf16)[1],
+             lambda m: nh.linear_weight(m, "lin", bf16),
+             lambda m: nh.fused_linear_weight(m, ("fused", "lin"), bf16)[64:],
+             lambda m: nh.derived_weight(m, "d", [m.lin.weight], lambda w: w.detach().to(bf16)))
+    with torch.no_grad():
+        for kind in kinds:
+            kind(module)
+            kind(module)                                # (a group is kept from its second pass on)
+            for _ in range(20):
+                _two_swaps(module.lin.weight)
+                assert torch.equal(kind(module), module.lin.weight.detach().bfloat16())
+            twin = copy.deepcopy(module)
+            for _ in range(20):
+                _two_swaps(twin.lin.weight)
+                assert torch.equal(kind(twin), twin.lin.weight.detach().bfloat16())
+
+
+def test_projection_bias_notices_a_reused_address():
+    from xfold_cpu_amd.nn.diffusion_transformer import _projection_bias
+    module = torch.nn.Module()
+    module.q_projection = torch.nn.Linear(4, 4096)
+    with torch.no_grad():
+        _projection_bias(module, 4096, 2, torch.device("cpu"))
+        for _ in range(20):
+            _two_swaps(module.q_projection.bias)
+            assert torch.equal(_projection_bias(module, 4096, 2, torch.device("cpu"))[:4096], module.q_projection.bias)
+
+
+def test_mask_words_notice_a_reused_address(monkeypatch):
+    from xfold_cpu_amd.fastnn import ops
+    calls = []
+    monkeypatch.setattr(nh, "call", lambda name, *args: calls.append(name))
+    monkeypatch.setattr(nh, "ptr", lambda t: t.data_ptr())
+    monkeypatch.setattr(nh, "stream_of", lambda device: 0)
+    operands = ops.AttentionOperands.__new__(ops.AttentionOperands)
+    operands.shape, operands.device, operands.words = (1, 4096, 1, 32), torch.device("cpu"), torch.zeros(1)
+    operands._mask_key = ()
+    mask = torch.ones(4096)
+    operands.set_mask(mask)
+    operands.set_mask(mask)
+    assert len(calls) == 1
+    for i in range(20):
+        _two_swaps(mask)
+        operands.set_mask(mask)
+        assert len(calls) == 2 + i
+
+
 @pytest.mark.parametrize("fixture,cls", [
     ("pairformer_block", "PairformerBlock"), ("diffusion_transformer", "DiffusionTransformer"),
     ("grid_attention_start", "GridSelfAttention"), ("self_attention_cond", "SelfAttention"),

@@ -39,6 +39,18 @@ def test_reuses_and_invalidates_on_feature_and_weight_updates():
     assert not cache._entries
 
 
+def test_a_reused_address_is_not_the_same_tensor():
+    """Two ``.data`` swaps of a feature or a weight (offload and reload) may end at the old address."""
+    owner, cache, feature = nn.Linear(64, 64).eval(), InputCache(), torch.randn(64, 64)
+    with torch.no_grad(), input_cache_scope():
+        for tensor in (feature, owner.weight):
+            cache.get("x", (feature,), owner, lambda: owner(feature))
+            for _ in range(20):
+                tensor.data = torch.empty(8)
+                tensor.data = torch.randn(64, 64)
+                torch.testing.assert_close(cache.get("x", (feature,), owner, lambda: owner(feature)), owner(feature))
+
+
 def test_copy_budget_training_and_exception_cleanup():
     owner, cache, feature = nn.Linear(3, 3).eval(), InputCache(), torch.randn(2, 3)
     calls = []

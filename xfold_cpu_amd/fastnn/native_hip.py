@@ -260,35 +260,78 @@ def mask_arg(mask: Optional[torch.Tensor], shape) -> tuple:
     return mask.contiguous(), dtype_code(mask.dtype)
 
 
-class HipWeightCache:
+def stamp(t: torch.Tensor) -> tuple:
+    """What changes with a tensor's storage, contents or layout (``data`` swaps leave the version
+    as it is). RuntimeError for an inference tensor, which carries no version counter."""
+    return (t.data_ptr(), t._version, t.shape, t.stride(), t.dtype, t.device)
+
+
+_expired = torch.UntypedStorage._expired
+
+
+class Storages:
+    """Weak references to the storages of tensors, as each was when the object was made. An address
+    means the same storage only while the old one is alive: after ``p.data = a; p.data = b`` the
+    parameter object and its version are the old ones, and ``b`` may sit where the first storage was.
+    (Weak, so that weights moved off the device free their memory.)"""
+
+    __slots__ = ("_refs",)
+
+    def __init__(self, tensors):
+        self._refs = [t.untyped_storage()._weak_ref() for t in tensors if t is not None]
+
+    def alive(self) -> bool:
+        return not any(map(_expired, self._refs))
+
+    def __del__(self, _free=torch.UntypedStorage._free_weak_ref):
+        for ref in self._refs:
+            _free(ref)
+
+
+class _Kept:
+    """One kept value and what it was made from, replaced as a whole (threads may share a module);
+    a copied or pickled one starts empty."""
+
+    def __init__(self):
+        self.clear()
+
+    def __reduce__(self):
+        return type(self), ()
+
+    @property
+    def _key(self):
+        return self._entry[0]
+
+    def clear(self):
+        self._entry = (None, None, None)
+
+    def lookup(self, key):
+        kept, storages, value = self._entry
+        return value if kept == key and storages.alive() else None
+
+    def keep(self, key, sources, value):
+        self._entry = (key, Storages(sources), value)
+        return value
+
+
+class HipWeightCache(_Kept):
     """Device copy of one weight in a compute dtype, re-made when the weight changes.
 
     Keyed like the reference ``GLUWeightCache`` (``gated_linear_unit.py:15-30``) on
-    (data_ptr, _version, shape, stride, dtype, device, compute dtype, layout); tensors
-    without a version counter (inference tensors) are never cached. ``layout`` is
-    ``"plain"`` (contiguous copy) or ``"glu"`` (the packed gate/value layout).
+    (data_ptr, _version, shape, stride, dtype, device, compute dtype, layout) and on the
+    storage (:class:`Storages`); tensors without a version counter (inference tensors) are
+    never cached. ``layout`` is ``"plain"`` (contiguous copy) or ``"glu"`` (the packed
+    gate/value layout).
     """
-
-    def __init__(self):
-        self._key = None
-        self._source = None
-        self._value = None
-
-    def clear(self):
-        self._key = self._source = self._value = None
 
     def get(self, weight: torch.Tensor, dtype: torch.dtype, layout: str = "plain") -> torch.Tensor:
         try:
-            version = weight._version
+            key = (*stamp(weight), dtype, layout)
         except RuntimeError:
             self.clear()
             return _prepare(weight, dtype, layout)
-        key = (weight.data_ptr(), version, weight.shape, weight.stride(), weight.dtype, weight.device, dtype, layout)
-        if self._key != key:
-            self._value = _prepare(weight, dtype, layout)
-            self._source = weight          # keeps the address from being reused
-            self._key = key
-        return self._value
+        value = self.lookup(key)
+        return value if value is not None else self.keep(key, [weight], _prepare(weight, dtype, layout))
 
 
 def _prepare(weight: torch.Tensor, dtype: torch.dtype, layout: str) -> torch.Tensor:
@@ -320,27 +363,19 @@ def linear_weight(module: torch.nn.Module, name: str, dtype: torch.dtype, layout
     return module_cache(module, name).get(getattr(module, name).weight, dtype, layout)
 
 
-class FusedWeightCache:
+class FusedWeightCache(_Kept):
     """Row-concatenation of several weights ([out_i, in] -> [sum out_i, in]) in one dtype,
     re-made when any source weight changes (same keys as :class:`HipWeightCache`)."""
 
-    def __init__(self):
-        self._key = None
-        self._sources = None
-        self._value = None
-
     def get(self, weights, dtype: torch.dtype) -> torch.Tensor:
+        build = lambda: torch.cat([w.detach().to(dtype) for w in weights], dim=0).contiguous()  # noqa: E731
         try:
-            key = tuple((w.data_ptr(), w._version, w.shape, w.stride(), w.dtype, w.device)
-                        for w in weights) + (dtype,)
+            key = (*map(stamp, weights), dtype)
         except RuntimeError:
-            self._key = self._sources = self._value = None
-            return torch.cat([w.detach().to(dtype) for w in weights], dim=0).contiguous()
-        if self._key != key:
-            self._value = torch.cat([w.detach().to(dtype) for w in weights], dim=0).contiguous()
-            self._sources = tuple(weights)
-            self._key = key
-        return self._value
+            self.clear()
+            return build()
+        value = self.lookup(key)
+        return value if value is not None else self.keep(key, weights, build())
 
 
 def fused_linear_weight(module: torch.nn.Module, names, dtype: torch.dtype) -> torch.Tensor:
@@ -352,27 +387,19 @@ def fused_linear_weight(module: torch.nn.Module, names, dtype: torch.dtype) -> t
     return cache.get([getattr(module, n).weight for n in names], dtype)
 
 
-class DerivedWeightCache:
+class DerivedWeightCache(_Kept):
     """A tensor built from several parameters by ``build(*sources)`` (a one-time weight
     preparation), re-made when any source changes (same keys as :class:`HipWeightCache`;
     never cached when a source is an inference tensor)."""
 
-    def __init__(self):
-        self._key = None
-        self._sources = None
-        self._value = None
-
     def get(self, sources, build):
         try:
-            key = tuple((t.data_ptr(), t._version, t.shape, t.stride(), t.dtype, t.device) for t in sources)
+            key = tuple(map(stamp, sources))
         except RuntimeError:
-            self._key = self._sources = self._value = None
+            self.clear()
             return build(*sources)
-        if self._key != key:
-            self._value = build(*sources)
-            self._sources = tuple(sources)
-            self._key = key
-        return self._value
+        value = self.lookup(key)
+        return value if value is not None else self.keep(key, sources, build(*sources))
 
 
 def derived_weight(module: torch.nn.Module, tag: str, sources, build):
@@ -412,14 +439,14 @@ def params(module: torch.nn.Module, names, norms=()) -> list:
 
 
 class WeightGroup:
-    """The prepared weights of one module call, checked as a whole: the same key per source as
-    :class:`HipWeightCache`, compared once. The sources are held, so no address of the key can
-    pass to another tensor; a copied or pickled module starts with an empty group."""
+    """The prepared weights of one module call, checked as a whole: the same key and storages per
+    source as :class:`HipWeightCache`, compared once. A copied or pickled module starts with an
+    empty group."""
 
-    __slots__ = ("key", "sources", "dtypes", "values")
+    __slots__ = ("key", "storages", "dtypes", "values")
 
     def __init__(self):
-        self.key = self.sources = self.dtypes = self.values = None
+        self.key = self.storages = self.dtypes = self.values = None
 
     def __reduce__(self):
         return WeightGroup, ()
@@ -442,15 +469,14 @@ def gather(module: torch.nn.Module, tag: str, sources, weights: int, x: torch.Te
         dtype = dtype or _compute_dtype(x.dtype, [p.dtype for p in sources[:weights]])
         return dtype, None if again else build(dtype)
     try:
-        key = [None if p is None else (p.data_ptr(), p._version, p.shape, p.stride(), p.dtype, p.device)
-               for p in sources]
+        key = [None if p is None else stamp(p) for p in sources]
     except RuntimeError:                             # inference tensors carry no version: nothing is kept
         dtype = dtype or _compute_dtype(x.dtype, [p.dtype for p in sources[:weights]])
         return dtype, None if again else build(dtype)
-    changed = group.key is not None and group.key != key
+    changed = group.key is not None and (group.key != key or not group.storages.alive())
     if changed or group.key is None:
         group = WeightGroup()
-        group.key, group.sources = key, sources
+        group.key, group.storages = key, Storages(sources)
         group.dtypes = {p.dtype for p in sources[:weights]}
         groups[tag] = group
     dtype = dtype or _compute_dtype(x.dtype, group.dtypes)

@@ -224,8 +224,7 @@ class AttentionOperands:
         self.gate = torch.empty((B, T, H * Dh), dtype=torch.bfloat16, device=device)
         self.words = torch.empty(B * (self.tpad // 64), dtype=torch.int64, device=device)
         self.words_shared = True
-        self._mask_key = ()
-        self._mask_ref = None
+        self._mask_key, self._mask_ref, self._mask_storage = (), None, nh.Storages([])
 
     @staticmethod
     def supported(T: int, H: int, Dh: int) -> bool:
@@ -237,10 +236,10 @@ class AttentionOperands:
     def set_mask(self, mask: Optional[torch.Tensor]) -> None:
         """Kept-key words of a key mask: None, [T] (shared by the samples) or [B, T]."""
         # Inference tensors carry no version counter: their words are recomputed every time.
-        # The mask of the cached words is held, so its address cannot pass to another tensor.
-        key = (None,) if mask is None else \
-            None if mask.is_inference() else (id(mask), mask.data_ptr(), mask._version, tuple(mask.shape), mask.dtype)
-        if key is not None and key == self._mask_key:
+        # Else the words stay while the mask is the same tensor (held, so that its id cannot pass to
+        # another), unchanged, on the same storage.
+        key = (None,) if mask is None else None if mask.is_inference() else (id(mask), *nh.stamp(mask))
+        if key is not None and key == self._mask_key and self._mask_storage.alive():
             return
         B, T = self.shape[0], self.shape[1]
         rows, code, m = 1, nh.BOOL, None
@@ -255,8 +254,7 @@ class AttentionOperands:
         nh.call("xfh_attention_mask_words", nh.ptr(m), code, T, rows, T, nh.ptr(self.words),
                 nh.stream_of(self.device))
         self.words_shared = rows == 1
-        self._mask_key = key
-        self._mask_ref = mask
+        self._mask_key, self._mask_ref, self._mask_storage = key, mask, nh.Storages([mask])
 
 
 _SHARED_OPERANDS: "collections.OrderedDict" = collections.OrderedDict()

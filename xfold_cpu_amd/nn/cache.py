@@ -17,8 +17,9 @@ Design (this module's own):
     shape, strides, dtype, device), plus a *context* tuple (the non-tensor leaves of the
     dependencies, the modules' ``eps`` and ``normalized_shape``, the autocast state of
     both device types and the backend switches). It is valid while every tensor passed now
-    is the very object it holds (``is``, so no id or address reuse can alias) with an
-    unchanged stamp, and the context compares equal. Holding the objects keeps them alive
+    is the very object it holds (``is``, so no id reuse can alias) with an unchanged stamp,
+    the storages it was computed from are alive (so no address has passed to another one by
+    ``.data`` swaps), and the context compares equal. Holding the objects keeps them alive
     for as long as the entry does.
   * A tensor without a version counter (created under ``torch.inference_mode``) cannot
     show an in-place update: it is accepted as an input feature, which the scope declares
@@ -41,6 +42,7 @@ import torch
 from torch.utils._pytree import tree_map
 
 from ..fastnn import config
+from ..fastnn.native_hip import Storages
 
 _ACTIVE: ContextVar[Optional["ExampleScope"]] = ContextVar("xfold_cpu_amd_example_scope", default=None)
 
@@ -148,6 +150,7 @@ class _Entry:
     value: Any
     held: Tuple[torch.Tensor, ...]            # dependency tensors, then parameters
     stamps: Tuple[tuple, ...]
+    storages: Storages
     context: tuple
     nbytes: int
 
@@ -163,7 +166,7 @@ class _Entry:
                 version = -1
             if (version, now.data_ptr(), tuple(now.shape), tuple(now.stride()), now.dtype, now.device) != stamp:
                 return False
-        return True
+        return self.storages.alive()
 
 
 def _members(owner: torch.nn.Module, modules) -> List[torch.nn.Module]:
@@ -229,7 +232,7 @@ class InputCache:
         except _Refused:
             return value
         if scope.charge(self, name, nbytes):
-            self._entries[name] = _Entry(scope, value, held, stamps, context, nbytes)
+            self._entries[name] = _Entry(scope, value, held, stamps, Storages(held), context, nbytes)
         return value if copy is None else copy(value)
 
 

@@ -124,15 +124,12 @@ def _projection_bias(module: nn.Module, c: int, parts: int, device: torch.device
     q_bias = module.q_projection.bias
     if q_bias is None:
         return None
-    cached = module.__dict__.get(f"_hip_proj_bias{parts}")
-    key = (q_bias.data_ptr(), q_bias._version) if not q_bias.is_inference() else None
-    if cached is None or key is None or cached[0] != key:
+
+    def build(bias):
         full = torch.zeros(parts * c, dtype=torch.float32, device=device)
-        full[:c] = q_bias.detach().to(torch.float32)
-        cached = (key, full)
-        if key is not None:
-            module.__dict__[f"_hip_proj_bias{parts}"] = cached
-    return cached[1]
+        full[:c] = bias.detach().to(torch.float32)
+        return full
+    return nh.derived_weight(module, f"projection_bias{parts}", [q_bias], build)
 
 
 def qkvg_weights(module: nn.Module, dtype: torch.dtype):
