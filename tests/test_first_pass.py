@@ -1,0 +1,116 @@
+"""What a module prepares of its weights, and when (CPU, the library's calls stubbed): everything on
+its first pass, so that a second pass may be a graph capture, and nothing that is made while a
+stream is captured outlives the call."""
+
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from xfold_cpu_amd import nn as hnn
+from xfold_cpu_amd.fastnn import native_hip as nh
+from xfold_cpu_amd.nn.cache import InputCache, input_cache_scope
+
+
+class Library:
+    def __getattr__(self, name):
+        return {"xfh_glu_packed_rows": lambda f: 2 * f, "xfh_attention_max_keys": lambda: 4096}.get(name, lambda *a: 256)
+
+
+def stub_call(name, *args):
+    if name == "xfh_attention_operands_size":
+        B, T, H, Dh, sizes = args
+        dp, tpad = 32 if Dh <= 32 else 64, (T + 63) // 64 * 64
+        sizes[:] = [dp, tpad, B * H * T * dp, B * H * tpad * dp, B * H * dp * tpad]
+
+
+@pytest.fixture
+def stubbed(monkeypatch):
+    library = Library()
+    monkeypatch.setattr(nh, "load_library", lambda path=None: library)
+    monkeypatch.setattr(nh, "attention_max_keys", lambda: 4096)
+    monkeypatch.setattr(nh, "call", stub_call)
+    monkeypatch.setattr(nh, "ptr", lambda t: None if t is None else t.data_ptr())
+    monkeypatch.setattr(nh, "stream_of", lambda device: 0)
+    monkeypatch.setattr(nh, "check_gpu_inference", lambda *tensors: None)
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda device="cuda": True)
+    monkeypatch.setattr(torch, "get_autocast_dtype", lambda device="cuda": torch.bfloat16)
+
+
+def bf16(*shape):
+    return torch.randn(shape).bfloat16()
+
+
+MODULES = {
+    "diffusion_transition": (lambda: hnn.DiffusionTransition(64, 32, use_single_cond=True),
+                             lambda: (bf16(5, 64), bf16(5, 32))),
+    "self_attention": (lambda: hnn.SelfAttention(c_x=64, num_head=2, c_single_cond=32, use_single_cond=True),
+                       lambda: (bf16(5, 64), torch.ones(5), bf16(2, 5, 5), bf16(5, 32))),
+    "cross_attention": (lambda: hnn.CrossAttention(key_dim=64, value_dim=64, c_single_cond=64, num_head=2),
+                        lambda: (bf16(3, 4, 64), bf16(3, 6, 64), torch.ones(3, 4), torch.ones(3, 6), bf16(3, 2, 4, 6),
+                                 bf16(3, 4, 64), bf16(3, 6, 64))),
+    "cross_attention_fused": (hnn.CrossAttention,
+                              lambda: (bf16(3, 4, 128), bf16(3, 6, 128), torch.ones(3, 4), torch.ones(3, 6),
+                                       bf16(3, 4, 4, 6), bf16(3, 4, 128), bf16(3, 6, 128))),
+    "pairformer": (lambda: hnn.PairformerBlock(c_single=64), lambda: (bf16(5, 5, 128), torch.ones(5, 5), bf16(5, 64),
+                                                                     torch.ones(5))),
+    "evoformer": (hnn.EvoformerBlock, lambda: (bf16(3, 5, 64), bf16(5, 5, 128), torch.ones(3, 5), torch.ones(5, 5))),
+    "diffusion_transformer": (lambda: hnn.DiffusionTransformer(c_act=64, c_single_cond=32, num_head=16, num_blocks=4,
+                                                               super_block_size=2),
+                              lambda: (bf16(2, 5, 64), torch.ones(5), bf16(5, 32), bf16(5, 5, 128))),
+}
+
+
+class Computed(TorchDispatchMode):
+    """The operators that write new memory."""
+
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        if not func.is_view and "empty" not in func.name():
+            self.names.append(func.name())
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("kind", MODULES)
+def test_the_first_pass_prepares_every_weight(stubbed, kind):
+    make, inputs = MODULES[kind]
+    module, args, passes = make().eval(), inputs(), []
+    with torch.inference_mode(False), torch.no_grad():
+        for _ in range(3):
+            with Computed() as computed:
+                module(*args)
+            passes.append(computed.names)
+    assert passes[0] and passes[1] == passes[2]
+
+
+@pytest.mark.parametrize("kind", MODULES)
+def test_nothing_made_in_a_capture_is_kept(stubbed, monkeypatch, kind):
+    make, inputs = MODULES[kind]
+    module, args = make().eval(), inputs()
+    with torch.no_grad():
+        monkeypatch.setattr(nh, "capturing", lambda: True)
+        module(*args)
+        module(*args)
+        for m in module.modules():
+            assert all(c._key is None for c in m.__dict__.get("_hip_weight_caches", {}).values())
+            assert all(g.values is None for g in m.__dict__.get("_hip_weight_groups", {}).values())
+        monkeypatch.setattr(nh, "capturing", lambda: False)
+        module(*args)
+        assert any(c._key is not None for m in module.modules() for c in m.__dict__.get("_hip_weight_caches", {}).values())
+
+
+def test_a_memo_entry_is_not_made_in_a_capture(monkeypatch):
+    from xfold_cpu_amd.fastnn import config
+    from xfold_cpu_amd.nn import cache as cache_module
+    monkeypatch.setattr(config, "input_cache_enabled", True)
+    owner, cache, feature = torch.nn.Linear(3, 3).eval(), InputCache(), torch.randn(2, 3)
+    with torch.no_grad(), input_cache_scope():
+        monkeypatch.setattr(cache_module, "capturing", lambda: True)
+        cache.get("x", (feature,), owner, lambda: owner(feature))
+        assert not cache._entries
+        monkeypatch.setattr(cache_module, "capturing", lambda: False)
+        kept = cache.get("x", (feature,), owner, lambda: owner(feature))
+        monkeypatch.setattr(cache_module, "capturing", lambda: True)
+        assert cache.get("x", (feature,), owner, lambda: owner(feature)) is kept

@@ -113,3 +113,46 @@ def test_diffusion_transformer_graph_replay(device):
         reset()
         graph = capture(forward)
         replay_and_check(graph, reset, (out["act"],), (want,))
+
+
+def linear_inputs(kind, n, device):
+    """A module's inputs at n tokens, one of them updated in place or none."""
+    g = torch.Generator().manual_seed(n)
+    randn = lambda *s: torch.randn(s, generator=g).to(device)  # noqa: E731
+    if kind == "DiffusionTransition":
+        return randn(2, n, 256), randn(n, 64)
+    if kind == "SelfAttention":
+        return randn(2, n, 256), torch.ones(n, device=device), randn(16, n, n), randn(n, 64)
+    return (randn(3, n, 128), randn(3, 2 * n, 128), torch.ones(3, n, device=device), torch.ones(3, 2 * n, device=device),
+            randn(3, 4, n, 2 * n), randn(3, n, 128), randn(3, 2 * n, 128))
+
+
+@pytest.mark.parametrize("kind,args,bf16", [
+    ("DiffusionTransition", dict(c_x=256, c_single_cond=64, use_single_cond=True), True),
+    ("SelfAttention", dict(c_x=256, num_head=16, c_single_cond=64, use_single_cond=True), True),
+    ("CrossAttention", dict(), False), ("CrossAttention", dict(), True)])
+def test_capture_after_one_eager_pass(device, kind, args, bf16):
+    """One eager pass, then two captures of other lengths: the eager module before the first replay, and
+    the second graph replayed before the first, equal the eager results of a module of its own."""
+    announce("graph after one pass", kind, bf16)
+    _, twin = pair_of(kind, args, seed=3, device=device)
+    _, hip = pair_of(kind, args, seed=3, device=device)
+    inputs = [linear_inputs(kind, n, device) for n in (33, 48, 20)]
+    with torch.inference_mode(), autocast(bf16):
+        wants = [twin(*i).clone() for i in inputs]
+        hip(*inputs[0])
+        torch.cuda.synchronize()
+        graphs, outs = [], []
+        for i in inputs[1:]:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                outs.append(hip(*i))
+            graphs.append(graph)
+        assert torch.equal(hip(*inputs[0]), wants[0])
+        for _ in range(3):
+            for k in (1, 0):
+                outs[k].zero_()
+                graphs[k].replay()
+                torch.cuda.synchronize()
+                assert torch.equal(outs[k], wants[1 + k])
+                assert torch.equal(hip(*inputs[0]), wants[0])

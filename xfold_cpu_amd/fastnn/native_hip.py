@@ -288,6 +288,12 @@ class Storages:
             _free(ref)
 
 
+def capturing() -> bool:
+    """Whether the current stream records a graph. What is prepared then lives in the graph's memory
+    and is written by its replays only: it serves the capture and is not kept."""
+    return torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing()
+
+
 class _Kept:
     """One kept value and what it was made from, replaced as a whole (threads may share a module);
     a copied or pickled one starts empty."""
@@ -310,7 +316,8 @@ class _Kept:
         return value if kept == key and storages.alive() else None
 
     def keep(self, key, sources, value):
-        self._entry = (key, Storages(sources), value)
+        if not capturing():
+            self._entry = (key, Storages(sources), value)
         return value
 
 
@@ -461,7 +468,9 @@ def gather(module: torch.nn.Module, tag: str, sources, weights: int, x: torch.Te
     The first pass over a module keeps nothing and takes no key: its weights are being prepared
     (each in its own cache) while the GPU waits. ``again``: the values are None on that pass and
     on the first one after a change, when a whole block's weights are prepared operator by
-    operator behind the operators already queued; the block's one call starts with the next."""
+    operator behind the operators already queued; the block's one call starts with the next.
+    Its ``build`` only collects what the operators prepared: a capture may be that next pass,
+    and what it makes is not kept (:func:`capturing`)."""
     groups = module.__dict__.setdefault("_hip_weight_groups", {})
     group = groups.get(tag)
     if group is None:
@@ -484,7 +493,9 @@ def gather(module: torch.nn.Module, tag: str, sources, weights: int, x: torch.Te
     if values is None or values[0] != dtype:
         if again and changed:
             return dtype, None
-        values = group.values = (dtype, build(dtype))
+        values = (dtype, build(dtype))
+        if not capturing():
+            group.values = values
     return values
 
 

@@ -29,7 +29,8 @@ Design (this module's own):
     budget is returned without being kept. Closing the scope, normally or by an exception,
     releases every entry it paid for.
   * Nothing is kept outside a scope, with grad mode on, or while the owner or a listed
-    module is training; such a call also drops what the cache held.
+    module is training; such a call also drops what the cache held. A value made while the
+    stream records a graph is not kept either: only the graph's replays write it.
 """
 
 from __future__ import annotations
@@ -42,7 +43,7 @@ import torch
 from torch.utils._pytree import tree_map
 
 from ..fastnn import config
-from ..fastnn.native_hip import Storages
+from ..fastnn.native_hip import Storages, capturing
 
 _ACTIVE: ContextVar[Optional["ExampleScope"]] = ContextVar("xfold_cpu_amd_example_scope", default=None)
 
@@ -231,7 +232,7 @@ class InputCache:
             nbytes = _storage_footprint(value)
         except _Refused:
             return value
-        if scope.charge(self, name, nbytes):
+        if not capturing() and scope.charge(self, name, nbytes):
             self._entries[name] = _Entry(scope, value, held, stamps, Storages(held), context, nbytes)
         return value if copy is None else copy(value)
 

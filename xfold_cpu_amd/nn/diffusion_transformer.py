@@ -16,6 +16,7 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
 
 from ..fastnn import LayerNorm
 from ..fastnn import config as fastnn_config
@@ -44,25 +45,20 @@ def _adaptive_layer_norm(aln: nn.Module, x: torch.Tensor, single_cond: Optional[
     cond = ops.layer_norm(single_cond, cln.normalized_shape, nh.param(aln, "single_cond_layer_norm"),
                           nh.param(aln, "single_cond_layer_norm", "bias"), cln.eps, out_dtype=dtype, owner=cln)
     # scale and shift stay fp32 (one rounding fewer before the sigmoid and the add); one launch
-    # over the stacked weights from the second pass on.
-    _, stacked = nh.gather(aln, "scale_shift", sources, 0, x, lambda dt: _scale_shift_weights(sources, dt), dtype,
-                           again=True)
-    if stacked is not None:
-        scale, shift = ops.linear_batched(cond.reshape(-1, cond.shape[-1]), *stacked, dtype, out_dtype=torch.float32)
-    else:
-        scale, shift = (ops.linear(cond, w.detach().to(dtype).contiguous(), b, dtype, out_dtype=torch.float32)
-                        for w, b in ((sources[0], sources[2]), (sources[1], None)))
+    # over the stacked weights, made on the first pass (the next one may be a graph capture).
+    w, b = nh.derived_weight(aln, f"scale_shift:{dtype}", [t for t in sources if t is not None],
+                             lambda *ts: _scale_shift_weights(dtype, *ts))
+    scale, shift = ops.linear_batched(cond.reshape(-1, cond.shape[-1]), w, b, dtype, out_dtype=torch.float32)
     return ops.adaptive_layer_norm(x, scale, shift, aln.layer_norm.eps, out_dtype=out_dtype)
 
 
-def _scale_shift_weights(sources, dtype: torch.dtype):
+def _scale_shift_weights(dtype: torch.dtype, scale: torch.Tensor, shift: torch.Tensor,
+                         bias: Optional[torch.Tensor] = None):
     """single_cond_scale and single_cond_bias as one [2, c, c_cond] weight in ``dtype`` and their
-    [2, c] fp32 bias (zeros for single_cond_bias, which has none)."""
-    scale, shift, bias = (None if t is None else t.detach() for t in sources)
-    b = torch.zeros((2, scale.shape[0]), dtype=torch.float32, device=scale.device)
-    if bias is not None:
-        b[0] = bias
-    return torch.stack([scale.to(dtype), shift.to(dtype)]), b
+    [2, c] fp32 bias (zeros for single_cond_bias, which has none; None without a bias)."""
+    c, k = scale.shape
+    w = torch.cat([scale.detach(), shift.detach()]).to(dtype).view(2, c, k)
+    return w, None if bias is None else F.pad(bias.detach().float(), (0, c)).view(2, c)
 
 
 def _ada_ln_zero(zero: nn.Module, hidden: torch.Tensor, single_cond: Optional[torch.Tensor],
