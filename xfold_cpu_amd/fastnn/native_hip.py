@@ -288,10 +288,10 @@ class Storages:
             _free(ref)
 
 
-def capturing() -> bool:
+def capturing(_stream_capturing=torch._C._cuda_isCurrentStreamCapturing) -> bool:
     """Whether the current stream records a graph. What is prepared then lives in the graph's memory
     and is written by its replays only: it serves the capture and is not kept."""
-    return torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing()
+    return torch.cuda.is_initialized() and _stream_capturing()
 
 
 class _Kept:
@@ -367,7 +367,7 @@ def module_cache(module: torch.nn.Module, name: str) -> HipWeightCache:
 
 def linear_weight(module: torch.nn.Module, name: str, dtype: torch.dtype, layout: str = "plain"):
     """Device copy of ``module.<name>.weight`` ([out, in]) in ``dtype``."""
-    return module_cache(module, name).get(getattr(module, name).weight, dtype, layout)
+    return module_cache(module, name).get(param(module, name), dtype, layout)
 
 
 class FusedWeightCache(_Kept):
@@ -391,7 +391,7 @@ def fused_linear_weight(module: torch.nn.Module, names, dtype: torch.dtype) -> t
     cache = caches.get(tag)
     if cache is None:
         cache = caches[tag] = FusedWeightCache()
-    return cache.get([getattr(module, n).weight for n in names], dtype)
+    return cache.get([param(module, n) for n in names], dtype)
 
 
 class DerivedWeightCache(_Kept):
