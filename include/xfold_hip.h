@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define XFH_ABI_VERSION 10
+#define XFH_ABI_VERSION 11
 
 enum { XFH_F32 = 0, XFH_BF16 = 1, XFH_BOOL = 2 };
 enum { XFH_OK = 0, XFH_EINVAL = 1, XFH_EUNSUPPORTED = 2, XFH_EWORKSPACE = 3, XFH_EHIP = 4 };
@@ -166,6 +166,11 @@ int xfh_attention_bias_pack(const void *bias, int dtype, const int64_t *shape, c
  * sizes[0..4] = {Dp, Tpad, q elements, k elements, vt elements}; XFH_EUNSUPPORTED for other
  * head dims or token counts. */
 int xfh_attention_operands_size(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t *sizes);
+
+/* *id = the id of the graph capture that the stream is recording, 0 when it records none. Buffers that
+ * are cleared once and reused (the operands above) belong to one capture: the clearing is recorded
+ * in its graph. */
+int xfh_stream_capture_id(void *stream, uint64_t *id);
 
 /* [q | k | v (| gate)] = x w^T + bias in one bf16 GEMM, straight into those layouts:
  * x [B*T][K] bf16 (row stride ldx), w [N][K] bf16 = the stacked projection weights

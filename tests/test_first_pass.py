@@ -114,3 +114,22 @@ def test_a_memo_entry_is_not_made_in_a_capture(monkeypatch):
         kept = cache.get("x", (feature,), owner, lambda: owner(feature))
         monkeypatch.setattr(cache_module, "capturing", lambda: True)
         assert cache.get("x", (feature,), owner, lambda: owner(feature)) is kept
+
+
+def test_each_capture_has_attention_operands_of_its_own(stubbed, monkeypatch):
+    """The buffers' zero fill and mask words are recorded in the graph that makes them."""
+    from xfold_cpu_amd.fastnn import ops
+    monkeypatch.setattr(ops, "_SHARED_OPERANDS", type(ops._SHARED_OPERANDS)())
+    capture = 0
+    monkeypatch.setattr(nh, "capture_id", lambda device: capture, raising=False)
+    get = lambda T=40: ops.shared_attention_operands(1, T, 4, 32, torch.device("cpu"))  # noqa: E731
+    eager = get()
+    capture = 7
+    first = get()
+    assert first is not eager and get() is first and get(50) is not first
+    capture = 8
+    second = get()
+    assert second is not first and second is not eager and get() is second
+    capture = 0
+    assert get() is eager
+    assert [k[-1] for k in ops._SHARED_OPERANDS] == [0]      # the captures' sets are given back

@@ -156,3 +156,36 @@ def test_capture_after_one_eager_pass(device, kind, args, bf16):
                 torch.cuda.synchronize()
                 assert torch.equal(outs[k], wants[1 + k])
                 assert torch.equal(hip(*inputs[0]), wants[0])
+
+
+def test_graphs_of_one_shape_share_no_buffers(device):
+    """Two captures of one shape and mask: the second is replayed before the first, then eager calls with
+    another mask run between the replays on the captures' own stream."""
+    announce("graphs of one shape")
+    args = dict(c_act=256, c_single_cond=64, c_pair_cond=128, num_head=16, num_blocks=4, super_block_size=2)
+    _, hip = pair_of("DiffusionTransformer", args, seed=6, device=device)
+    torch.manual_seed(6)
+    n = 40
+    acts = [torch.randn(2, n, 256).to(device) for _ in range(2)]
+    masks = [torch.ones(n, device=device), (torch.arange(n, device=device) % 3 > 0).float()]
+    scond, pcond = torch.randn(n, 64).to(device), torch.randn(n, n, 128).to(device)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.inference_mode(), autocast(True), torch.cuda.stream(stream):
+        run = lambda act, mask: hip(act.clone(), mask, scond, pcond)  # noqa: E731
+        run(acts[0], masks[0])
+        wants = [[run(a, m) for m in masks] for a in acts]
+        torch.cuda.synchronize()
+        graphs, outs = [], []
+        for act in acts:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                outs.append(run(act, masks[0]))
+            graphs.append(graph)
+        for _ in range(3):
+            for k in (1, 0):
+                outs[k].zero_()
+                graphs[k].replay()
+                torch.cuda.synchronize()
+                assert torch.equal(outs[k], wants[k][0])
+                assert torch.equal(run(acts[k], masks[1]), wants[k][1])

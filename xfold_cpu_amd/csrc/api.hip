@@ -409,6 +409,16 @@ int xfh_attention_operands_size(int64_t B, int64_t T, int64_t H, int64_t Dh, int
   return XFH_OK;
 }
 
+int xfh_stream_capture_id(void *stream, uint64_t *id) {
+  XFH_REQUIRE(id, "stream_capture_id: null argument");
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long capture = 0;
+  const hipError_t err = hipStreamGetCaptureInfo(as_stream(stream), &status, &capture);
+  if (err != hipSuccess) return fail(XFH_EHIP, std::string("stream_capture_id: ") + hipGetErrorString(err));
+  *id = status == hipStreamCaptureStatusNone ? 0 : capture;
+  return XFH_OK;
+}
+
 int xfh_attention_project(const void *x, int64_t ldx, const void *w, const float *bias, int64_t B, int64_t T,
                           int64_t K, int64_t H, int64_t Dh, float qscale, void *q, void *k, void *vt, void *gate,
                           void *stream) {

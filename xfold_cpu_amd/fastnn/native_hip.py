@@ -28,7 +28,7 @@ from typing import Optional
 import torch
 
 LIBRARY_PATH = Path(__file__).resolve().parent.parent / "lib" / "libxfold_hip.so"
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 F32, BF16, BOOL = 0, 1, 2
 BIAS_PACKED = 3                 # bias 'dtype' of a packed fp32 block (times log2(e))
@@ -59,6 +59,7 @@ SIGNATURES = {
     "xfh_attention_max_keys": (_i64, []),
     "xfh_attention_bias_pack": (_i, [_p, _i, _pi64, _pi64, _p, _p]),
     "xfh_attention_operands_size": (_i, [_i64, _i64, _i64, _i64, _pi64]),
+    "xfh_stream_capture_id": (_i, [_p, ctypes.POINTER(ctypes.c_uint64)]),
     "xfh_attention_project": (_i, [_p, _i64, _p, _p, _i64, _i64, _i64, _i64, _i64, _f, _p, _p, _p, _p, _p]),
     "xfh_attention_mask_words": (_i, [_p, _i, _i64, _i64, _i64, _p, _p]),
     "xfh_attention_operands": (_i, [_p, _p, _p, _p, _i, _p, _i, _p, _p, _i64, _i64, _i64, _i64, _p]),
@@ -240,6 +241,15 @@ def stream_of(device: torch.device) -> int:
     """The current stream of ``device`` as a raw hipStream_t."""
     index = device.index if device.index is not None else torch.cuda.current_device()
     return torch._C._cuda_getCurrentRawStream(index)
+
+
+def capture_id(device: torch.device) -> int:
+    """The id of the graph capture that the current stream records, 0 when it records none."""
+    if not capturing():
+        return 0
+    value = ctypes.c_uint64()
+    call("xfh_stream_capture_id", stream_of(device), ctypes.byref(value))
+    return value.value
 
 
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:

@@ -263,14 +263,20 @@ _SHARED_OPERANDS_LOCK = threading.Lock()
 
 
 def shared_attention_operands(B: int, T: int, H: int, Dh: int, device: torch.device) -> AttentionOperands:
-    """One :class:`AttentionOperands` set per (shape, device, current stream, thread), kept
-    between calls: work queued on one stream runs in order, so every attention call of that
+    """One :class:`AttentionOperands` set per (shape, device, current stream, thread, graph capture),
+    kept between calls: work queued on one stream runs in order, so every attention call of that
     stream can reuse the same buffers (zeroed once, padding never written) instead of
-    allocating and zero-filling its own. The least recently used of more than 8 sets is
-    released (the caching allocator keeps it from reuse until the queued work is done)."""
+    allocating and zero-filling its own. A capture has sets of its own: their zero fill and mask words
+    are recorded in its graph, and another graph or an eager call must not rely on its replays.
+    They leave the table with the thread's next call outside that capture. The least recently used
+    of more than 8 sets is released (the caching allocator keeps it from reuse until the queued
+    work is done)."""
     device = torch.device(device)
-    key = (B, T, H, Dh, device, nh.stream_of(device), threading.get_ident())
+    thread, capture = threading.get_ident(), nh.capture_id(device)
+    key = (B, T, H, Dh, device, nh.stream_of(device), thread, capture)
     with _SHARED_OPERANDS_LOCK:                  # one table for every host thread
+        for other in [k for k in _SHARED_OPERANDS if k[-1] not in (0, capture) and k[-2] == thread]:
+            del _SHARED_OPERANDS[other]
         ops_ = _SHARED_OPERANDS.pop(key, None)
         if ops_ is None:
             ops_ = AttentionOperands(B, T, H, Dh, device)
