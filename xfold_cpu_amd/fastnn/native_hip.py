@@ -318,6 +318,10 @@ class _Kept:
     def _key(self):
         return self._entry[0]
 
+    @property
+    def _value(self):
+        return self._entry[2]
+
     def clear(self):
         self._entry = (None, None, None)
 
