@@ -885,6 +885,53 @@ def test_gemm_fp32(device, m, k, n, kind):
     assert_parity(got, want, TOL_FP32, f"gemm fp32 {kind} {m}x{k}->{n}")
 
 
+@pytest.mark.parametrize("m,k,n", [(33, 64, 35), (129, 72, 130), (700, 40, 65)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["linear", "glu", "accumulate"])
+def test_gemm_wide_loads_with_unaligned_output_rows(device, m, k, n, dtype, kind):
+    """Aligned operands are loaded 16 bytes at a time whatever the output's rows are."""
+    announce("gemm loads", m, k, n, dtype, kind)
+    g = torch.Generator().manual_seed(m + k + n)
+    x = torch.randn(m, k, generator=g).to(dtype)
+    w = (torch.randn(n, k, generator=g) / math.sqrt(k)).to(dtype)
+    out = torch.zeros(m * n + 1, device=device)[1:].view(m, n)    # fp32 rows off their 16 bytes
+    nh.kernel_timing_read("gemm_nt"), nh.kernel_timing_read("gemm_nt_elements")
+    nh.set_kernel_timing(True)
+    if kind == "glu":
+        f = n // 2 if n // 2 % 4 else n // 2 - 1
+        packed = nh._prepare(w[:2 * f].to(device), dtype, "glu")
+        got, want = ops.gated_linear_unit(x.to(device), packed, f, dtype, out_dtype=torch.float32), \
+            R.gated_linear_unit(x.float(), w[:2 * f].float().T)
+    elif kind == "linear":
+        bias = torch.randn(n, generator=g)
+        got, want = ops.linear(x.to(device), w.to(device), bias.to(device), dtype, out=out), \
+            x.float() @ w.float().T + bias
+    else:
+        start, aux = torch.randn(m, n, generator=g), torch.randn(m, n, generator=g)
+        got = ops.linear(x.to(device), w.to(device), None, dtype, out=out.copy_(start),
+                         epilogue=nh.EPI_MUL_SIGMOID_AUX_ACCUMULATE, aux=aux.to(device))
+        want = start + x.float() @ w.float().T * torch.sigmoid(aux)
+    torch.cuda.synchronize()
+    nh.set_kernel_timing(False)
+    assert nh.kernel_timing_read("gemm_nt_elements")[1] == 0 and nh.kernel_timing_read("gemm_nt")[1] == 1
+    assert_parity(got, want, TOL_FP32, f"gemm loads {kind} {m}x{k}->{n}")
+
+
+@pytest.mark.parametrize("n", [65, 98, 100])
+def test_grid_attention_fp32_bias_product(device, n):
+    """The fp32 bias product, [heads][n n], keeps its wide loads where its rows are odd."""
+    announce("grid fp32 bias", n)
+    ref, hip = pair_of("GridSelfAttention", dict(c_pair=64, num_head=4, transpose=True), seed=n)
+    pair, mask = torch.randn(n, n, 64, generator=torch.Generator().manual_seed(n)), torch.ones(n, n)
+    mask[:, -2:] = 0
+    nh.kernel_timing_read("gemm_nt_elements")
+    nh.set_kernel_timing(True)
+    check_module(ref, hip, hnn.grid_self_attention_hip, (pair, mask), (pair.to(device), mask.to(device)), False, "grid fp32")
+    torch.cuda.synchronize()
+    nh.set_kernel_timing(False)
+    assert nh.kernel_timing_read("gemm_nt_elements")[1] == 0
+
+
 def test_gemm_fp32_more_rows_than_a_grid_of_small_tiles(device):
     """65535 tiles of 64 rows and one more: the 128 x 128 tiles take over."""
     m = 65535 * 64 + 1

@@ -10,9 +10,9 @@
 // per CU, and fp32, take 64 x 64 tiles (32 x 32 per wavefront) instead, four times as many
 // workgroups. Global -> register prefetch of the next k-step overlaps the MFMAs of the current
 // one; LDS rows are padded by 16 bytes so the 16 rows a fragment read touches fall in distinct
-// banks. Aligned operands (VEC) take the vector
-// epilogue of gemm_epilogue.h: the per-element one, with its divisions and its switch, is ten
-// times the main loop's code and cost 2 us a launch.
+// banks. Aligned operands (VEC) are loaded 16 bytes at a time; with an output that takes four
+// columns in one access too (VECOUT) the epilogue is gemm_epilogue.h's: the per-element one, with
+// its divisions and its switch, is ten times the main loop's code and cost 2 us a launch.
 #include <type_traits>
 
 #include "common.h"
@@ -77,7 +77,7 @@ __device__ __forceinline__ float apply_epilogue(int epi, float acc, TO *c, const
 }
 
 // BT x BT block tile (BT = 128 or 64), each wavefront BT/2 x BT/2 = TW x TW MFMA tiles.
-template <typename T, typename TO, bool VEC, bool GLU, int BT>
+template <typename T, typename TO, bool VEC, bool VECOUT, bool GLU, int BT>
 __global__ __launch_bounds__(THREADS) void gemm_nt_kernel(GemmArgs p) {
   constexpr int BM = BT, BN = BT, WT = BT / 2, TW = WT / 16;
   typedef GemmSmem<T, BT> Smem;
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(THREADS) void gemm_nt_kernel(GemmArgs p) {
   const T *B = static_cast<const T *>(p.B) + batch * p.sB + int64_t(n0) * p.ldb;
   const int rowsA = p.M - m0, rowsB = p.N - n0;
 
-  // acc[j][i]: output tile (row tile i, column tile j); with VEC a lane holds four consecutive
+  // acc[j][i]: output tile (row tile i, column tile j); with VECOUT a lane holds four consecutive
   // columns of a row (the B rows as the MFMA's A operand), else four rows of a column.
   f32x4 acc[TW][TW];
 #pragma unroll
@@ -133,26 +133,23 @@ __global__ __launch_bounds__(THREADS) void gemm_nt_kernel(GemmArgs p) {
     stash();
     __syncthreads();
     if (k0 + BK < p.K) fetch(k0 + BK);
+    typename Frag<T>::type fa[TW], fb[TW];
 #pragma unroll
-    for (int ks = 0; ks < BK; ks += 32) {
-      typename Frag<T>::type fa[TW], fb[TW];
+    for (int i = 0; i < TW; ++i) fa[i] = read_frag<T>(&smem.a[(wm * WT + i * 16 + fr) * kPitch + fk]);
 #pragma unroll
-      for (int i = 0; i < TW; ++i) fa[i] = read_frag<T>(&smem.a[(wm * WT + i * 16 + fr) * kPitch + ks + fk]);
+    for (int j = 0; j < TW; ++j) fb[j] = read_frag<T>(&smem.b[(wn * WT + j * 16 + fr) * kPitch + fk]);
+    if constexpr (VECOUT) {
+      mfma_tiles(fb, fa, acc);
+    } else {
 #pragma unroll
-      for (int j = 0; j < TW; ++j) fb[j] = read_frag<T>(&smem.b[(wn * WT + j * 16 + fr) * kPitch + ks + fk]);
-      if constexpr (VEC) {
-        mfma_tiles(fb, fa, acc);
-      } else {
+      for (int i = 0; i < TW; ++i)
 #pragma unroll
-        for (int i = 0; i < TW; ++i)
-#pragma unroll
-          for (int j = 0; j < TW; ++j) acc[j][i] = mfma16(fa[i], fb[j], acc[j][i]);
-      }
+        for (int j = 0; j < TW; ++j) acc[j][i] = mfma16(fa[i], fb[j], acc[j][i]);
     }
   }
 
   TO *C = static_cast<TO *>(p.C) + batch * p.sC;
-  if constexpr (VEC) {
+  if constexpr (VECOUT) {
     const int mw = m0 + wm * WT, nw = n0 + wn * WT, col = lane & 15, grp = lane >> 4;
     if constexpr (GLU) {
 #pragma unroll
@@ -225,13 +222,28 @@ __global__ __launch_bounds__(THREADS) void gemm_nt_kernel(GemmArgs p) {
   }
 }
 
+template <typename T, typename TO, int BT>
+void launch_tiles(const GemmArgs &p, int64_t batch, bool glu, bool vec, bool vecout, KernelTimer &timer) {
+  const dim3 grid(ceil_div(p.N, BT), ceil_div(p.M, BT), batch), block(THREADS);
+  auto go = [&](auto v, auto o) {
+    constexpr bool V = decltype(v)::value, O = decltype(o)::value;
+    if (glu) timer.launch(gemm_nt_kernel<T, TO, V, O, true, BT>, grid, block, 0, p);
+    else timer.launch(gemm_nt_kernel<T, TO, V, O, false, BT>, grid, block, 0, p);
+  };
+  if (vec && vecout) go(std::true_type(), std::true_type());
+  else if (vec) go(std::true_type(), std::false_type());
+  else go(std::false_type(), std::false_type());
+}
+
+// Operand loads and the epilogue are wide each by its own alignment: an output row off four columns
+// (a [n][n] product at odd n) says nothing about the rows that are read.
 template <typename T, typename TO>
 int launch_typed(const GemmArgs &p, int64_t batch, bool glu, hipStream_t s) {
   constexpr int kChunk = 16 / sizeof(T);
   const bool vec = (p.K % kChunk == 0) && (p.lda % kChunk == 0) && (p.ldb % kChunk == 0) &&
                    (p.sA % kChunk == 0) && (p.sB % kChunk == 0) &&
                    (reinterpret_cast<uintptr_t>(p.A) % 16 == 0) &&
-                   (reinterpret_cast<uintptr_t>(p.B) % 16 == 0) && vector_output(p, sizeof(TO));
+                   (reinterpret_cast<uintptr_t>(p.B) % 16 == 0);
   int cus = 0;
   XFH_TRY(device_cu_count(&cus));
   // fp32 takes 64 x 64 tiles: a 128 x 128 tile's fragments leave one wavefront per SIMD
@@ -239,25 +251,11 @@ int launch_typed(const GemmArgs &p, int64_t batch, bool glu, hipStream_t s) {
   // 64-row tiles can hold (M > 4194240) keep the larger ones.
   const bool small = (std::is_same<T, float>::value && ceil_div(p.M, int64_t(64)) <= 65535) ||
                      ceil_div(p.N, int64_t(128)) * ceil_div(p.M, int64_t(128)) * batch < 2 * int64_t(cus);
-  if (small) {
-    dim3 grid(ceil_div(p.N, 64), ceil_div(p.M, 64), batch);
-    if (glu) {
-      if (vec) gemm_nt_kernel<T, TO, true, true, 64><<<grid, THREADS, 0, s>>>(p);
-      else gemm_nt_kernel<T, TO, false, true, 64><<<grid, THREADS, 0, s>>>(p);
-    } else {
-      if (vec) gemm_nt_kernel<T, TO, true, false, 64><<<grid, THREADS, 0, s>>>(p);
-      else gemm_nt_kernel<T, TO, false, false, 64><<<grid, THREADS, 0, s>>>(p);
-    }
-    return check_launch("gemm_nt");
-  }
-  dim3 grid(ceil_div(p.N, 128), ceil_div(p.M, 128), batch);
-  if (glu) {
-    if (vec) gemm_nt_kernel<T, TO, true, true, 128><<<grid, THREADS, 0, s>>>(p);
-    else gemm_nt_kernel<T, TO, false, true, 128><<<grid, THREADS, 0, s>>>(p);
-  } else {
-    if (vec) gemm_nt_kernel<T, TO, true, false, 128><<<grid, THREADS, 0, s>>>(p);
-    else gemm_nt_kernel<T, TO, false, false, 128><<<grid, THREADS, 0, s>>>(p);
-  }
+  KernelTimer timer(vec ? "gemm_nt" : "gemm_nt_elements", s,
+                    2.0 * double(p.M) * double(p.N) * double(p.K) * double(batch), true);
+  const bool vecout = vector_output(p, sizeof(TO));
+  if (small) launch_tiles<T, TO, 64>(p, batch, glu, vec, vecout, timer);
+  else launch_tiles<T, TO, 128>(p, batch, glu, vec, vecout, timer);
   return check_launch("gemm_nt");
 }
 
