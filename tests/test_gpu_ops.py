@@ -461,6 +461,22 @@ def test_pair_operators_at_64_channels(device, n):
             assert_parity_bf16(hip(odd, *dev), want, f"{name} c=64 unaligned", floor=bf16_stored(floor))
 
 
+@pytest.mark.parametrize("name,args", [("TriangleMultiplication", dict(_outgoing=True)),
+                                       ("GridSelfAttention", dict(num_head=4, transpose=True))])
+def test_updates_at_64_channels_are_added_in_fp32(device, name, args):
+    """An update accumulated into an fp32 pair keeps fp32 bits (a bf16 rounding would leave 16 zero bits
+    in every value)."""
+    announce("64 channels fp32 update", name)
+    n = 50
+    fn = {"TriangleMultiplication": hnn.triangle_multiplication_hip, "GridSelfAttention": hnn.grid_self_attention_hip}[name]
+    _, hip = pair_of(name, dict(c_pair=64, **args), seed=n)
+    pair = torch.randn(n, n, 64, generator=torch.Generator().manual_seed(n)).to(device)
+    out = torch.zeros(n, n, 64, device=device)
+    with torch.inference_mode(), autocast(True):
+        fn(hip, pair, torch.ones(n, n, device=device), accumulate_into=out)
+    assert (out != out.bfloat16().float()).float().mean() > 0.98        # (2^-16 of all values by chance)
+
+
 # n = 520: enough 32-position units (520 x 17) for the 32-position projection path on a
 # 256-CU device; the smaller sizes take the 16-position path.
 @pytest.mark.parametrize("n,mask_dtype", [(33, torch.float32), (96, torch.bfloat16), (45, torch.bool),

@@ -217,7 +217,7 @@ __global__ __launch_bounds__(512, wgs_per_cu(K)) void grid_project_kernel(GridPr
 //   y      = bf16(sigmoid(gate) * o)   (o: attention output rows, K-layout loads moved to
 //                                       O-layout by identity MFMAs)
 //   u^T    = Wout . y^T                (y is the k operand as it stands, Wout in kperm order)
-//   z     += bf16(u)                   (bf16 pair updated in place: the residual is the z
+//   z     += u                         (rowstep::update_value; bf16 pair updated in place: the residual is the z
 //                                       already loaded, moved to O-layout the same way)
 template <typename TIN, typename TOUT, int K>
 __global__ __launch_bounds__(512, wgs_per_cu(K)) void grid_output_kernel(GridOutputArgs a) {
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(512, wgs_per_cu(K)) void grid_output_kernel(GridOut
       for (int t = 0; t < NT; ++t) {
         float o[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = res[t][e] + static_cast<float>(bf16(acc[t][e]));  // bf16 update
+        for (int e = 0; e < 4; ++e) o[e] = res[t][e] + rowstep::update_value<K>(acc[t][e]);
         rowstep::store4f<TOUT>(out + pos * K + 16 * t + 4 * g, o);
       }
     }

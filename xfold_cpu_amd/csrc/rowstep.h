@@ -268,6 +268,14 @@ __device__ __forceinline__ void k_to_o(const bf16x8 (&id)[2], const bf16x8 (&x)[
     for (int h = 0; h < 2; ++h) o[2 * ks + h] = mfma16(id[h], x[ks], f32x4{0.f, 0.f, 0.f, 0.f});
 }
 
+// What a pair update adds to the residual: rounded to bf16 at 128 channels, as an autocast Linear
+// returns it; unrounded at 64, where the general kernels (whose residual add is a GEMM epilogue)
+// take operands that are not aligned and both must give one result.
+template <int CC> __device__ __forceinline__ float update_value(float v) {
+  if constexpr (CC == 64) return v;
+  else return static_cast<float>(bf16(v));
+}
+
 // Pairs the O-layout values of tiles 2 ks and 2 ks + 1 into k-operand ks (kperm order).
 template <int KS>
 __device__ __forceinline__ void o_to_operand(const float (&y)[2 * KS][4], bf16x8 (&x)[KS]) {

@@ -150,7 +150,7 @@ __global__ __launch_bounds__(512, wgs_per_cu(K)) void trimul_project_kernel(TriP
 //            fragment, times an identity B (either k-half) they land in O-layout (exact)
 //   y      = bf16(LN_c(c))                    (statistics over the 4 lanes of a position)
 //   u^T    = Wout . y^T                       (Wout in kperm order)
-//   z     += bf16(u * sigmoid(gate))
+//   z     += u * sigmoid(gate)               (rowstep::update_value)
 template <typename TIN, typename TOUT, int K>
 __global__ __launch_bounds__(512, wgs_per_cu(K)) void trimul_output_kernel(TriOutputArgs a) {
   constexpr int KS = K / 32, NT = K / 16;
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(512, wgs_per_cu(K)) void trimul_output_kernel(TriOu
       for (int t = 0; t < NT; ++t) {
         float o[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = res[t][e] + static_cast<float>(bf16(acc[t][e] * sig[t][e]));
+        for (int e = 0; e < 4; ++e) o[e] = res[t][e] + rowstep::update_value<K>(acc[t][e] * sig[t][e]);
         rowstep::store4f<TOUT>(out + pos * K + 16 * t + 4 * g, o);
       }
     }
