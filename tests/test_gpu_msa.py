@@ -206,3 +206,17 @@ def test_evoformer_block(device, rows, n, mode):
     assert got_pair.dtype == torch.bfloat16
     assert_parity_bf16(got_msa, want_msa, "evoformer msa", floor=floor_msa)
     assert_parity_bf16(got_pair, want_pair, "evoformer pair", floor=floor_pair)
+
+
+@pytest.mark.parametrize("rows,n", [(3, 20), (7, 41), (11, 200)])
+def test_outer_product_mean_fp32_divides(device, rows, n):
+    """With zero output weights the module's result is output_b / (epsilon + rows), one fp32 division: every
+    bit is that of the quotient (a product with the rounded reciprocal is not, in a share of them)."""
+    announce("opm fp32 division", rows, n)
+    _, hip = pair_of("OuterProductMean", dict(c_msa=64, num_output_channel=128, num_outer_channel=32), seed=n)
+    with torch.no_grad():
+        hip.output_w.zero_()
+        msa, mask = torch.randn(rows, n, 64, device=device), torch.ones(rows, n, device=device)
+        got = hip(msa, mask)
+        want = hip.output_b / torch.tensor(hip.epsilon + rows, dtype=torch.float32, device=device)
+    assert torch.equal(got, want.expand_as(got))

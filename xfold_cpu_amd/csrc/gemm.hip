@@ -173,7 +173,7 @@ __global__ __launch_bounds__(THREADS) void gemm_nt_kernel(GemmArgs p) {
         }
       }
     } else {
-      store_any<TO>(p, acc, batch, mw, nw, col, grp);
+      store_any<true, TO>(p, acc, batch, mw, nw, col, grp);
     }
     return;
   }

@@ -123,7 +123,7 @@ __global__ __launch_bounds__(64 * G::KW) void gemm_direct_kernel(GemmArgs p) {
       if constexpr (ATTN) {
         store_attn<1, 1>(p, t, mw, nw, col, grp);
       } else {
-        store_any<TO>(p, t, batch, mw, nw, col, grp);
+        store_any<sizeof(T) == 4, TO>(p, t, batch, mw, nw, col, grp);
       }
     }
   }

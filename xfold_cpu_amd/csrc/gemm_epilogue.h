@@ -45,21 +45,24 @@ template <int EPI> __device__ __forceinline__ float epilogue(float acc, float c,
 // 4 grp + e) through epilogue EPI. The epilogue kind is a template parameter and the row
 // quantities (row divisor, auxiliary row) are taken once per row: a runtime switch per
 // element made this code ~10x larger than the main loop, and its instruction-cache misses
-// cost ~10 us per launch whatever the grid.
-template <int EPI, typename TO, int NT, int MT>
+// cost ~10 us per launch whatever the grid. DIV divides by the row divisor; else its
+// reciprocal, taken once per row, multiplies (one fp32 rounding more, on bf16 products).
+template <int EPI, typename TO, int NT, bool DIV = false, int MT>
 __device__ __forceinline__ void store_tile(const GemmArgs &p, const f32x4 (&acc)[NT][MT], int64_t batch, int mw,
                                            int nw, int col, int grp) {
   constexpr bool READS_C = EPI == XFH_EPI_ACCUMULATE || EPI == XFH_EPI_MUL_SIGMOID_AUX_ACCUMULATE;
   constexpr bool AUX = EPI == XFH_EPI_MUL_SIGMOID_AUX || EPI == XFH_EPI_SIGMOID_MUL_AUX ||
                        EPI == XFH_EPI_MUL_SIGMOID_AUX_ACCUMULATE;
   TO *C = static_cast<TO *>(p.C) + batch * p.sC;
+  auto scaled = [](float v, float r) { return DIV ? v / r : v * r; };
   int m[MT];
   float rs[MT];
   const TO *arow[MT];
 #pragma unroll
   for (int y = 0; y < MT; ++y) {
     m[y] = mw + y * 16 + col;
-    rs[y] = p.row_div && m[y] < p.M ? 1.0f / (p.row_div_eps + p.row_div[m[y]]) : 1.0f;
+    rs[y] = p.row_div && m[y] < p.M ? p.row_div_eps + p.row_div[m[y]] : 1.0f;
+    if constexpr (!DIV) rs[y] = 1.0f / rs[y];
     arow[y] = nullptr;
     if constexpr (AUX) {
       const int ar = p.aux_rows > 0 ? m[y] % int(p.aux_rows) : m[y];
@@ -83,7 +86,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs &p, const f32x4 (&acc)
         if constexpr (READS_C) Vec4<TO>::load(c, cv);
         if constexpr (AUX) Vec4<TO>::load(arow[y] + n, av);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) out[e] = epilogue<EPI>((acc[x][y][e] + bias[e]) * rs[y], cv[e], av[e]);
+        for (int e = 0; e < 4; ++e) out[e] = epilogue<EPI>(scaled(acc[x][y][e] + bias[e], rs[y]), cv[e], av[e]);
         Vec4<TO>::store(c, out);
       }
     }
@@ -116,7 +119,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs &p, const f32x4 (&acc)
       }
       // (acc + bias) * 1.0f is exact, so rows without a divisor keep acc + bias.
 #pragma unroll
-      for (int e = 0; e < 4; ++e) out[e] = epilogue<EPI>((acc[x][y][e] + bias[e]) * rs[y], cv[e], av[e]);
+      for (int e = 0; e < 4; ++e) out[e] = epilogue<EPI>(scaled(acc[x][y][e] + bias[e], rs[y]), cv[e], av[e]);
       if (full) {
         Vec4<TO>::store(c, out);
       } else {
@@ -128,10 +131,17 @@ __device__ __forceinline__ void store_tile(const GemmArgs &p, const f32x4 (&acc)
   }
 }
 
-// The runtime switch over the epilogue kinds, once per sub-tile.
-template <typename TO, int NT, int MT>
+// The runtime switch over the epilogue kinds, once per sub-tile. DIV: products with a row divisor
+// (OuterProductMean's, stored or accumulated) divide.
+template <bool DIV, typename TO, int NT, int MT>
 __device__ __forceinline__ void store_any(const GemmArgs &p, const f32x4 (&acc)[NT][MT], int64_t batch, int mw, int nw,
                                           int col, int grp) {
+  if constexpr (DIV) {
+    if (p.row_div && p.epi == XFH_EPI_STORE)
+      return store_tile<XFH_EPI_STORE, TO, NT, true>(p, acc, batch, mw, nw, col, grp);
+    if (p.row_div && p.epi == XFH_EPI_ACCUMULATE)
+      return store_tile<XFH_EPI_ACCUMULATE, TO, NT, true>(p, acc, batch, mw, nw, col, grp);
+  }
   switch (p.epi) {
     case XFH_EPI_MUL_SIGMOID_AUX: store_tile<XFH_EPI_MUL_SIGMOID_AUX, TO, NT>(p, acc, batch, mw, nw, col, grp); break;
     case XFH_EPI_SIGMOID_MUL_AUX: store_tile<XFH_EPI_SIGMOID_MUL_AUX, TO, NT>(p, acc, batch, mw, nw, col, grp); break;

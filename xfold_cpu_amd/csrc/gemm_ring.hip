@@ -291,7 +291,7 @@ __global__ __launch_bounds__(256, G::WGS) void gemm_ring_kernel(GemmArgs p) {
     store_attn(p, acc, mw, nw, col, grp);
     return;
   }
-  store_any<TO>(p, acc, batch, mw, nw, col, grp);
+  store_any<false, TO>(p, acc, batch, mw, nw, col, grp);
 }
 
 }  // namespace
