@@ -308,8 +308,7 @@ class _Kept:
     """One kept value and what it was made from, replaced as a whole (threads may share a module);
     a copied or pickled one starts empty."""
 
-    def __init__(self):
-        self.clear()
+    _entry = (None, None, None)
 
     def __reduce__(self):
         return type(self), ()
@@ -323,7 +322,7 @@ class _Kept:
         return self._entry[2]
 
     def clear(self):
-        self._entry = (None, None, None)
+        self._entry = _Kept._entry
 
     def lookup(self, key):
         kept, storages, value = self._entry

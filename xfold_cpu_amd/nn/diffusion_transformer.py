@@ -204,31 +204,30 @@ def _conditioning_weights(module: nn.Module, alns, zeros, dtype: torch.dtype):
     ([2A, c, c_s] scale/shift weights with the single_cond LayerNorm's weight folded into
     their input columns, [2A, c] fp32 biases, [Z, c, c_s] adaptive_zero_cond weights, [Z, c]
     biases). LayerNorm(s) = s_hat * g + b, so Linear(LayerNorm(s)) = s_hat (W g)^T + (W b + bias)."""
-    srcs = []
-    for a in alns:
-        cln = a.single_cond_layer_norm
-        srcs += [t for t in (cln.weight, cln.bias, a.single_cond_scale.weight, a.single_cond_scale.bias,
-                             a.single_cond_bias.weight, a.single_cond_bias.bias) if t is not None]
-    for z in zeros:
-        srcs += [t for t in (z.adaptive_zero_cond.weight, z.adaptive_zero_cond.bias) if t is not None]
+    linears = ("single_cond_scale", "single_cond_bias")
+    norms = [nh.params(a, (), ("single_cond_layer_norm",)) for a in alns]
+    conds = [[(nh.param(a, name), nh.param(a, name, "bias")) for name in linears] for a in alns]
+    zero_conds = [(nh.param(z, "adaptive_zero_cond"), nh.param(z, "adaptive_zero_cond", "bias")) for z in zeros]
+    srcs = [t for norm, cond in zip(norms, conds) for t in (*norm, *cond[0], *cond[1]) if t is not None]
+    srcs += [t for pair in zero_conds for t in pair if t is not None]
 
     def build(*_):
         with torch.no_grad():
+            none = torch.zeros(conds[0][0][0].shape[0], dtype=torch.float32, device=srcs[0].device)
+
+            def bias_of(w, b):
+                return b.detach().float() if b is not None else none if w.shape[0] == len(none) else w.new_zeros(w.shape[0])
             ws, bs = [], []
-            for a in alns:
-                cln = a.single_cond_layer_norm
-                for lin in (a.single_cond_scale, a.single_cond_bias):
-                    w = lin.weight.detach().float()
-                    b = (lin.bias.detach().float() if lin.bias is not None
-                         else torch.zeros(w.shape[0], dtype=torch.float32, device=w.device))
-                    if cln.bias is not None:
-                        b = b + w @ cln.bias.detach().float()
-                    ws.append(w * cln.weight.detach().float() if cln.weight is not None else w)
+            for (nw, nb), cond in zip(norms, conds):
+                for weight, bias in cond:
+                    w = weight.detach().float()
+                    b = bias_of(w, bias)
+                    if nb is not None:
+                        b = b + w @ nb.detach().float()
+                    ws.append(w * nw.detach().float() if nw is not None else w)
                     bs.append(b)
-            zw = [z.adaptive_zero_cond.weight.detach().float() for z in zeros]
-            zb = [z.adaptive_zero_cond.bias.detach().float() if z.adaptive_zero_cond.bias is not None
-                  else torch.zeros(w.shape[0], dtype=torch.float32, device=w.device)
-                  for z, w in zip(zeros, zw)]
+            zw = [w.detach().float() for w, _ in zero_conds]
+            zb = [bias_of(w, b) for w, (_, b) in zip(zw, zero_conds)]
             return (torch.stack(ws).to(dtype).contiguous(), torch.stack(bs).contiguous(),
                     torch.stack(zw).to(dtype).contiguous(), torch.stack(zb).contiguous())
 
