@@ -220,3 +220,23 @@ def test_outer_product_mean_fp32_divides(device, rows, n):
         got = hip(msa, mask)
         want = hip.output_b / torch.tensor(hip.epsilon + rows, dtype=torch.float32, device=device)
     assert torch.equal(got, want.expand_as(got))
+
+
+@pytest.mark.parametrize("rows,n,bad", [(17, 40, (3, 16)), (16, 65, (0,)), (33, 7, (31,))])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_msa_attention_keeps_a_bad_row_to_itself(device, rows, n, bad, value):
+    """MSA rows share the attention's weights and nothing else: a row that is not finite leaves the others
+    as they are, bit for bit (the fused tail turns 16 rows at a time)."""
+    announce("msa bad row", rows, n, bad, value)
+    _, hip = pair_of("MSAAttention", dict(c_msa=64, c_pair=128, num_head=8), seed=n)
+    torch.manual_seed(rows)
+    msa, pair = torch.randn(rows, n, 64).bfloat16().to(device), torch.randn(n, n, 128).bfloat16().to(device)
+    mask = torch.ones(rows, n, device=device)
+    broken = msa.clone()
+    broken[list(bad), n // 2, 5] = value
+    good = [r for r in range(rows) if r not in bad]
+    with torch.inference_mode(), autocast(True):
+        for x in (msa, msa.float()):
+            want, got = hip(x, mask, pair), hip(broken.to(x.dtype), mask, pair)
+            assert torch.isfinite(want).all() and torch.equal(got[good], want[good])
+            assert not torch.isfinite(got[list(bad)]).any()

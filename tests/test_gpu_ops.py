@@ -477,6 +477,25 @@ def test_updates_at_64_channels_are_added_in_fp32(device, name, args):
     assert (out != out.bfloat16().float()).float().mean() > 0.98        # (2^-16 of all values by chance)
 
 
+@pytest.mark.parametrize("c", [64, 128])
+@pytest.mark.parametrize("n,at", [(37, (20, 5)), (16, (15, 15)), (33, (32, 0))])
+@pytest.mark.parametrize("outgoing", [True, False])
+def test_triangle_multiplication_keeps_nan_where_it_belongs(device, c, n, at, outgoing):
+    """A position that is not finite reaches its row and column of the contraction and no other result (the
+    fused output kernel turns 16 positions at a time); the rest is as with a finite value there."""
+    announce("trimul nan", c, n, at, outgoing)
+    ref, hip = pair_of("TriangleMultiplication", dict(c_pair=c, _outgoing=outgoing), seed=n)
+    pair, mask = torch.randn(n, n, c, generator=torch.Generator().manual_seed(n)).bfloat16(), torch.ones(n, n)
+    broken = pair.clone()
+    broken[at] = float("nan")
+    with torch.inference_mode():
+        bad = ref(broken.float(), mask).isnan()
+        with autocast(True):
+            want, got = (hip(p.to(device), mask.to(device)).cpu() for p in (pair, broken))
+    assert torch.isfinite(want).all() and not bad.all()
+    assert torch.equal(got.isnan(), bad) and torch.equal(got[~bad], want[~bad])
+
+
 # n = 520: enough 32-position units (520 x 17) for the 32-position projection path on a
 # 256-CU device; the smaller sizes take the 16-position path.
 @pytest.mark.parametrize("n,mask_dtype", [(33, torch.float32), (96, torch.bfloat16), (45, torch.bool),

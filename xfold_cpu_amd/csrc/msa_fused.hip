@@ -169,6 +169,18 @@ __global__ __launch_bounds__(512, 2) void msa_output_kernel(MsaOutputArgs a) {
       avg[k] = mfma16(cur.c[k], id[0], f32x4{0.f, 0.f, 0.f, 0.f});
       avg[k + KS] = mfma16(cur.c[k], id[1], f32x4{0.f, 0.f, 0.f, 0.f});
     }
+    if (any_nonfinite(avg)) {                        // a bad sequence leaves the 15 others of its step alone
+      const int q = st / blocks, s0 = (st - q * blocks) * 16;
+      int p0 = 4 * g;
+      asm volatile("" : "+v"(p0));                   // (keeps the 16 addresses' divisions in here: 66 registers)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int p = 16 * t + p0 + e, h = p / a.dv, c = p - h * a.dv;
+          avg[t][e] = static_cast<float>(a.avg_t[((int64_t(h) * a.n + q) * a.dv + c) * a.rows_pad + s0 + r]);
+        }
+    }
     float y[NT][4];
 #pragma unroll
     for (int t = 0; t < NT; ++t)

@@ -268,6 +268,18 @@ __device__ __forceinline__ void k_to_o(const bf16x8 (&id)[2], const bf16x8 (&x)[
     for (int h = 0; h < 2; ++h) o[2 * ks + h] = mfma16(id[h], x[ks], f32x4{0.f, 0.f, 0.f, 0.f});
 }
 
+// A product with identity fragments moves finite values exactly, but 0 * NaN and 0 * infinity are NaN:
+// one such value makes the others of its k-half NaN. Whether that may have happened in this
+// wavefront's tiles (uniform); the caller then reads the values again one by one.
+template <int NT> __device__ __forceinline__ bool any_nonfinite(const f32x4 (&o)[NT]) {
+  float zero = 0.f;                       // 0 * x: NaN from the first value on that is not finite
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) zero = __builtin_fmaf(o[t][e], 0.f, zero);
+  return __ballot(zero != zero) != 0;
+}
+
 // What a pair update adds to the residual: rounded to bf16 at 128 channels, as an autocast Linear
 // returns it; unrounded at 64, where the general kernels (whose residual add is a GEMM epilogue)
 // take operands that are not aligned and both must give one result.
