@@ -61,8 +61,8 @@ __device__ __forceinline__ void store_tile(const GemmArgs &p, const f32x4 (&acc)
 #pragma unroll
   for (int y = 0; y < MT; ++y) {
     m[y] = mw + y * 16 + col;
-    rs[y] = p.row_div && m[y] < p.M ? p.row_div_eps + p.row_div[m[y]] : 1.0f;
-    if constexpr (!DIV) rs[y] = 1.0f / rs[y];
+    rs[y] = 1.0f;
+    if (p.row_div && m[y] < p.M) rs[y] = DIV ? p.row_div_eps + p.row_div[m[y]] : 1.0f / (p.row_div_eps + p.row_div[m[y]]);
     arow[y] = nullptr;
     if constexpr (AUX) {
       const int ar = p.aux_rows > 0 ? m[y] % int(p.aux_rows) : m[y];

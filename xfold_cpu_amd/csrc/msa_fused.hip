@@ -116,6 +116,7 @@ __global__ __launch_bounds__(512, 2) void msa_output_kernel(MsaOutputArgs a) {
   constexpr bool kBf16 = sizeof(TIN) == 2 && sizeof(TOUT) == 2;
   const bool res_from_x = kBf16 && a.accumulate && a.x == a.out;
   const bool res_load = a.accumulate && !res_from_x;
+  const int dv_log2 = __builtin_ctz(a.dv);           // (dv divides 64)
   bf16x8 id[2];
   identity_frags(id);
   struct Rows {
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(512, 2) void msa_output_kernel(MsaOutputArgs a) {
     const int q = st / blocks, s0 = (st - q * blocks) * 16;
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
-      const int p = 16 * (k + KS * (g >> 1)) + r, h = p / a.dv, c = p - h * a.dv;
+      const int p = 16 * (k + KS * (g >> 1)) + r, h = p >> dv_log2, c = p - h * a.dv;
       rw.c[k] = *reinterpret_cast<const bf16x8 *>(a.avg_t + ((int64_t(h) * a.n + q) * a.dv + c) * a.rows_pad + s0 + 8 * (g & 1));
     }
   };
@@ -169,15 +170,15 @@ __global__ __launch_bounds__(512, 2) void msa_output_kernel(MsaOutputArgs a) {
       avg[k] = mfma16(cur.c[k], id[0], f32x4{0.f, 0.f, 0.f, 0.f});
       avg[k + KS] = mfma16(cur.c[k], id[1], f32x4{0.f, 0.f, 0.f, 0.f});
     }
-    if (any_nonfinite(avg)) {                        // a bad sequence leaves the 15 others of its step alone
+    if (moved_nonfinite(avg)) {                      // a bad sequence leaves the 15 others of its step alone
       const int q = st / blocks, s0 = (st - q * blocks) * 16;
       int p0 = 4 * g;
-      asm volatile("" : "+v"(p0));                   // (keeps the 16 addresses' divisions in here: 66 registers)
+      asm volatile("" : "+v"(p0));                   // (keeps the 16 offsets in here: 60 registers)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int p = 16 * t + p0 + e, h = p / a.dv, c = p - h * a.dv;
+          const int p = 16 * t + p0 + e, h = p >> dv_log2, c = p - h * a.dv;
           avg[t][e] = static_cast<float>(a.avg_t[((int64_t(h) * a.n + q) * a.dv + c) * a.rows_pad + s0 + r]);
         }
     }

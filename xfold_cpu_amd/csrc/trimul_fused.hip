@@ -231,7 +231,7 @@ __global__ __launch_bounds__(512, wgs_per_cu(K)) void trimul_output_kernel(TriOu
         co[q] = mfma16(cur.c[q], id[0], f32x4{0.f, 0.f, 0.f, 0.f});
         co[q + KS] = mfma16(cur.c[q], id[1], f32x4{0.f, 0.f, 0.f, 0.f});
       }
-      if (rowstep::any_nonfinite(co)) {              // a bad position leaves the 15 others of its block alone
+      if (rowstep::moved_nonfinite(co)) {            // a bad position leaves the 15 others of its block alone
         const bf16 *src = a.contracted + st * res_block_stride(K) + 64 * g + r;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
