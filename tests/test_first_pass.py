@@ -85,6 +85,17 @@ def test_the_first_pass_prepares_every_weight(stubbed, kind):
     assert passes[0] and passes[1] == passes[2]
 
 
+def test_the_fused_cross_attention_prepares_its_own_weights_only(stubbed):
+    """No stacked k and v for the general path beside the fused kernels' separate ones."""
+    make, inputs = MODULES["cross_attention_fused"]
+    module, args = make().eval(), inputs()
+    with torch.no_grad():
+        module(*args)
+        module(*args)
+    assert set(module.__dict__["_hip_weight_groups"]) == {"fused"}
+    assert not [tag for tag in module.__dict__["_hip_weight_caches"] if tag.startswith("fused:")]
+
+
 @pytest.mark.parametrize("kind", MODULES)
 def test_nothing_made_in_a_capture_is_kept(stubbed, monkeypatch, kind):
     make, inputs = MODULES[kind]

@@ -541,11 +541,8 @@ def cross_attention_hip(module: nn.Module, x_q: torch.Tensor, x_k: torch.Tensor,
                          f"{tuple(x_q.shape)}; {tuple(mask_k.shape)}, {tuple(x_k.shape)})")
     nh.check_gpu_inference(x_q, x_k, mask_q, mask_k, pair_logits, single_cond_q, single_cond_k)
     nh.check_module(module)
-    dtype, (w_q, w_kv, w_gate) = nh.gather(
-        module, "cross_attention", nh.params(module, _QKV + ("gating_query",)), 4, x_q,
-        lambda dt: (nh.linear_weight(module, "q_projection", dt),
-                    nh.fused_linear_weight(module, ("k_projection", "v_projection"), dt),
-                    nh.linear_weight(module, "gating_query", dt)))
+    sources = nh.params(module, _QKV + ("gating_query",))
+    dtype = nh.compute_dtype(x_q, *sources)
     lead, nq, nk = tuple(x_q.shape[:-2]), x_q.shape[-2], x_k.shape[-2]
     if tuple(x_k.shape[:-2]) != lead:
         raise ValueError("CrossAttention: x_q and x_k must share their leading (subset) dims")
@@ -561,6 +558,11 @@ def cross_attention_hip(module: nn.Module, x_q: torch.Tensor, x_k: torch.Tensor,
                                    lead, batch, accumulate_into)
     if fused is not None:
         return fused
+    _, (w_q, w_kv, w_gate) = nh.gather(
+        module, "cross_attention", sources, 4, x_q,
+        lambda dt: (nh.linear_weight(module, "q_projection", dt),
+                    nh.fused_linear_weight(module, ("k_projection", "v_projection"), dt),
+                    nh.linear_weight(module, "gating_query", dt)), dtype)
     xq = _adaptive_layer_norm(module.q_adaptive_layernorm, x_q, single_cond_q, dtype)
     xk = _adaptive_layer_norm(module.k_adaptive_layernorm, x_k, single_cond_k, dtype)
     q = ops.linear(xq, w_q, nh.param(module, "q_projection", "bias"), dtype)
