@@ -85,6 +85,22 @@ def test_the_first_pass_prepares_every_weight(stubbed, kind):
     assert passes[0] and passes[1] == passes[2]
 
 
+def test_an_operators_weights_are_copied_together(stubbed):
+    """The four plain weights of a triangle multiplication and the six of a grid attention, in one call and
+    one allocation each: a block's first pass is bound by this host work."""
+    make, inputs = MODULES["pairformer"]
+    module, args = make().eval(), inputs()
+    with torch.no_grad(), Computed() as computed:
+        module(*args)
+    assert computed.names.count("aten::_foreach_copy_") == 4
+    # What is left: both transitions' two, the pair logits' one, the attention's four and output.
+    assert computed.names.count("aten::_to_copy") == 10
+    weights = nh.linear_weights(module.pair_attention1, ("q_projection", "pair_bias_projection", "k_projection"), torch.bfloat16)
+    for name, w in zip(("q_projection", "pair_bias_projection", "k_projection"), weights):
+        assert torch.equal(w, getattr(module.pair_attention1, name).weight.detach().bfloat16()) and w.is_contiguous()
+        assert (w.data_ptr() - weights[0].data_ptr()) % 256 == 0
+
+
 def test_the_fused_cross_attention_prepares_its_own_weights_only(stubbed):
     """No stacked k and v for the general path beside the fused kernels' separate ones."""
     make, inputs = MODULES["cross_attention_fused"]

@@ -26,7 +26,7 @@ def grid_self_attention_hip(module: nn.Module, pair: torch.Tensor, mask: Optiona
     nh.check_module(module)
     dtype, (w, nw, nb) = nh.gather(
         module, "grid_self_attention", nh.params(module, _GRID_WEIGHTS, ("act_norm",)), len(_GRID_WEIGHTS), pair,
-        lambda dt: ([nh.linear_weight(module, n, dt) for n in _GRID_WEIGHTS], *nh.norm_params(module, "act_norm")))
+        lambda dt: (nh.linear_weights(module, _GRID_WEIGHTS, dt), *nh.norm_params(module, "act_norm")))
     if pair.dim() != 3 or pair.shape[0] != pair.shape[1] or pair.shape[2] != module.c_pair:
         raise ValueError("GridSelfAttention expects pair [N, N, c_pair].")
     n, c = pair.shape[0], pair.shape[2]
@@ -85,7 +85,7 @@ def msa_attention_hip(module: nn.Module, msa: torch.Tensor, msa_mask: Optional[t
     nh.check_module(module)
     dtype, (w, aw, ab, pw, pb) = nh.gather(
         module, "msa_attention", nh.params(module, _MSA_WEIGHTS, ("act_norm", "pair_norm")), len(_MSA_WEIGHTS), msa,
-        lambda dt: ([nh.linear_weight(module, n, dt) for n in _MSA_WEIGHTS], *nh.norm_params(module, "act_norm"),
+        lambda dt: (nh.linear_weights(module, _MSA_WEIGHTS, dt), *nh.norm_params(module, "act_norm"),
                     *nh.norm_params(module, "pair_norm")))
     if msa.dim() != 3 or msa.shape[-1] != module.c_msa:
         raise ValueError("MSAAttention expects msa [S, N, c_msa].")

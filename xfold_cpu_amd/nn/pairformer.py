@@ -213,10 +213,10 @@ def _pair_updates_hip(block: nn.Module, pair: torch.Tensor, pair_mask: torch.Ten
         out = []
         for t in triangles:
             out += (*nh.norm_params(t, _TRIANGLE_NORMS[0]), *nh.norm_params(t, _TRIANGLE_NORMS[1]))
-            out += (nh.linear_weight(t, name, dt) for name in _TRIANGLE_WEIGHTS)
+            out += nh.linear_weights(t, _TRIANGLE_WEIGHTS, dt)
         for g in grids:
             out += nh.norm_params(g, "act_norm")
-            out += (nh.linear_weight(g, name, dt) for name in _GRID_WEIGHTS)
+            out += nh.linear_weights(g, _GRID_WEIGHTS, dt)
         out += nh.norm_params(tr, "input_layer_norm")
         out += (nh.linear_weight(tr, "transition1", dt, "glu"), nh.linear_weight(tr, "transition2", dt))
         return out

@@ -30,7 +30,7 @@ def triangle_multiplication_hip(module: nn.Module, pair: torch.Tensor, mask: Opt
     nh.check_module(module)
     dtype, (w_proj, w_gate, w_out, w_gating, lw, lb, cw, cb) = nh.gather(
         module, "triangle_multiplication", nh.params(module, _WEIGHTS, _NORMS), 4, pair,
-        lambda dt: (*(nh.linear_weight(module, n, dt) for n in _WEIGHTS),
+        lambda dt: (*nh.linear_weights(module, _WEIGHTS, dt),
                     *nh.norm_params(module, _NORMS[0]), *nh.norm_params(module, _NORMS[1])))
     if pair.dim() != 3 or pair.shape[0] != pair.shape[1] or pair.shape[2] != module.c_pair:
         raise ValueError("TriangleMultiplication expects pair [N, N, c_pair].")
