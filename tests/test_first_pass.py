@@ -160,3 +160,17 @@ def test_each_capture_has_attention_operands_of_its_own(stubbed, monkeypatch):
     capture = 0
     assert get() is eager
     assert [k[-1] for k in ops._SHARED_OPERANDS] == [0]      # the captures' sets are given back
+
+
+def test_a_single_weight_is_checked_once(stubbed, monkeypatch):
+    """A conditioned transition's later passes take each weight's key once, without a group around it."""
+    make, inputs = MODULES["diffusion_transition"]
+    module, args = make().eval(), inputs()
+    seen, stamp = [], nh.stamp
+    monkeypatch.setattr(nh, "stamp", lambda t: seen.append(t) or stamp(t))
+    with torch.no_grad():
+        for _ in range(2):
+            del seen[:]
+            module(*args)
+            assert len(seen) == len({id(t) for t in seen}) == 6     # (three Linears, scale, shift and its bias)
+    assert not any("_hip_weight_groups" in m.__dict__ for m in module.modules())

@@ -16,7 +16,6 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from ..fastnn import LayerNorm
 from ..fastnn import config as fastnn_config
@@ -57,8 +56,13 @@ def _scale_shift_weights(dtype: torch.dtype, scale: torch.Tensor, shift: torch.T
     """single_cond_scale and single_cond_bias as one [2, c, c_cond] weight in ``dtype`` and their
     [2, c] fp32 bias (zeros for single_cond_bias, which has none; None without a bias)."""
     c, k = scale.shape
-    w = torch.cat([scale.detach(), shift.detach()]).to(dtype).view(2, c, k)
-    return w, None if bias is None else F.pad(bias.detach().float(), (0, c)).view(2, c)
+    w = torch.empty((2, c, k), dtype=dtype, device=scale.device)
+    torch._foreach_copy_(w.unbind(0), (scale, shift))
+    if bias is None:
+        return w, None
+    b = torch.zeros((2, c), dtype=torch.float32, device=scale.device)
+    b[0].copy_(bias)
+    return w, b
 
 
 def _ada_ln_zero(zero: nn.Module, hidden: torch.Tensor, single_cond: Optional[torch.Tensor],
@@ -66,26 +70,19 @@ def _ada_ln_zero(zero: nn.Module, hidden: torch.Tensor, single_cond: Optional[to
                  cond: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``AdaLNZero.forward`` (``diffusion_transformer.py:85-95``), optionally added in place;
     ``cond`` = adaptive_zero_cond(single_cond) already computed, in the output dtype."""
-    conditioned = zero.use_single_cond and cond is None
-    sources = [nh.param(zero, "transition2")]
-    if conditioned:
-        sources.append(nh.param(zero, "adaptive_zero_cond"))
-    _, weights = nh.gather(
-        zero, "conditioned" if conditioned else "zero", sources, 0, hidden,
-        lambda dt: [nh.linear_weight(zero, name, dt) for name in ("transition2", "adaptive_zero_cond")[:len(sources)]],
-        dtype)
+    w = nh.linear_weight(zero, "transition2", dtype)
     out = accumulate_into
     out_dtype = out.dtype if out is not None else dtype
     acc = out is not None
     if zero.use_single_cond:
         if cond is None:
-            cond = ops.linear(single_cond, weights[1], nh.param(zero, "adaptive_zero_cond", "bias"), dtype,
-                              out_dtype=out_dtype)
+            cond = ops.linear(single_cond, nh.linear_weight(zero, "adaptive_zero_cond", dtype),
+                              nh.param(zero, "adaptive_zero_cond", "bias"), dtype, out_dtype=out_dtype)
         epi = nh.EPI_MUL_SIGMOID_AUX_ACCUMULATE if acc else nh.EPI_MUL_SIGMOID_AUX
-        return ops.linear(hidden, weights[0], None, dtype, out=out, out_dtype=out_dtype, epilogue=epi,
+        return ops.linear(hidden, w, None, dtype, out=out, out_dtype=out_dtype, epilogue=epi,
                           aux=cond, aux_rows=cond.numel() // cond.shape[-1])
     epi = nh.EPI_ACCUMULATE if acc else nh.EPI_STORE
-    return ops.linear(hidden, weights[0], None, dtype, out=out, out_dtype=out_dtype, epilogue=epi)
+    return ops.linear(hidden, w, None, dtype, out=out, out_dtype=out_dtype, epilogue=epi)
 
 
 def _check_accumulate(out, x):
@@ -100,13 +97,12 @@ def diffusion_transition_hip(module: nn.Module, x: torch.Tensor, single_cond=Non
     (scale, shift, zero_cond) precomputed by :func:`_block_conditioning`."""
     nh.check_gpu_inference(x, single_cond)
     nh.check_module(module)
-    sources = [nh.param(module, "transition1")]
-    dtype, w_glu = nh.gather(module, "transition1", sources, 1, x,
-                             lambda dt: nh.linear_weight(module, "transition1", dt, "glu"))
+    w1 = nh.param(module, "transition1")
+    dtype = nh.compute_dtype(x, w1)
     _check_accumulate(accumulate_into, x)
     xn = _adaptive_layer_norm(module.adaptive_layernorm, x, single_cond, dtype,
                               cond=None if _cond is None else _cond[:2])
-    hidden = ops.gated_linear_unit(xn, w_glu, sources[0].shape[0] // 2, dtype)
+    hidden = ops.gated_linear_unit(xn, nh.linear_weight(module, "transition1", dtype, "glu"), w1.shape[0] // 2, dtype)
     return _ada_ln_zero(module.adaptive_zero_init, hidden, single_cond, dtype, accumulate_into,
                         cond=None if _cond is None else _cond[2])
 
