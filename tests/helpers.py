@@ -173,3 +173,30 @@ def assert_parity_bf16(actual, expected, what="", floor=None, composition=False)
     assert max_err <= guard, (f"{what}: max|diff|/rms = {max_err:.3e} > {guard:.3e} "
                               f"(floor {floor_err:.3e})")
     return rms_err, max_err
+
+
+BLOCK_CALLS = ("xfh_pair_updates", "xfh_pairformer_single", "xfh_diffusion_blocks")
+
+
+def both_passes(run, *calls):
+    """``run()`` (which copies its inputs) as a module's first and second pass. The first goes operator by
+    operator while the weights are prepared, the second is the route of every later pass: it must
+    take exactly ``calls`` of the library's block calls and give the first one's result bit for
+    bit. Returns the second one's."""
+    from xfold_cpu_amd.fastnn import native_hip as nh
+    original, names, results = nh.call, [], []
+
+    def recorded(name, *args):
+        names[-1].append(name)
+        return original(name, *args)
+    nh.call = recorded
+    try:
+        for _ in range(2):
+            names.append([])
+            results.append(run())
+    finally:
+        nh.call = original
+    assert [sorted(set(BLOCK_CALLS).intersection(taken)) for taken in names] == [[], sorted(calls)]
+    first, second = (r if isinstance(r, tuple) else (r,) for r in results)
+    assert all(a is b is None or torch.equal(a, b) for a, b in zip(first, second))
+    return results[1]

@@ -5,10 +5,11 @@ import pytest
 import torch
 
 from oracle import restatement as R
-from tests.helpers import (TOL_BF16, TOL_FP32, assert_parity, assert_parity_bf16, floor_of,
+from tests.helpers import (TOL_BF16, TOL_FP32, assert_parity, assert_parity_bf16, both_passes, floor_of,
                            load_fixture, rel_err, residual)
 from tests.test_gpu_ops import announce, autocast, pair_of
 from xfold_cpu_amd import nn as hnn
+from xfold_cpu_amd.fastnn import native_hip as nh
 from xfold_cpu_amd.synthetic import init_module_, pair_block_inputs
 
 pytestmark = pytest.mark.gpu
@@ -94,13 +95,17 @@ def block_case(n, c_single, mode, pad, seed, device, with_single=True, c_pair=12
         floor_pair, floor_single = floor_of(oracle)
     with torch.inference_mode():
         want_pair, want_single = oracle()
-        dp = pair.to(device).contiguous()
-        ds = single.to(device).contiguous() if single is not None else None
-        with autocast(mode != "fp32"):
+
+        def run():
+            dp = pair.to(device).contiguous()
             if with_single:
-                got_pair, got_single = hip(dp, inp.pair_mask.to(device), ds, inp.seq_mask.to(device))
-            else:
-                got_pair, got_single = hip(dp, inp.pair_mask.to(device)), None
+                return hip(dp, inp.pair_mask.to(device), single.to(device).contiguous(), inp.seq_mask.to(device))
+            return hip(dp, inp.pair_mask.to(device)), None
+        calls = ["xfh_pair_updates"]
+        if with_single and mode == "bf16" and n <= nh.attention_max_keys():
+            calls.append("xfh_pairformer_single")
+        with autocast(mode != "fp32"):
+            got_pair, got_single = both_passes(run, *calls)
     return (got_pair, want_pair, floor_pair), (got_single, want_single, floor_single)
 
 
@@ -202,7 +207,7 @@ def test_diffusion_transformer_batched_samples(device, mode):
     with torch.inference_mode():
         want = oracle()
         with autocast(bf16):
-            got = hip(act.to(device).clone(), mask.to(device), scond.to(device), pcond.to(device))
+            got = both_passes(lambda: hip(act.to(device).clone(), mask.to(device), scond.to(device), pcond.to(device)))
     if not bf16:
         assert_parity(got, want, TOL_FP32, "diffusion transformer")
         return
@@ -216,7 +221,6 @@ def test_unpacked_bias_beyond_the_attention_key_limit(device, monkeypatch):
     [H, N, N] bias path (the general attention kernel) in the block's single track and in
     the diffusion transformer: with the limit lowered to 32, N = 40 must still match the
     oracle."""
-    from xfold_cpu_amd.fastnn import native_hip as nh
     monkeypatch.setattr(nh, "attention_max_keys", lambda: 32)
     (gp, wp, fp), (gs, ws, fs) = block_case(40, 64, "bf16", pad=3, seed=5, device=device)
     assert_parity_bf16(gp, wp, "pair (limit 32)", floor=fp)
@@ -244,7 +248,6 @@ def test_diffusion_input_cache_skips_the_pair_logits_on_repeat_calls(device):
     same pair_cond and weights reuses the packed pair logits (no pair_bias_kernel launch)
     and gives the same result bit for bit; an in-place update of pair_cond invalidates them."""
     from xfold_cpu_amd.fastnn import config
-    from xfold_cpu_amd.fastnn import native_hip as nh
     from xfold_cpu_amd.nn.cache import input_cache_scope
     args = dict(c_act=256, c_single_cond=64, c_pair_cond=128, num_head=16, num_blocks=4, super_block_size=2)
     _, hip = pair_of("DiffusionTransformer", args, seed=8, device=device)

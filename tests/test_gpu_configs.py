@@ -27,7 +27,7 @@ import pytest
 import torch
 
 from oracle import restatement as R
-from tests.helpers import TOL_FP32, assert_parity, assert_parity_bf16, floor_of, residual
+from tests.helpers import TOL_FP32, assert_parity, assert_parity_bf16, both_passes, floor_of, residual
 from tests.test_gpu_ops import announce, autocast
 from xfold_cpu_amd import nn as hnn
 from xfold_cpu_amd.synthetic import CONFIGS, diffusion_inputs, init_module_, pair_block_inputs
@@ -64,7 +64,7 @@ def test_c1_pair_block_fp32(device):
     inp = bench_inputs(cfg)
     with torch.inference_mode():
         want = ref(inp.pair.clone(), inp.pair_mask)
-        got = hip(inp.pair.to(device).contiguous(), inp.pair_mask.to(device))
+        got = both_passes(lambda: hip(inp.pair.to(device).contiguous(), inp.pair_mask.to(device)), "xfh_pair_updates")
     assert got.dtype == torch.float32
     assert_parity(got, want, TOL_FP32, "C1 pair block")
 
@@ -80,7 +80,7 @@ def test_c2_pair_block(device):
         return ref(wrap(pair.float()), inp.pair_mask, attention=chunked_attention)
     with torch.inference_mode():
         with autocast(True):
-            got = hip(pair.to(device).contiguous(), inp.pair_mask.to(device))
+            got = both_passes(lambda: hip(pair.to(device).contiguous(), inp.pair_mask.to(device)), "xfh_pair_updates")
         want = oracle()
     # bf16 residual stream, rounded at each of its 5 in-place updates (so is the floor's).
     floor = floor_of(lambda: oracle(residual))
@@ -100,8 +100,9 @@ def test_c3_block_with_single_track(device):
                    attention=chunked_attention)
     with torch.inference_mode():
         with autocast(True):
-            got_pair, got_single = hip(pair.to(device).contiguous(), inp.pair_mask.to(device),
-                                       single.to(device).contiguous(), inp.seq_mask.to(device))
+            got_pair, got_single = both_passes(
+                lambda: hip(pair.to(device).contiguous(), inp.pair_mask.to(device), single.to(device).contiguous(),
+                            inp.seq_mask.to(device)), "xfh_pair_updates", "xfh_pairformer_single")
         want_pair, want_single = oracle()
     floor_pair, floor_single = floor_of(lambda: oracle(residual))
     assert torch.isfinite(got_pair.float()).all() and torch.isfinite(got_single.float()).all()
@@ -150,8 +151,8 @@ def test_c4_diffusion_transformer(device):
                             for s in range(cfg["samples"])])
     with torch.inference_mode():
         with autocast(True):
-            got = hip(act.to(device).clone(), inp.mask.to(device), inp.single_cond.to(device),
-                      inp.pair_cond.to(device))
+            got = both_passes(lambda: hip(act.to(device).clone(), inp.mask.to(device), inp.single_cond.to(device),
+                                          inp.pair_cond.to(device)), "xfh_diffusion_blocks")
         want = oracle()
     # act is a bf16 residual stream rounded at each of its 2 updates per block.
     floor = floor_of(lambda: oracle(residual))

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import restatement as R
-from tests.helpers import TOL_FP32, assert_parity, assert_parity_bf16, floor_of, residual
+from tests.helpers import TOL_FP32, assert_parity, assert_parity_bf16, both_passes, floor_of, residual
 from tests.test_gpu_ops import announce, autocast, pair_of, run_both
 from xfold_cpu_amd import fastnn
 
@@ -138,7 +138,8 @@ def test_diffusion_transformer_tiny(device, n, samples):
     with torch.inference_mode():
         want = oracle()
         with autocast(True):
-            got = hip(act.to(device).clone(), mask.to(device), scond.to(device), pcond.to(device))
+            got = both_passes(lambda: hip(act.to(device).clone(), mask.to(device), scond.to(device), pcond.to(device)),
+                              "xfh_diffusion_blocks")
     assert torch.isfinite(got.float()).all()
     assert_parity_bf16(got, want, "diffusion transformer tiny", floor=floor_of(lambda: oracle(residual)))
 

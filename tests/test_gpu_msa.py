@@ -11,8 +11,8 @@ import pytest
 import torch
 
 from oracle import restatement as R
-from tests.helpers import (TOL_FP32, assert_parity, assert_parity_bf16, bf16_stored, floor_of, load_fixture,
-                           residual)
+from tests.helpers import (TOL_FP32, assert_parity, assert_parity_bf16, bf16_stored, both_passes, floor_of,
+                           load_fixture, residual)
 from tests.test_gpu_ops import announce, autocast, check_module, pair_of
 from xfold_cpu_amd import nn as hnn
 from xfold_cpu_amd.synthetic import init_module_
@@ -196,8 +196,8 @@ def test_evoformer_block(device, rows, n, mode):
     with torch.no_grad():
         want_msa, want_pair = oracle()
     with torch.inference_mode(), autocast(mode == "bf16"):
-        got_msa, got_pair = hip(msa.to(device).contiguous(), pair.to(device).contiguous(), mask.to(device),
-                                pair_mask.to(device))
+        got_msa, got_pair = both_passes(lambda: hip(msa.to(device, copy=True), pair.to(device, copy=True),
+                                                    mask.to(device), pair_mask.to(device)), "xfh_pair_updates")
     if mode == "fp32":
         assert_parity(got_msa, want_msa, TOL_FP32, "evoformer msa")
         assert_parity(got_pair, want_pair, TOL_FP32, "evoformer pair")
