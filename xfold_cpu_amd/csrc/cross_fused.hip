@@ -182,7 +182,6 @@ struct AttendArgs {
   const bf16 *q, *k, *vt;
   const float *gate;
   const void *logits;                    // element (b, h, q, key) at the strides ls, or null
-  int logit_dtype;
   int64_t ls[4];
   const void *mask_q, *mask_k;           // [subsets][nq], [subsets][nk]
   int mask_q_dtype, mask_k_dtype;
@@ -195,7 +194,6 @@ struct AttendArgs {
 // read straight from memory into its MFMA lanes: the whole problem of a wavefront is 8 K and 8 V
 // fragments per 128 keys. 192 subsets with the heads of the logits innermost: 13 us (42 for the bias
 // pass and the general kernel before).
-constexpr int QT = 1;                  // 16-query tiles per wavefront
 // How a wavefront reads its logits: one by one; four consecutive keys at a time; or all four
 // heads of a (query, key) at a time into LDS, for views with the heads innermost (a projection
 // for several layers): lane after lane takes the next key, where the direct reads touch a cache
@@ -205,17 +203,12 @@ template <typename TL, Logits MODE>
 __global__ __launch_bounds__(256, 2) void cross_attend_kernel(AttendArgs a) {
   const int lane = threadIdx.x & 63, h = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
   const int64_t b = int(blockIdx.x) / a.qtiles;
-  const int q0 = (int(blockIdx.x) - int(b) * a.qtiles) * 16 * QT;
+  const int q0 = (int(blockIdx.x) - int(b) * a.qtiles) * 16;
   constexpr int KT = MAXK / 16;          // key tiles
   const int tiles = a.kpad / 16;
-  bf16x8 qf[QT];
-  bool masked_q[QT];
-#pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    const int q = min(q0 + 16 * t + col, a.nq - 1);
-    qf[t] = *reinterpret_cast<const bf16x8 *>(a.q + (b * a.nq + q) * C + h * HD + g * 8);
-    masked_q[t] = load_any(a.mask_q, a.mask_q_dtype, b * a.nq + q) == 0.f;
-  }
+  const int qc = min(q0 + col, a.nq - 1);
+  const bf16x8 qf = *reinterpret_cast<const bf16x8 *>(a.q + (b * a.nq + qc) * C + h * HD + g * 8);
+  const bool masked_q = load_any(a.mask_q, a.mask_q_dtype, b * a.nq + qc) == 0.f;
   // Bit k of the words: key k is masked (wavefront ballots, so the tile loop has no mask loads).
   uint64_t masked_k[2];
 #pragma unroll
@@ -226,7 +219,6 @@ __global__ __launch_bounds__(256, 2) void cross_attend_kernel(AttendArgs a) {
   constexpr int PITCH = MAXK + 8;
   __shared__ __attribute__((aligned(16))) TL tile[MODE == Logits::Heads ? HEADS * 16 * PITCH : 1];
   if constexpr (MODE == Logits::Heads) {
-    static_assert(QT == 1, "one query tile per workgroup");
     struct alignas(4 * sizeof(TL)) Four { TL v[4]; };
 #pragma unroll
     for (int i = threadIdx.x; i < 16 * MAXK; i += 256) {
@@ -239,60 +231,46 @@ __global__ __launch_bounds__(256, 2) void cross_attend_kernel(AttendArgs a) {
     __syncthreads();
   }
   // Every logit of the wavefront is in flight before the first product.
-  TL raw[QT][KT][4];
+  TL raw[KT][4];
+  const TL *row = static_cast<const TL *>(a.logits) + b * a.ls[0] + h * a.ls[1] + qc * a.ls[2];
 #pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    const int q = min(q0 + 16 * t + col, a.nq - 1);
-    const TL *row = static_cast<const TL *>(a.logits) + b * a.ls[0] + h * a.ls[1] + q * a.ls[2];
+  for (int kt = 0; kt < KT; ++kt) {
+    const int key0 = kt * 16 + 4 * g;
+    if (!a.logits || kt >= tiles) {                  // (uniform)
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      const int key0 = kt * 16 + 4 * g;
-      if (!a.logits || kt >= tiles) {                  // (uniform)
+      for (int e = 0; e < 4; ++e) raw[kt][e] = TL(0.f);
+    } else if (MODE == Logits::Heads) {
+      __builtin_memcpy(raw[kt], __builtin_assume_aligned(tile + (h * 16 + col) * PITCH + key0, 4 * sizeof(TL)),
+                       4 * sizeof(TL));
+    } else if (MODE == Logits::Keys && key0 + 4 <= a.nk) {
+      __builtin_memcpy(raw[kt], __builtin_assume_aligned(row + key0, 4 * sizeof(TL)), 4 * sizeof(TL));
+    } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) raw[t][kt][e] = TL(0.f);
-      } else if (MODE == Logits::Heads) {
-        __builtin_memcpy(raw[t][kt], __builtin_assume_aligned(tile + (h * 16 + col) * PITCH + key0, 4 * sizeof(TL)),
-                         4 * sizeof(TL));
-      } else if (MODE == Logits::Keys && key0 + 4 <= a.nk) {
-        __builtin_memcpy(raw[t][kt], __builtin_assume_aligned(row + key0, 4 * sizeof(TL)), 4 * sizeof(TL));
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) raw[t][kt][e] = row[min(key0 + e, a.nk - 1) * a.ls[3]];
-      }
+      for (int e = 0; e < 4; ++e) raw[kt][e] = row[min(key0 + e, a.nk - 1) * a.ls[3]];
     }
   }
-  f32x4 s[QT][KT];
-  float mx[QT];
-#pragma unroll
-  for (int t = 0; t < QT; ++t) mx[t] = -INFINITY;
+  f32x4 s[KT];
+  float mx = -INFINITY;
   const float qscale = a.scale * kLog2e;
 #pragma unroll
   for (int kt = 0; kt < KT; ++kt) {
-#pragma unroll
-    for (int t = 0; t < QT; ++t) s[t][kt] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    s[kt] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     if (kt >= tiles) continue;           // (uniform)
     const bf16x8 kf = *reinterpret_cast<const bf16x8 *>(a.k + (b * a.kpad + kt * 16 + col) * C + h * HD + g * 8);
     const int key0 = kt * 16 + 4 * g;
+    const f32x4 acc = mfma16(kf, qf, f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-      const f32x4 acc = mfma16(kf, qf[t], f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool both = masked_q[t] && ((masked_k[kt / 4] >> ((key0 + e) & 63)) & 1);
-        const float bias = to_f32(raw[t][kt][e]) + (both ? 1e9f : 0.f);
-        s[t][kt][e] = key0 + e < a.nk ? acc[e] * qscale + bias * kLog2e : -INFINITY;
-        mx[t] = fmaxf(mx[t], s[t][kt][e]);
-      }
+    for (int e = 0; e < 4; ++e) {
+      const bool both = masked_q && ((masked_k[kt / 4] >> ((key0 + e) & 63)) & 1);
+      const float bias = to_f32(raw[kt][e]) + (both ? 1e9f : 0.f);
+      s[kt][e] = key0 + e < a.nk ? acc[e] * qscale + bias * kLog2e : -INFINITY;
+      mx = fmaxf(mx, s[kt][e]);
     }
   }
-  float sum[QT] = {};
-  f32x4 o[QT][2];
-#pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    mx[t] = fmaxf(mx[t], __shfl_xor(mx[t], 16, 64));
-    mx[t] = fmaxf(mx[t], __shfl_xor(mx[t], 32, 64));
-    o[t][0] = o[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  float sum = 0.f;
+  f32x4 o[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
 #pragma unroll
   for (int c = 0; c < KT / 2; ++c) {
     if (2 * c >= tiles) continue;
@@ -300,36 +278,30 @@ __global__ __launch_bounds__(256, 2) void cross_attend_kernel(AttendArgs a) {
 #pragma unroll
     for (int d = 0; d < 2; ++d)
       vf[d] = *reinterpret_cast<const bf16x8 *>(a.vt + (b * C + h * HD + 16 * d + col) * a.kpad + 32 * c + 8 * g);
+    bf16x8 pf;
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-      bf16x8 pf;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float p0 = exp2f(s[t][2 * c][e] - mx[t]), p1 = exp2f(s[t][2 * c + 1][e] - mx[t]);
-        sum[t] += p0 + p1;
-        pf[e] = bf16(p0);
-        pf[4 + e] = bf16(p1);
-      }
-#pragma unroll
-      for (int d = 0; d < 2; ++d) o[t][d] = mfma16(vf[d], pf, o[t][d]);
+    for (int e = 0; e < 4; ++e) {
+      const float p0 = exp2f(s[2 * c][e] - mx), p1 = exp2f(s[2 * c + 1][e] - mx);
+      sum += p0 + p1;
+      pf[e] = bf16(p0);
+      pf[4 + e] = bf16(p1);
     }
+#pragma unroll
+    for (int d = 0; d < 2; ++d) o[d] = mfma16(vf[d], pf, o[d]);
   }
+  float l = sum + __shfl_xor(sum, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  const int q = q0 + col;
+  if (q >= a.nq) return;
+  const float inv = 1.0f / l;
 #pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    float l = sum[t] + __shfl_xor(sum[t], 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    const int q = q0 + 16 * t + col;
-    if (q >= a.nq) continue;
-    const float inv = 1.0f / l;
+  for (int d = 0; d < 2; ++d) {
+    const int64_t at = (b * a.nq + q) * C + h * HD + 16 * d + 4 * g;
+    const f32x4 gt = *reinterpret_cast<const f32x4 *>(a.gate + at);
+    float v[4];
 #pragma unroll
-    for (int d = 0; d < 2; ++d) {
-      const int64_t at = (b * a.nq + q) * C + h * HD + 16 * d + 4 * g;
-      const f32x4 gt = *reinterpret_cast<const f32x4 *>(a.gate + at);
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = sigmoidf_(gt[e]) * static_cast<float>(bf16(o[t][d][e] * inv));
-      rowstep::store4f<bf16>(a.o + at, v);
-    }
+    for (int e = 0; e < 4; ++e) v[e] = sigmoidf_(gt[e]) * static_cast<float>(bf16(o[d][e] * inv));
+    rowstep::store4f<bf16>(a.o + at, v);
   }
 }
 
@@ -486,10 +458,10 @@ int xfh_cross_attention(const void *x_q, const void *x_k, const void *cond_q, co
   AttendArgs aa;
   std::memset(&aa, 0, sizeof(aa));
   aa.q = p.q; aa.k = p.k; aa.vt = p.vt; aa.gate = p.gate; aa.o = p.o;
-  aa.logits = logits; aa.logit_dtype = logit_dtype;
+  aa.logits = logits;
   if (logits) for (int i = 0; i < 4; ++i) aa.ls[i] = logit_strides[i];
   aa.mask_q = mask_q; aa.mask_q_dtype = mask_q_dtype; aa.mask_k = mask_k; aa.mask_k_dtype = mask_k_dtype;
-  aa.nq = int(nq); aa.nk = int(nk); aa.kpad = int(kpad); aa.qtiles = int(ceil_div(nq, int64_t(16 * QT)));
+  aa.nq = int(nq); aa.nk = int(nk); aa.kpad = int(kpad); aa.qtiles = int(ceil_div(nq, int64_t(16)));
   aa.scale = scale;
   const int64_t grid = subsets * aa.qtiles;
   XFH_REQUIRE(grid < (int64_t(1) << 31), "cross_attention: too many subsets");
