@@ -195,7 +195,12 @@ template <class T> int launch(const ContractionArgs &a, hipStream_t s) {
 // Small 0.45 up to n = 384, 0.65-0.75 above. In us per launch, the tile taken against Wide up to n = 1024, Square above: n = 72
 // 4.3 (Small) / 6.7, 128 5.4 (Small) / 9.4, 256 13.0 (Small) / 18.0, 420 42.5 (Half) / 75.0, 509 49.8 (Half)
 // / 81.4, 576 81.8 (Square) / 89.9, 640 120.5 (Half) / 128.2, 900 307 (Square) / 331, 1100 470 (Wide) / 500; Wide
-// stays at 384 and 768 (26.1, 155).
+// stays at 384 and 768 (26.1, 155). A tile's time jumps where its edge divides n: on either side, Wide / Square /
+// Half / Small, n = 383 26.3 / 29.8 / 33.5 / 33.8, 385 70.4 / 47.8 / 40.9 / 42.6, 767 153 / 160 / 196 / 325, 769 262 / 234 /
+// 247 / 359, 1151 492 / 527 / 582 / 927, 1153 714 / 637 / 639 / 997: the pick is the fastest or within noise of it at
+// each. It is 5% off at n = 700 (Wide 138, Square 132). With 64 channels, whose rounds are half as many, the
+// same weights serve: right at 300, 385 to 600 and 769 up, 8-12% off Square at 352 (17.1 / 15.7), 383, 700 (68.4 / 61.1)
+// and 767.
 enum class Tile { Wide, Square, Half, Small };
 template <class T> double tile_cost(int64_t n, int64_t channels, int cus, double step_us) {
   const int64_t wgs = ceil_div(n, T::TBI) * ceil_div(n, T::TBJ) * channels, slots = int64_t(cus) * T::WGS;

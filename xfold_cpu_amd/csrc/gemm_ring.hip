@@ -382,8 +382,10 @@ RingPick pick_ring(const GemmArgs &p, int64_t batch, bool glu, int cus) {
 // gemm_direct: a second workgroup on a CU doubles its time (its loads share the CU's 64 bytes
 // per clock), and the ring is then as fast or faster. us per launch, direct against ring:
 // [96][768] k = 768 4.6 / 9.1, k = 1536 6.9 / 13.9, [437][768] k = 768 7.9 / 10.4, [96][3072] k = 768 6.9 / 8.8;
-// past the line [768][768] k = 768 12.9 / 9.9, [200][3072] 11.1 / 8.7. Below k = 256 the two are equal;
-// [512][128] k = 384 (4.7 / 5.3) stays with the ring: no operator here has such a shape.
+// past the line [768][768] k = 768 12.9 / 9.9, [200][3072] 11.1 / 8.7. Below k = 256 the two are equal ([96][768]
+// k = 128 4.8 / 4.8, [512][128] 4.6 / 4.8). At most 128 columns with k < 512 would be faster here too ([512][128] k = 384
+// 5.0 / 5.7, [4096][128] 5.2 / 6.2, [2048][64] 4.7 / 6.2), but the ring's configurations are tested there and no
+// operator of this library has such a product.
 using Direct16 = Direct<1, 2, 8, 4>;      // 16 x 32 tile, k over 8 wavefronts
 using Direct32 = Direct<2, 2, 4, 4>;      // 32 x 32, 4
 using Direct64 = Direct<2, 4, 8, 2>;      // 32 x 64, 8
@@ -440,10 +442,12 @@ int gemm_ring(const GemmArgs &p, int64_t batch, int out_dtype, bool glu, hipStre
 }
 
 // fp32: 32 x 32 tiles while they leave a CU to each, 32 x 64 up to twice as many tiles as CUs, then
-// gemm_nt's 64 x 64. us per launch, direct against gemm_nt: [256][128] k = 128 4.1 / 8.6, k = 512 7.3 / 20, k = 1536
-// ([256][384]) 14 / 49; [4096][128] k = 128 5.4 / 9.3, k = 512 10.6 / 20.7; [16384][4] (the pair bias) 4.3 / 8.8; past the
-// line [16384][128] 13.3 / 12.6, [4096][384] 11.3 / 12.6. The error against 64 bits is half of gemm_nt's (four
-// partial sums of a quarter of the terms).
+// gemm_nt's 64 x 64, of which that line leaves one to a CU. us per launch, direct against gemm_nt: [900][96]
+// k = 128 4.5 / 6.9, k = 512 8.2 / 17.2; [4096][128] (one 32 x 64 tile per CU) 6.1 / 7.0, 11.7 / 17.7; [6144][128] (1.5)
+// 7.6 / 7.3, 17.5 / 18.0; at the line [8192][128] 8.3 / 7.7, 18.6 / 18.1; past it [4096][384] 11.7 / 10.7, 27.8 / 26.7,
+// [16384][128] 13.0 / 11.3, 34.2 / 27.3. From 1.5 tiles per CU to the line the two are within 8% of each other;
+// fewer than 64 columns gain most ([16384][4] k = 128, the pair bias' shape, 4.3 / 8.8). The error against 64
+// bits is half of gemm_nt's (four partial sums of a quarter of the terms).
 int gemm_direct_f32(const GemmArgs &p, int64_t batch, bool glu, hipStream_t s, bool *taken) {
   *taken = false;
   if (p.K < 32 || p.K % 32 || p.lda % 4 || p.ldb % 4 || p.sA % 4 || p.sB % 4 || !aligned(p.A, 16) || !aligned(p.B, 16) ||
