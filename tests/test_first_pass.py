@@ -174,3 +174,20 @@ def test_a_single_weight_is_checked_once(stubbed, monkeypatch):
             module(*args)
             assert len(seen) == len({id(t) for t in seen}) == 6     # (three Linears, scale, shift and its bias)
     assert not any("_hip_weight_groups" in m.__dict__ for m in module.modules())
+
+
+def test_weights_that_cannot_be_kept_are_not_stacked(stubbed, monkeypatch):
+    """Inference tensors carry no version: their copies are made on every call, where scale and shift take two
+    products of plain copies rather than one of a stack."""
+    make, inputs = MODULES["diffusion_transition"]
+    made, prepare, calls = [], nh._prepare, []
+    monkeypatch.setattr(nh, "_prepare", lambda *args: made.append(args) or prepare(*args))
+    monkeypatch.setattr(nh, "call", lambda name, *args: calls.append(name))
+    with torch.inference_mode():
+        module, args = make().eval(), inputs()
+        for _ in range(2):
+            del made[:], calls[:]
+            module(*args)
+            assert len(made) == 5 and "xfh_linear_batched" not in calls
+    for m in module.modules():
+        assert all(c._key is None for c in m.__dict__.get("_hip_weight_caches", {}).values())

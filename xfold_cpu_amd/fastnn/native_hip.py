@@ -277,6 +277,7 @@ def stamp(t: torch.Tensor) -> tuple:
 
 
 _expired = torch.UntypedStorage._expired
+_is_inference = torch.Tensor.is_inference
 
 
 class Storages:
@@ -345,11 +346,10 @@ class HipWeightCache(_Kept):
     """
 
     def get(self, weight: torch.Tensor, dtype: torch.dtype, layout: str = "plain") -> torch.Tensor:
-        try:
-            key = (*stamp(weight), dtype, layout)
-        except RuntimeError:
+        if weight.is_inference():
             self.clear()
             return _prepare(weight, dtype, layout)
+        key = (*stamp(weight), dtype, layout)
         value = self.lookup(key)
         return value if value is not None else self.keep(key, [weight], _prepare(weight, dtype, layout))
 
@@ -389,11 +389,10 @@ class FusedWeightCache(_Kept):
 
     def get(self, weights, dtype: torch.dtype) -> torch.Tensor:
         build = lambda: torch.cat([w.detach().to(dtype) for w in weights], dim=0).contiguous()  # noqa: E731
-        try:
-            key = (*map(stamp, weights), dtype)
-        except RuntimeError:
+        if any(map(_is_inference, weights)):
             self.clear()
             return build()
+        key = (*map(stamp, weights), dtype)
         value = self.lookup(key)
         return value if value is not None else self.keep(key, weights, build())
 
@@ -413,11 +412,10 @@ class DerivedWeightCache(_Kept):
     never cached when a source is an inference tensor)."""
 
     def get(self, sources, build):
-        try:
-            key = tuple(map(stamp, sources))
-        except RuntimeError:
+        if any(map(_is_inference, sources)):
             self.clear()
             return build(*sources)
+        key = tuple(map(stamp, sources))
         value = self.lookup(key)
         return value if value is not None else self.keep(key, sources, build(*sources))
 
@@ -512,8 +510,10 @@ def gather(module: torch.nn.Module, tag: str, sources, weights: int, x: torch.Te
         dtype = dtype or _compute_dtype(x.dtype, [p.dtype for p in sources[:weights]])
         return dtype, None if again else build(dtype)
     try:
-        key = [None if p is None else stamp(p) for p in sources]
-    except RuntimeError:                             # inference tensors carry no version: nothing is kept
+        key = None if sources[0].is_inference() else [None if p is None else stamp(p) for p in sources]
+    except RuntimeError:                             # (a mixture)
+        key = None
+    if key is None:                                  # inference tensors carry no version: nothing is kept
         dtype = dtype or _compute_dtype(x.dtype, [p.dtype for p in sources[:weights]])
         return dtype, None if again else build(dtype)
     changed = group.key is not None and (group.key != key or not group.storages.alive())

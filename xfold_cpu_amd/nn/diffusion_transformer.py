@@ -43,11 +43,16 @@ def _adaptive_layer_norm(aln: nn.Module, x: torch.Tensor, single_cond: Optional[
     sources = [*nh.params(aln, ("single_cond_scale", "single_cond_bias")), nh.param(aln, "single_cond_scale", "bias")]
     cond = ops.layer_norm(single_cond, cln.normalized_shape, nh.param(aln, "single_cond_layer_norm"),
                           nh.param(aln, "single_cond_layer_norm", "bias"), cln.eps, out_dtype=dtype, owner=cln)
-    # scale and shift stay fp32 (one rounding fewer before the sigmoid and the add); one launch
-    # over the stacked weights, made on the first pass (the next one may be a graph capture).
-    w, b = nh.derived_weight(aln, f"scale_shift:{dtype}", [t for t in sources if t is not None],
-                             lambda *ts: _scale_shift_weights(dtype, *ts))
-    scale, shift = ops.linear_batched(cond.reshape(-1, cond.shape[-1]), w, b, dtype, out_dtype=torch.float32)
+    # scale and shift stay fp32 (one rounding fewer before the sigmoid and the add); one launch over the
+    # stacked weights, made on the first pass (the next one may be a graph capture). Weights of which
+    # nothing is kept are not worth stacking on every call (fp32 CrossAttention 300 us, 279 in two launches).
+    if sources[0].is_inference():
+        scale, shift = (ops.linear(cond, nh.linear_weight(aln, name, dtype), b, dtype, out_dtype=torch.float32)
+                        for name, b in (("single_cond_scale", sources[2]), ("single_cond_bias", None)))
+    else:
+        w, b = nh.derived_weight(aln, f"scale_shift:{dtype}", [t for t in sources if t is not None],
+                                 lambda *ts: _scale_shift_weights(dtype, *ts))
+        scale, shift = ops.linear_batched(cond.reshape(-1, cond.shape[-1]), w, b, dtype, out_dtype=torch.float32)
     return ops.adaptive_layer_norm(x, scale, shift, aln.layer_norm.eps, out_dtype=out_dtype)
 
 
