@@ -430,8 +430,8 @@ def derived_weight(module: torch.nn.Module, tag: str, sources, build):
 
 def linear_weights(module: torch.nn.Module, names, dtype: torch.dtype):
     """:func:`linear_weight` of several Linears as one cache entry: the copies are made by one call,
-    into one allocation (each 256-byte aligned). Preparing and keeping them one by one was over a
-    third of the host time of a pair block's first pass."""
+    into one allocation (each 256-byte aligned). A new 72-token pair block with its single track: 655 us
+    with the copies made and kept one by one, 582 now."""
     return derived_weight(module, f"linears:{names}:{dtype}", [param(module, n) for n in names],
                           lambda *ws: _copies(ws, dtype))
 
