@@ -26,10 +26,11 @@ from .cache import InputCache
 
 def _adaptive_layer_norm(aln: nn.Module, x: torch.Tensor, single_cond: Optional[torch.Tensor],
                          dtype: torch.dtype, out_dtype: Optional[torch.dtype] = None,
-                         cond: Optional[tuple] = None) -> torch.Tensor:
+                         cond: Optional[tuple] = None, stacked: Optional[tuple] = None) -> torch.Tensor:
     """``AdaptiveLayerNorm.forward`` (``diffusion_transformer.py:51-64``); Linears in
     ``dtype``, result in ``out_dtype`` (default ``dtype``). ``cond`` = (scale, shift) already
-    computed from single_cond (see :func:`_block_conditioning`)."""
+    computed from single_cond (see :func:`_block_conditioning`); ``stacked`` = the weights of
+    :func:`_scale_shift_weights` that the caller has at hand."""
     if (single_cond is None) != (not aln.use_single_cond):
         raise ValueError("single_cond must be given exactly when use_single_cond is set")
     out_dtype = out_dtype or dtype
@@ -40,49 +41,58 @@ def _adaptive_layer_norm(aln: nn.Module, x: torch.Tensor, single_cond: Optional[
         return ops.layer_norm(x, ln.normalized_shape, ln.weight, ln.bias, ln.eps, out_dtype=out_dtype,
                               owner=ln)
     cln = aln.single_cond_layer_norm
-    sources = [*nh.params(aln, ("single_cond_scale", "single_cond_bias")), nh.param(aln, "single_cond_scale", "bias")]
     cond = ops.layer_norm(single_cond, cln.normalized_shape, nh.param(aln, "single_cond_layer_norm"),
                           nh.param(aln, "single_cond_layer_norm", "bias"), cln.eps, out_dtype=dtype, owner=cln)
     # scale and shift stay fp32 (one rounding fewer before the sigmoid and the add); one launch over the
     # stacked weights, made on the first pass (the next one may be a graph capture). Weights of which
     # nothing is kept are not worth stacking on every call (fp32 CrossAttention 300 us, 279 in two launches).
-    if sources[0].is_inference():
-        scale, shift = (ops.linear(cond, nh.linear_weight(aln, name, dtype), b, dtype, out_dtype=torch.float32)
-                        for name, b in (("single_cond_scale", sources[2]), ("single_cond_bias", None)))
-    else:
-        w, b = nh.derived_weight(aln, f"scale_shift:{dtype}", [t for t in sources if t is not None],
-                                 lambda *ts: _scale_shift_weights(dtype, *ts))
-        scale, shift = ops.linear_batched(cond.reshape(-1, cond.shape[-1]), w, b, dtype, out_dtype=torch.float32)
+    if stacked is None:
+        sources = _scale_shift_sources(aln)
+        if sources[0].is_inference():
+            scale, shift = (ops.linear(cond, nh.linear_weight(aln, name, dtype), b, dtype, out_dtype=torch.float32)
+                            for name, b in (("single_cond_scale", sources[2]), ("single_cond_bias", None)))
+            return ops.adaptive_layer_norm(x, scale, shift, aln.layer_norm.eps, out_dtype=out_dtype)
+        stacked = nh.derived_weight(aln, f"scale_shift:{dtype}", [t for t in sources if t is not None],
+                                    lambda *ts: _scale_shift_weights(dtype, *ts))
+    scale, shift = ops.linear_batched(cond.reshape(-1, cond.shape[-1]), *stacked[:2], dtype, out_dtype=torch.float32)
     return ops.adaptive_layer_norm(x, scale, shift, aln.layer_norm.eps, out_dtype=out_dtype)
 
 
+def _scale_shift_sources(aln: nn.Module) -> tuple:
+    return (*nh.params(aln, ("single_cond_scale", "single_cond_bias")), nh.param(aln, "single_cond_scale", "bias"))
+
+
 def _scale_shift_weights(dtype: torch.dtype, scale: torch.Tensor, shift: torch.Tensor,
-                         bias: Optional[torch.Tensor] = None):
+                         bias: Optional[torch.Tensor] = None, others=()):
     """single_cond_scale and single_cond_bias as one [2, c, c_cond] weight in ``dtype`` and their
-    [2, c] fp32 bias (zeros for single_cond_bias, which has none; None without a bias)."""
+    [2, c] fp32 bias (zeros for single_cond_bias, which has none; None without a bias); then copies
+    of ``others``, made by the same call."""
     c, k = scale.shape
     w = torch.empty((2, c, k), dtype=dtype, device=scale.device)
-    torch._foreach_copy_(w.unbind(0), (scale, shift))
+    copies = [torch.empty(t.shape, dtype=dtype, device=t.device) for t in others]
+    torch._foreach_copy_([*w.unbind(0), *copies], [scale, shift, *others])
     if bias is None:
-        return w, None
+        return (w, None, *copies)
     b = torch.zeros((2, c), dtype=torch.float32, device=scale.device)
     b[0].copy_(bias)
-    return w, b
+    return (w, b, *copies)
 
 
 def _ada_ln_zero(zero: nn.Module, hidden: torch.Tensor, single_cond: Optional[torch.Tensor],
                  dtype: torch.dtype, accumulate_into: Optional[torch.Tensor],
-                 cond: Optional[torch.Tensor] = None) -> torch.Tensor:
+                 cond: Optional[torch.Tensor] = None, weights: Optional[tuple] = None) -> torch.Tensor:
     """``AdaLNZero.forward`` (``diffusion_transformer.py:85-95``), optionally added in place;
-    ``cond`` = adaptive_zero_cond(single_cond) already computed, in the output dtype."""
-    w = nh.linear_weight(zero, "transition2", dtype)
+    ``cond`` = adaptive_zero_cond(single_cond) already computed, in the output dtype; ``weights`` =
+    the prepared transition2 and adaptive_zero_cond that the caller has at hand."""
+    w = weights[0] if weights is not None else nh.linear_weight(zero, "transition2", dtype)
     out = accumulate_into
     out_dtype = out.dtype if out is not None else dtype
     acc = out is not None
     if zero.use_single_cond:
         if cond is None:
-            cond = ops.linear(single_cond, nh.linear_weight(zero, "adaptive_zero_cond", dtype),
-                              nh.param(zero, "adaptive_zero_cond", "bias"), dtype, out_dtype=out_dtype)
+            w_cond = weights[1] if weights is not None else nh.linear_weight(zero, "adaptive_zero_cond", dtype)
+            cond = ops.linear(single_cond, w_cond, nh.param(zero, "adaptive_zero_cond", "bias"), dtype,
+                              out_dtype=out_dtype)
         epi = nh.EPI_MUL_SIGMOID_AUX_ACCUMULATE if acc else nh.EPI_MUL_SIGMOID_AUX
         return ops.linear(hidden, w, None, dtype, out=out, out_dtype=out_dtype, epilogue=epi,
                           aux=cond, aux_rows=cond.numel() // cond.shape[-1])
@@ -105,11 +115,20 @@ def diffusion_transition_hip(module: nn.Module, x: torch.Tensor, single_cond=Non
     w1 = nh.param(module, "transition1")
     dtype = nh.compute_dtype(x, w1)
     _check_accumulate(accumulate_into, x)
-    xn = _adaptive_layer_norm(module.adaptive_layernorm, x, single_cond, dtype,
-                              cond=None if _cond is None else _cond[:2])
+    aln, zero = module._modules["adaptive_layernorm"], module._modules["adaptive_zero_init"]
+    stacked = weights = None
+    if _cond is None and aln.use_single_cond and zero.use_single_cond and w1.dtype != dtype and not w1.is_inference():
+        # A call of its own under autocast: every plain weight in one entry, copied by one call.
+        *scale_shift, bias = _scale_shift_sources(aln)
+        others = nh.params(zero, ("transition2", "adaptive_zero_cond"))
+        stacked = nh.derived_weight(
+            module, f"conditioned:{dtype}", [*scale_shift, *others] if bias is None else [*scale_shift, *others, bias],
+            lambda scale, shift, *ts: _scale_shift_weights(dtype, scale, shift, bias, ts[:2]))
+        weights = stacked[2:]
+    xn = _adaptive_layer_norm(aln, x, single_cond, dtype, cond=None if _cond is None else _cond[:2], stacked=stacked)
     hidden = ops.gated_linear_unit(xn, nh.linear_weight(module, "transition1", dtype, "glu"), w1.shape[0] // 2, dtype)
-    return _ada_ln_zero(module.adaptive_zero_init, hidden, single_cond, dtype, accumulate_into,
-                        cond=None if _cond is None else _cond[2])
+    return _ada_ln_zero(zero, hidden, single_cond, dtype, accumulate_into, cond=None if _cond is None else _cond[2],
+                        weights=weights)
 
 
 _QKV = ("q_projection", "k_projection", "v_projection")
