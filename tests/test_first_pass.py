@@ -96,8 +96,9 @@ def test_an_operators_weights_are_copied_together(stubbed):
     # What is left: both transitions' two, the pair logits' one, the attention's four and output.
     assert computed.names.count("aten::_to_copy") == 10
     make, inputs = MODULES["diffusion_transition"]
+    transition, args = make().eval(), inputs()
     with torch.no_grad(), Computed() as computed:
-        make().eval()(*inputs())
+        transition(*args)
     # scale, shift, the condition and transition2 in one call; transition1 is packed.
     assert computed.names.count("aten::_foreach_copy_") == 1 and computed.names.count("aten::_to_copy") == 1
     weights = nh.linear_weights(module.pair_attention1, ("q_projection", "pair_bias_projection", "k_projection"), torch.bfloat16)
