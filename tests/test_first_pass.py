@@ -197,3 +197,14 @@ def test_weights_that_cannot_be_kept_are_not_stacked(stubbed, monkeypatch):
             assert len(made) == 5 and "xfh_linear_batched" not in calls
     for m in module.modules():
         assert all(c._key is None for c in m.__dict__.get("_hip_weight_caches", {}).values())
+
+
+def test_weights_on_two_devices_are_refused():
+    """One call copies several weights: a weight that lies elsewhere is not brought along."""
+    from xfold_cpu_amd.nn.diffusion_transformer import _scale_shift_weights
+    here, elsewhere = torch.randn(8, 8), torch.empty(8, 8, device="meta")
+    with pytest.raises(ValueError, match="one device"):
+        nh._copies((here, elsewhere), torch.bfloat16)
+    for weights in ((here, elsewhere), (here, here, None, (elsewhere,))):
+        with pytest.raises(ValueError, match="one device"):
+            _scale_shift_weights(torch.bfloat16, *weights)

@@ -436,10 +436,18 @@ def linear_weights(module: torch.nn.Module, names, dtype: torch.dtype):
                           lambda *ws: _copies(ws, dtype))
 
 
+def check_one_device(weights) -> None:
+    """Copies made by one call land where the first weight is: one that lies elsewhere (a host weight, which
+    :func:`ptr` refuses) must not be brought along."""
+    if any(w.device != weights[0].device for w in weights):
+        raise ValueError("The 'hip' backend requires strided ROCm (cuda) tensors, a module's weights on one device.")
+
+
 def _copies(weights, dtype: torch.dtype) -> list:
     ws = [w.detach() for w in weights]
     if all(w.dtype == dtype and w.is_contiguous() for w in ws):
         return ws
+    check_one_device(ws)
     flat = torch.empty(sum((w.numel() + 127) // 128 * 128 for w in ws), dtype=dtype, device=ws[0].device)
     out, at = [], 0
     for w in ws:

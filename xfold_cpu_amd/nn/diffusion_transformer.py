@@ -67,6 +67,7 @@ def _scale_shift_weights(dtype: torch.dtype, scale: torch.Tensor, shift: torch.T
     """single_cond_scale and single_cond_bias as one [2, c, c_cond] weight in ``dtype`` and their
     [2, c] fp32 bias (zeros for single_cond_bias, which has none; None without a bias); then copies
     of ``others``, made by the same call."""
+    nh.check_one_device([scale, shift, *others])
     c, k = scale.shape
     w = torch.empty((2, c, k), dtype=dtype, device=scale.device)
     copies = [torch.empty(t.shape, dtype=dtype, device=t.device) for t in others]
